@@ -48,6 +48,20 @@ enum krn_epilogue_op {
 int krn_gemm_nt(int in_kind, const void* a, const void* b, void* c, int out_kind, int64_t m, int64_t n, int64_t k,
                 int nops, const int* ops, const float* scalars, const void* const* vectors, void* stream);
 
+/* krn_gemm_nt (b_kn = 0) or the product with B stored K x N (b_kn = 1, bf16 or f16 operands) with a workspace of
+ * device memory: K may then be split over workgroups, whose float32 (int32) partial sums meet there, and a K x N
+ * operand is read as it lies or, where the transposed copy pays, transposed into it. krn_gemm_workspace gives the
+ * bytes the call uses; with fewer, or none, another kernel runs (only a K x N operand with N < 8, K < 8 or 2 GiB and
+ * more needs them, else an error). The workspace needs no preparation, is 16-byte aligned, and must not be touched by
+ * other work until this call's work on `stream` has run; calls on one stream may share one. No counterpart in the
+ * reference: its products need no caller memory. */
+int krn_gemm(int b_kn, int in_kind, const void* a, const void* b, void* c, int out_kind, int64_t m, int64_t n,
+             int64_t k, int nops, const int* ops, const float* scalars, const void* const* vectors, void* workspace,
+             int64_t workspace_bytes, void* stream);
+
+/* Bytes of workspace this krn_gemm call uses (a and b matter by their alignment; nothing is dereferenced). */
+int64_t krn_gemm_workspace(int b_kn, int in_kind, const void* a, const void* b, int64_t m, int64_t n, int64_t k);
+
 /* C[m, n] = epilogue(sum_k A[m, k] * B[k, n]), A: M x K, B: K x N (the NN form), C: M x N, bf16 or f16 operands;
  * out_kind and the epilogue as for krn_gemm_nt. Replaces krn's own GEMM tile program `acc += a[rows, ks] @
  * b[ks, cols]` (reference examples/04_libraries/01_gemm_tiles.py:34-40) and the multiply of lib.matmul

@@ -122,6 +122,19 @@ class HIPStream(Stream):
         self.device, self.handle = device, handle
         self._open: list[tuple[str, tuple[object, ...]]] = []
         self._marks: deque[tuple[HIPEvent, list[tuple[str, tuple[object, ...]]]]] = deque()
+        self._workspace: HIPTensor | None = None
+
+    def workspace(self, nbytes: int) -> "HIPTensor":
+        """At least `nbytes` of device scratch for one launch on this stream. Launches on a stream run in order, so they
+        share one buffer, which grows to the largest request and is freed with the stream; a launch holds it until
+        it has completed, so a buffer outgrown meanwhile (by another thread, too) is freed after its last use. A
+        launch that a graph records gets memory of its own, which the graph keeps: its replays run on any stream."""
+        if self.capturing:
+            return self.device.empty_on(self, D.U8, nbytes)
+        held = self._workspace
+        if held is None or held.nbytes < nbytes:
+            held = self._workspace = self.device.empty_on(self, D.U8, nbytes)
+        return held
 
     @property
     def capturing(self) -> bool:
@@ -340,28 +353,21 @@ class Launch:
                     return None
                 code = base + (1 if op.axis == "row" else 2) + library.VECTOR_KINDS[vector.dtype]
                 ops.append((code, 0.0, vector.pointer))
-        if plan.layout == "nn":
-            need = library.gemm_nn_workspace_for(a.pointer, b.pointer, m, n, k)
-            if need == 0:  # B is read K x N as it lies: no workspace
-                direct = library.gemm_nn_call(plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k,
-                                              ops, 0, 0)
-                return lambda stream: direct(stream.handle)
-            scratch = StreamScratch(need)
-            products: dict[int, Callable[[int], None]] = {}  # workspace pointer -> the product marshalled for it
+        need = library.gemm_workspace(plan.layout, plan.operand, a.pointer, b.pointer, m, n, k)
+        if need == 0 and plan.layout == "nt":
+            direct = library.gemm_nt_call(plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k, ops)
+            return lambda stream: direct(stream.handle)
+        product = library.gemm_call(plan.layout, plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k,
+                                    ops, need)
+        if need == 0:
+            return lambda stream: product(0, stream.handle)
 
-            def nn(stream: HIPStream) -> None:
-                workspace = scratch.on(stream)
-                product = products.get(workspace.pointer)
-                if product is None:
-                    product = products[workspace.pointer] = library.gemm_nn_call(
-                        plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k, ops, workspace.pointer,
-                        max(need, 1))
-                product(stream.handle)
-                stream.note(self.kernel.name, (workspace,))
+        def run(stream: HIPStream) -> None:
+            workspace = stream.workspace(need)
+            product(workspace.pointer, stream.handle)
+            stream.note(self.kernel.name, (workspace,))
 
-            return nn
-        product = library.gemm_nt_call(plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k, ops)
-        return lambda stream: product(stream.handle)
+        return run
 
     def _attention(self, plan: cdna4.AttentionPlan, params: dict, grid: Blocks):
         q, k, v, o = (params[n] for n in (plan.q, plan.k, plan.v, plan.o))

@@ -36,6 +36,13 @@ def lib() -> ctypes.CDLL:
         c_int, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int, POINTER(c_int),
         POINTER(c_float), POINTER(c_void_p), c_void_p,
     ]  # fmt: skip
+    handle.krn_gemm.restype = c_int
+    handle.krn_gemm.argtypes = [
+        c_int, c_int, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int, POINTER(c_int),
+        POINTER(c_float), POINTER(c_void_p), c_void_p, c_int64, c_void_p,
+    ]  # fmt: skip
+    handle.krn_gemm_workspace.restype = c_int64
+    handle.krn_gemm_workspace.argtypes = [c_int, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64]
     handle.krn_attention_fwd.restype = c_int
     handle.krn_attention_fwd.argtypes = [
         c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p,
@@ -75,6 +82,25 @@ def kind(dtype: Dtype) -> int:
         raise KernelError(f"{dtype} has no kind in the kernel library's C ABI") from None
 
 
+def gemm_workspace(layout: str, in_dtype: Dtype, a: int, b: int, m: int, n: int, k: int) -> int:
+    """Bytes of device workspace `gemm_call` of these arguments uses (`layout` "nt" or "nn")."""
+    return lib().krn_gemm_workspace(int(layout == "nn"), kind(in_dtype), a, b, m, n, k)
+
+
+def gemm_call(layout: str, in_dtype: Dtype, a: int, b: int, c: int, out_dtype: Dtype, m: int, n: int, k: int,
+              ops: list[tuple[int, float, int]], workspace_bytes: int):
+    """The product (`layout` "nt": B is N x K, "nn": K x N) as a function of the workspace and the stream, with the
+    other arguments marshalled once."""
+    codes, scalars, vectors = marshal_ops(ops)
+    entry = lib().krn_gemm
+    head = (int(layout == "nn"), kind(in_dtype), a, b, c, kind(out_dtype), m, n, k, len(ops), codes, scalars, vectors)
+
+    def call(workspace: int, stream: int) -> None:
+        check(entry(*head, workspace, workspace_bytes, stream), "krn_gemm")
+
+    return call
+
+
 def gemm_nt_call(in_dtype: Dtype, a: int, b: int, c: int, out_dtype: Dtype, m: int, n: int, k: int,
                  ops: list[tuple[int, float, int]]):
     """`gemm_nt` of these arguments as a function of the stream, with the arguments marshalled once."""
@@ -106,24 +132,6 @@ def gemm_nn_workspace(n: int, k: int) -> int:
 def gemm_nn_workspace_for(a: int, b: int, m: int, n: int, k: int) -> int:
     """Bytes of workspace this NN product needs: 0 when the kernel reads B as it lies."""
     return lib().krn_gemm_nn_workspace_for(a, b, m, n, k)
-
-
-def gemm_nn_call(in_dtype: Dtype, a: int, b: int, c: int, out_dtype: Dtype, m: int, n: int, k: int,
-                 ops: list[tuple[int, float, int]], workspace: int, workspace_bytes: int):
-    """`gemm_nn` (B stored K x N, read as it lies or transposed into `workspace`) as a function of the stream,
-    marshalled once."""
-    count = len(ops)
-    codes = (c_int * max(count, 1))(*(op for op, _, _ in ops))
-    scalars = (c_float * max(count, 1))(*(s for _, s, _ in ops))
-    vectors = (c_void_p * max(count, 1))(*(v for _, _, v in ops))
-    entry = lib().krn_gemm_nn
-    head = (kind(in_dtype), a, b, c, kind(out_dtype), m, n, k, count, codes, scalars, vectors, workspace,
-            workspace_bytes)
-
-    def call(stream: int) -> None:
-        check(entry(*head, stream), "krn_gemm_nn")
-
-    return call
 
 
 def gemm_nt(in_dtype: Dtype, a: int, b: int, c: int, out_dtype: Dtype, m: int, n: int, k: int,

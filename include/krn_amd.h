@@ -115,6 +115,17 @@ int krn_transpose16(const void* in, void* out, int64_t rows, int64_t cols, void*
 int krn_attention_fwd(int kind, const void* q, const void* k, const void* v, void* o, int64_t bh, int64_t sq,
                       int64_t sk, int64_t d, float scale, int causal, void* stream);
 
+/* krn_attention_fwd with device memory for the launches that share one head's keys among several workgroups (few
+ * queries against many keys): krn_attention_workspace gives the bytes; with fewer, or none, the keys stay within a
+ * workgroup. The workspace needs no preparation, is 16-byte aligned, and must not be touched by other work until this
+ * call's work on `stream` has run; calls on one stream may share one. */
+int krn_attention_fwd_ws(int kind, const void* q, const void* k, const void* v, void* o, int64_t bh, int64_t sq,
+                         int64_t sk, int64_t d, float scale, int causal, void* workspace, int64_t workspace_bytes,
+                         void* stream);
+
+/* Bytes of workspace this krn_attention_fwd_ws call uses, 0 when none. */
+int64_t krn_attention_workspace(int64_t bh, int64_t sq, int64_t sk, int64_t d, int causal);
+
 /* Row softmax: y[r, c] = exp(x[r, c] - max) / sum exp(x[r, :] - max) over the first `width` columns of each of
  * `rows` rows, float32 arithmetic, one rounding to the element kind (KRN_F32, KRN_F16 or KRN_BF16, the same for x
  * and y). ldx / ldy are the row strides in elements (>= width); columns past width are neither read nor written.

@@ -31,7 +31,7 @@
 // than 8 (p <= 2^8), which scales p, acc and total by the same power of two and leaves acc / total unchanged; the
 // output is acc times the correctly rounded reciprocal of the row sum (at most one float32 rounding more than
 // acc / total, before the rounding to 16 bits).
-#include "common.h"
+#include "attention_parts.h"
 
 #ifndef KRN_FA_WAVES_DEFAULT
 #define KRN_FA_WAVES_DEFAULT 8
@@ -39,56 +39,9 @@
 
 namespace krn {
 
-typedef short v4s __attribute__((ext_vector_type(4)));
-
-template <bool BF>
-struct Half;
-template <>
-struct Half<true> {
-  __device__ static uint32_t pack(float lo, float hi) {
-    return f2bf2(lo, hi);  // v_cvt_pk_bf16_f32, nearest even
-  }
-  __device__ static uint16_t from(float x) { return f2bf(x); }
-  __device__ static void mma(f32x16& c, u32x4 a, u32x4 b) {
-    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                0, 0);
-  }
-};
-template <>
-struct Half<false> {
-  __device__ static uint32_t pack(float lo, float hi) { return (uint32_t)f2h(lo) | ((uint32_t)f2h(hi) << 16); }
-  __device__ static uint16_t from(float x) { return f2h(x); }
-  __device__ static void mma(f32x16& c, u32x4 a, u32x4 b) {
-    c = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0,
-                                               0);
-  }
-};
-
 constexpr int FA_WAVES = KRN_FA_WAVES_DEFAULT;  // waves per workgroup, 32 query rows each
 constexpr int BQ = 32 * FA_WAVES;               // query rows per workgroup
 constexpr int BKEY = 64;  // keys per LDS tile
-
-// LDS swizzles of the [key][d] tiles (64 banks serve 256 bytes per cycle). K: the 16-byte reads of 16 consecutive
-// keys must hit 16 distinct positions modulo 256 bytes. V: the transposed 8-byte reads cover 4 consecutive keys x
-// 64 bytes per 32 lanes. D = 128 (256-byte rows) and D = 64 (128-byte rows) need different XOR patterns.
-template <int D>
-__device__ __forceinline__ int k_slot(int key, int chunk) {
-  return D == 128 ? chunk ^ (key & 15) : chunk ^ ((key >> 1) & 7);
-}
-template <int D>
-__device__ __forceinline__ int v_slot(int key, int chunk) {
-  return D == 128 ? chunk ^ ((key & 3) << 2) : chunk ^ (((key >> 1) & 1) << 2);
-}
-
-// max(x, x of lane ^ 32): the two lanes that hold one query row (v_permlane32_swap, no LDS round trip). One
-// v_max_f32 (written as assembly: as fmaxf the compiler first quiets both operands, two more VALU instructions; the
-// instruction quiets a signaling NaN itself, and these operands are arithmetic results or swaps of them).
-__device__ __forceinline__ float pair_max(float x) {
-  const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
-  float y;
-  asm("v_max_f32 %0, %1, %2" : "=v"(y) : "v"(__uint_as_float(sw[0])), "v"(__uint_as_float(sw[1])));
-  return y;
-}
 
 // One query tile `qt` (BQ rows) of head `head`: the whole key pass and the store of its rows. `lds` is the
 // workgroup's ring of K and V tiles. `qf` holds this lane's Q fragments: loaded here unless `preloaded`, in which
@@ -433,45 +386,87 @@ static void launch_attention(const void* q, const void* k, const void* v, void* 
                      (const uint16_t*)v, (uint16_t*)o, sq, sk, scale, q_tiles, causal, (int)paired);
 }
 
-extern "C" int krn_attention_fwd(int kind, const void* q, const void* k, const void* v, void* o, int64_t bh,
-                                 int64_t sq, int64_t sk, int64_t d, float scale, int causal, void* stream) {
+// How a launch runs: parts = 0 is the kernel above (256 query rows per workgroup), otherwise the key-split kernel with
+// that many workgroups per block of 32 query rows. Both times are estimated in microseconds from sweeps on 256 CUs and
+// the shorter taken. A workgroup above takes 1.8 us (d = 64: 1.35) per 64 keys, whatever its rows, and the launch 4
+// more; a wave of the key-split kernel 1.6 us per 32 keys (d = 64: 0.93 alone on its CU, 1.15 in twos), a workgroup
+// 2.6, a launch 3, the reduction of several parts 3 and the planes' bytes. Measured, both sides: 128 heads x 1 query x
+// 4096 keys, d = 128: 113 -> 57 us (two parts; 268 MB of K and V); 32 x 1 x 8192: 203 -> 29 (eight); 16 x 1000 x 1000,
+// d = 64: 25.9 -> 13.0; causal 32 x 512 x 512, d = 128: 19.4 -> 15.6; causal 32 x 1024 x 1024: 33.3 against 41.0, so
+// launches that fill the chip with 256-row workgroups stay there.
+static int attention_parts(int64_t bh, int64_t sq, int64_t sk, int64_t d, int causal, int64_t workspace) {
+  const int64_t q_tiles = (sq + BQ - 1) / BQ, q32 = (sq + 31) / 32;
+  // keys of the longest and of an average row block
+  const double longest = causal ? (double)(sk < sq ? sk : sq) : (double)sk;
+  const double mean = causal ? longest / 2 : longest;
+  const double tile = d == 128 ? 1.8 : 1.35;
+  const double whole = 4.0 + tile * fmax(longest / 64, mean / 64 * (double)(bh * q_tiles) / 256);
+  double least = whole;
+  int best = 0;
+  if (bh * q32 * 16 > 0x7fffffff) return 0;
+  for (int parts = 1; parts <= 16; ++parts) {
+    const double steps = fmax(1.0, mean / 32 / (4 * parts)), wgs = (double)(bh * q32 * parts);
+    if (parts > 1 && (steps < 2.0 || attention_split_bytes(bh, sq, d, parts) > workspace)) break;
+    double us = d == 128 ? 3.0 + fmax(1.0, wgs / 256) * (2.6 + 1.6 * steps)
+                         : 3.0 + fmax(1.0, wgs / 512) * (2.6 + (wgs > 256 ? 1.15 : 0.93) * steps);
+    if (parts > 1) us += 3.0 + (double)attention_split_bytes(bh, sq, d, parts) / 5e6;
+    if (us < least) best = parts, least = us;
+  }
+  return best;
+}
+
+static bool attention_arguments(int kind, const void* q, const void* k, const void* v, const void* o, int64_t bh,
+                                int64_t sq, int64_t sk, int64_t d) {
   if (kind != BF16 && kind != F16) {
     krn_set_error("attention: element kind %d; bf16 or f16 tensors only", kind);
-    return -1;
+    return false;
   }
   if (d != 64 && d != 128) {
     krn_set_error("attention: head dimension %lld; 64 or 128 only", (long long)d);
-    return -1;
+    return false;
   }
   if (bh < 0 || sq < 0 || sk < 0) {
     krn_set_error("attention: negative extent");
-    return -1;
+    return false;
   }
   if ((uintptr_t)q % 16 || (uintptr_t)k % 16 || (uintptr_t)v % 16 || (uintptr_t)o % 16) {
     krn_set_error("attention: tensors must be 16-byte aligned");
-    return -1;
+    return false;
   }
   const int64_t blocks = bh * ((sq + BQ - 1) / BQ);
-  if (blocks == 0) return 0;
+  if (blocks == 0) return true;
   if (blocks > 0x7fffffff) {
     krn_set_error("attention: %lld workgroups exceed the grid limit", (long long)blocks);
-    return -1;
+    return false;
   }
   if (sk == 0) {
     // no keys: the tile program divides 0 by 0
     krn_set_error("attention: an empty key sequence has no softmax");
-    return -1;
+    return false;
   }
   if (sk * d * 2 > 0x7fffffff) {  // K and V tiles are addressed by 31-bit offsets within a head
     krn_set_error("attention: %lld keys of %lld elements exceed 2 GiB per head", (long long)sk, (long long)d);
-    return -1;
+    return false;
   }
   if ((sq + BQ) * d * 2 > 0x7fffffff) {  // so are the output rows, those of a last partial query tile included
     krn_set_error("attention: %lld queries of %lld elements exceed 2 GiB per head", (long long)sq, (long long)d);
-    return -1;
+    return false;
   }
+  return true;
+}
+
+extern "C" int krn_attention_fwd_ws(int kind, const void* q, const void* k, const void* v, void* o, int64_t bh,
+                                    int64_t sq, int64_t sk, int64_t d, float scale, int causal, void* workspace,
+                                    int64_t workspace_bytes, void* stream) {
+  if (!attention_arguments(kind, q, k, v, o, bh, sq, sk, d)) return -1;
+  if (bh == 0 || sq == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool bf = kind == BF16;
+  const int parts = attention_parts(bh, sq, sk, d, causal != 0, workspace ? workspace_bytes : 0);
+  if (parts > 0) {
+    const AttentionCall c{q, k, v, o, workspace, bh, sq, sk, scale, causal != 0, parts, s};
+    return launch_attention_split(bf, (int)d, c);
+  }
 #define KRN_FA(BFV, DV) \
   launch_attention<BFV, DV>(q, k, v, o, bh, sq, sk, scale, causal != 0, s)
   if (bf && d == 128) KRN_FA(true, 128);
@@ -485,4 +480,14 @@ extern "C" int krn_attention_fwd(int kind, const void* q, const void* k, const v
     return (int)err;
   }
   return 0;
+}
+
+extern "C" int krn_attention_fwd(int kind, const void* q, const void* k, const void* v, void* o, int64_t bh,
+                                 int64_t sq, int64_t sk, int64_t d, float scale, int causal, void* stream) {
+  return krn_attention_fwd_ws(kind, q, k, v, o, bh, sq, sk, d, scale, causal, nullptr, 0, stream);
+}
+
+extern "C" int64_t krn_attention_workspace(int64_t bh, int64_t sq, int64_t sk, int64_t d, int causal) {
+  if (bh <= 0 || sq <= 0 || sk <= 0 || (d != 64 && d != 128)) return 0;
+  return attention_split_bytes(bh, sq, d, attention_parts(bh, sq, sk, d, causal != 0, INT64_MAX));
 }

@@ -362,9 +362,14 @@ class Launch:
         if need == 0:
             return lambda stream: product(0, stream.handle)
 
+        return self._with_workspace(product, need)
+
+    def _with_workspace(self, call: Callable[[int, int], None], nbytes: int) -> Callable[[HIPStream], None]:
+        """`call(workspace, stream)` with the stream's workspace, held until the launch has completed."""
+
         def run(stream: HIPStream) -> None:
-            workspace = stream.workspace(need)
-            product(workspace.pointer, stream.handle)
+            workspace = stream.workspace(nbytes)
+            call(workspace.pointer, stream.handle)
             stream.note(self.kernel.name, (workspace,))
 
         return run
@@ -387,8 +392,12 @@ class Launch:
             return None
         # exp(x) is exp2(x * log2(e)): the kernel's exponent scale carries the base
         scale = float(np.float32(float(value) * plan.base))
-        return lambda stream: library.attention_fwd(plan.dtype, q.pointer, k.pointer, v.pointer, o.pointer, bh, sq,
-                                                    sk, d, scale, plan.causal, stream.handle)
+        need = library.attention_workspace(bh, sq, sk, d, plan.causal)
+        call = library.attention_call(plan.dtype, q.pointer, k.pointer, v.pointer, o.pointer, bh, sq, sk, d, scale,
+                                      plan.causal, need)
+        if need == 0:
+            return lambda stream: call(0, stream.handle)
+        return self._with_workspace(call, need)
 
     def _softmax(self, plan: cdna4.SoftmaxPlan, params: dict, grid: Blocks):
         x, y = params[plan.x], params[plan.y]

@@ -47,6 +47,13 @@ def lib() -> ctypes.CDLL:
     handle.krn_attention_fwd.argtypes = [
         c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p,
     ]  # fmt: skip
+    handle.krn_attention_fwd_ws.restype = c_int
+    handle.krn_attention_fwd_ws.argtypes = [
+        c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p,
+        c_int64, c_void_p,
+    ]  # fmt: skip
+    handle.krn_attention_workspace.restype = c_int64
+    handle.krn_attention_workspace.argtypes = [c_int64, c_int64, c_int64, c_int64, c_int]
     handle.krn_gemm_nn.restype = c_int
     handle.krn_gemm_nn.argtypes = [
         c_int, c_void_p, c_void_p, c_void_p, c_int, c_int64, c_int64, c_int64, c_int, POINTER(c_int),
@@ -144,6 +151,23 @@ def attention_fwd(dtype: Dtype, q: int, k: int, v: int, o: int, bh: int, sq: int
                   causal: bool, stream: int) -> None:
     check(lib().krn_attention_fwd(kind(dtype), q, k, v, o, bh, sq, sk, d, scale, int(causal), stream),
           "krn_attention_fwd")
+
+
+def attention_workspace(bh: int, sq: int, sk: int, d: int, causal: bool) -> int:
+    """Bytes of device workspace `attention_call` of these arguments uses."""
+    return lib().krn_attention_workspace(bh, sq, sk, d, int(causal))
+
+
+def attention_call(dtype: Dtype, q: int, k: int, v: int, o: int, bh: int, sq: int, sk: int, d: int, scale: float,
+                   causal: bool, workspace_bytes: int):
+    """The attention as a function of the workspace and the stream, with the other arguments marshalled once."""
+    entry = lib().krn_attention_fwd_ws
+    head = (kind(dtype), q, k, v, o, bh, sq, sk, d, scale, int(causal))
+
+    def call(workspace: int, stream: int) -> None:
+        check(entry(*head, workspace, workspace_bytes, stream), "krn_attention_fwd")
+
+    return call
 
 
 def transpose16(src: int, dst: int, rows: int, cols: int, stream: int) -> None:

@@ -845,7 +845,11 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_skinny(const uint8_t* __re
 #pragma unroll
   for (int q = 0; q < 4; ++q) rd[q] = r32 * 128 + (((half * 4 + q) ^ ((r32 >> 1) & 7)) * 16);
   const int slices = (int)(kbytes / 128), part = blockIdx.y;
-  const int from = slices * part / sp.parts, nk = slices * (part + 1) / sp.parts - from;  // this workgroup's slices
+  int from = 0, nk = slices;  // this workgroup's slices
+  if (sp.parts > 1) {
+    from = slices * part / sp.parts;
+    nk = slices * (part + 1) / sp.parts - from;
+  }
   const int per = nk / WAVES, rem = nk % WAVES;
   const int begin = from + wave * per + min(wave, rem), cnt = per + (wave < rem ? 1 : 0);
   // the storing waves fetch the epilogue's vector operands now: loads issued at the very end of a workgroup would
@@ -1147,7 +1151,7 @@ static double split_cost(int shape, bool nn, int64_t m, int64_t n, int64_t slice
   const int64_t wgs = ((m + T[shape].bm - 1) / T[shape].bm) * ((n + T[shape].bn - 1) / T[shape].bn) * parts;
   const double per_cu = (double)((wgs + 255) / 256);
   double us = (double)((slices + parts - 1) / parts) * fmax(T[shape].slice, (nn ? T[shape].more_nn : T[shape].more) * per_cu);
-  if (parts > 1) us += 5.0 + (double)parts * (double)split_plane(m, n) / 5e6;  // the second launch reads the planes
+  if (parts > 1) us += 8.0 + (double)parts * (double)split_plane(m, n) / 5e6;  // the second launch reads the planes
   return us;
 }
 
@@ -1172,19 +1176,20 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
   if (piped && m <= 128) {
     // One workgroup per 32 columns; with few columns K is split as well. A slice takes a workgroup 0.11 us with one
     // block of 32 rows, 0.35 with four (1 x 4096 x 4096 bf16: 9.2 us on 128 workgroups; 16 x 1024 x 14336: 28.1 on 32);
-    // the second launch of a split costs 4.
-    static const double RATE[] = {0.11, 0.14, 0.24, 0.35};
+    // the second launch of a split costs 8, most of it on the host (3 x 768 x 4992 f16: 7.8 us, split 11.6).
+    static const double RATE[] = {0.10, 0.14, 0.24, 0.35};
     const int64_t groups = (n + 31) / 32;
     const double whole_k = (double)slices * RATE[(m - 1) / 32] * (double)((groups + 255) / 256);
     best = {SKINNY, 0, 1, 0}, least = whole_k;
     for (int parts = 2; parts <= 16 && groups * parts <= 256 && slices / parts >= 8; ++parts) {
       const int64_t need = parts * split_plane(m, n);
-      const double us = whole_k / parts + 4.0 + (double)need / 5e6;
+      const double us = whole_k / parts + 8.0 + (double)need / 5e6;
       if (need <= workspace && us < least) best = {SKINNY, 0, parts, need}, least = us;
     }
     // 65 to 128 rows of 16-bit operands: four row blocks per wave make the skinny loop slower than 128 x 128 tiles
     // with K split (128 x 8192 x 8192 bf16 48.5 -> 41 us; fp8 the other way, 19 against 30 us)
     if (m <= 64 || elem == 1) return best;
+    least -= 2.0;  // near ties stay (89 x 1536 x 2560 f16: 11.0 us, 32 x 64 tiles 11.7)
   } else if (piped && 128 * kbytes <= 0x7fffffff) {
     if (t128 <= 256) best = {MID, 0, 1, 0}, least = 0.60 * (double)slices;
     else if (fmt != FMT_FP8 && 256 * kbytes <= 0x7fffffff)

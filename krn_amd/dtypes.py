@@ -31,6 +31,9 @@ class Dtype:
     bits: int = 0
     man: int = 0
 
+    def __hash__(self) -> int:
+        return hash(self.name)  # a type's name is its own (plan look-ups hash every argument's type on every launch)
+
     @property
     def is_int(self) -> bool:
         return self.kind in (Kind.UINT, Kind.SINT)

@@ -8,6 +8,7 @@ by the device backend. Calling a stub outside a kernel raises.
 
 import inspect
 from dataclasses import dataclass, fields, is_dataclass
+from functools import lru_cache
 from typing import Any, Generic, TypeVar, get_origin
 
 from krn_amd import dtypes as _d
@@ -105,8 +106,12 @@ def const_fields(config: object) -> dict[str, object]:
     """The `Const` fields of a configuration instance, by name."""
     if not (is_dataclass(config) and not isinstance(config, type)):
         raise TypeError(f"{config!r} is not a @struct configuration")
-    hints = {f.name: f.type for f in fields(config)}
-    return {name: getattr(config, name) for name, hint in hints.items() if is_const(hint)}
+    return {name: getattr(config, name) for name in _const_names(type(config))}
+
+
+@lru_cache(maxsize=1024)
+def _const_names(config: type) -> tuple[str, ...]:
+    return tuple(f.name for f in fields(config) if is_const(f.type))
 
 
 @dataclass(frozen=True)

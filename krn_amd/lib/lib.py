@@ -10,6 +10,7 @@ call falls to the next one.
 """
 
 import os
+import sys
 from abc import ABC, abstractmethod
 from dataclasses import dataclass
 from enum import Enum
@@ -124,7 +125,8 @@ def candidate(name: str) -> Candidate:
         return Host()
     if name not in MODULES:
         raise KeyError(f"unknown matmul candidate {name!r}; known: {', '.join(PREFERENCE[Op.MATMUL])}")
-    return import_module(MODULES[name]).CANDIDATE
+    module = sys.modules.get(MODULES[name]) or import_module(MODULES[name])  # import_module alone is 5 us a call
+    return module.CANDIDATE
 
 
 def order(library: str | None = None) -> tuple[str, ...]:

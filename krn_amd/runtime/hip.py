@@ -20,6 +20,7 @@ from collections import deque
 from collections.abc import Callable, Sequence
 from ctypes import c_float, c_int, c_int64, c_void_p
 from dataclasses import is_dataclass
+from functools import lru_cache
 from pathlib import Path
 
 import numpy as np
@@ -497,6 +498,11 @@ _plans: dict[tuple, Launch] = {}  # (kernel, argument kinds) -> its captured IR 
 _plans_lock = threading.Lock()
 
 
+@lru_cache(maxsize=1024)
+def _parameters(fn: Callable) -> tuple[str, ...]:
+    return tuple(inspect.signature(fn).parameters)  # 18 us, and a launcher is made for every `kernel[config](...)`
+
+
 class HIPLauncher(Launcher):
     """A kernel with an optional explicit geometry. The first call of a signature captures and plans it."""
 
@@ -504,7 +510,7 @@ class HIPLauncher(Launcher):
         # only `fn` and `name` are read, as the reference's SourceLauncher does (src/krn/runtime/runtime.py:463-470),
         # so krn's own Kernel objects launch here unchanged
         self.device, self.kernel, self.launch = device, kernel, _blocks(launch)
-        self.parameters = tuple(inspect.signature(kernel.fn).parameters)
+        self.parameters = _parameters(kernel.fn)
 
     def ordered(self, args: tuple, kwargs: dict) -> tuple:
         if not kwargs and len(args) == len(self.parameters):

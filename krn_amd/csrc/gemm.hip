@@ -806,7 +806,7 @@ template <int FMT, int MT, int WAVES, int STAGES, bool ACT, int AL = MT * 4>
 __global__ __launch_bounds__(WAVES * 64, 1) void gemm_skinny(const uint8_t* __restrict__ A,
                                                               const uint8_t* __restrict__ B, void* __restrict__ C,
                                                               int64_t M, int64_t N, int64_t kbytes, int64_t lda,
-                                                              int64_t ldb, int64_t ldc, Epilogue e, Split sp) {
+                                                              int64_t ldb, int64_t ldc, Epilogue e, int parts) {
   typedef Mfma<FMT> Unit;
   typedef typename Unit::Acc Acc;
   typedef std::conditional_t<FMT == FMT_I8, int, float> Elem;
@@ -846,9 +846,10 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_skinny(const uint8_t* __re
   for (int q = 0; q < 4; ++q) rd[q] = r32 * 128 + (((half * 4 + q) ^ ((r32 >> 1) & 7)) * 16);
   const int slices = (int)(kbytes / 128), part = blockIdx.y;
   int from = 0, nk = slices;  // this workgroup's slices
-  if (sp.parts > 1) {
-    from = slices * part / sp.parts;
-    nk = slices * (part + 1) / sp.parts - from;
+  if (parts > 1) {
+    from = slices * part / parts;
+    nk = slices * (part + 1) / parts - from;
+    C = static_cast<uint8_t*>(C) + part * (M * ldc * 4);
   }
   const int per = nk / WAVES, rem = nk % WAVES;
   const int begin = from + wave * per + min(wave, rem), cnt = per + (wave < rem ? 1 : 0);
@@ -930,8 +931,8 @@ __global__ __launch_bounds__(WAVES * 64, 1) void gemm_skinny(const uint8_t* __re
   __syncthreads();
   if (wave < MT) {
     patch_put<FMT == FMT_I8>(sum, lds + wave * PATCH_WORDS, lane);
-    patch_store_inline<FMT == FMT_I8, ACT, true>(lds + wave * PATCH_WORDS, static_cast<uint8_t*>(C) + part * sp.plane,
-                                                 ldc, (int64_t)wave * 32, n0, M, N, e, lane, &pre);
+    patch_store_inline<FMT == FMT_I8, ACT, true>(lds + wave * PATCH_WORDS, C, ldc, (int64_t)wave * 32, n0, M, N, e,
+                                                 lane, &pre);
   }
 }
 
@@ -1022,11 +1023,11 @@ static int launch_pp(const void* a, const void* b, void* c, int64_t m, int64_t n
 
 template <int FMT, int MT, int STAGES>
 static int launch_skinny_mt(const SplitCall& g, int parts) {
-  Split sp{1, 0, g.n};
+  int64_t ldc = g.n;
   Epilogue e = g.e;
   void* c = g.c;
   if (parts > 1) {
-    sp = Split{parts, split_plane(g.m, g.n), split_ld(g.n)};
+    ldc = split_ld(g.n);
     e = plane_epilogue(FMT);
     c = g.workspace;
   }
@@ -1040,10 +1041,10 @@ static int launch_skinny_mt(const SplitCall& g, int parts) {
   do {                                                                                                           \
     if (act)                                                                                                     \
       hipLaunchKernelGGL((gemm_skinny<FMT, MT, 4, STAGES, true, AL>), grid, block, 0, g.stream,                  \
-                         (const uint8_t*)g.a, (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, sp.ld, e, sp); \
+                         (const uint8_t*)g.a, (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, ldc, e, parts); \
     else                                                                                                         \
       hipLaunchKernelGGL((gemm_skinny<FMT, MT, 4, STAGES, false, AL>), grid, block, 0, g.stream,                 \
-                         (const uint8_t*)g.a, (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, sp.ld, e, sp); \
+                         (const uint8_t*)g.a, (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, ldc, e, parts); \
   } while (0)
   if constexpr (MT == 1) {
     if (g.m <= 8) KRN_SKINNY(1);

@@ -5,11 +5,7 @@
 namespace krn {
 
 // K in `parts` runs of slices, one workgroup per tile and run. With more than one part each writes its sums, without
-// an epilogue, to a plane of its own (`plane` bytes apart, rows of `ld` elements); a second kernel adds the planes.
-struct Split {
-  int parts;
-  int64_t plane, ld;
-};
+// an epilogue, to a plane of its own (M rows of split_ld(N) four-byte elements); a second kernel adds the planes.
 
 // NN: where chunk c (8 columns) of k row k lies in its LDS row: the four k rows of a transposed read, 64 bytes each,
 // on distinct banks
@@ -33,7 +29,8 @@ struct SplitCall {
   hipStream_t stream;
 };
 
-// the planes' row length in elements: whole 32-byte pieces, so that every row is aligned for 16-byte accesses
+// the planes' row length in elements: whole 32-byte pieces, so that every row is aligned for 16-byte accesses; the
+// kernels get it as ldc, and find plane p at p * M * ldc elements
 inline int64_t split_ld(int64_t n) { return (n + 7) / 8 * 8; }
 inline int64_t split_plane(int64_t m, int64_t n) { return m * split_ld(n) * 4; }
 

@@ -39,10 +39,10 @@ __device__ __forceinline__ u32x4 drop_bytes(u32x4 v, int drop) {
 // AGPRs (a called function may use them) and copy all of them to VGPRs and back around every slice.
 template <bool INT, int TM, int TN, typename Acc>
 __device__ __forceinline__ void store_blocks(const Acc (&acc)[TM][TN], uint32_t* lds, int wave, void* C,
-                                             const Split& sp, int part, int64_t ldc, int64_t row0, int64_t col0,
-                                             int64_t M, int64_t N, const Epilogue& e, int lane) {
+                                             int part, int64_t ldc, int64_t row0, int64_t col0, int64_t M,
+                                             int64_t N, const Epilogue& e, int lane) {
   uint32_t* patch = lds + wave * TN * PATCH_WORDS;
-  void* out = static_cast<uint8_t*>(C) + part * sp.plane;
+  void* out = static_cast<uint8_t*>(C) + part * (M * ldc * 4);  // part 0 of one: C itself
 #pragma unroll
   for (int i = 0; i < TM; ++i) {
 #pragma unroll
@@ -58,7 +58,7 @@ __device__ __forceinline__ void store_blocks(const Acc (&acc)[TM][TN], uint32_t*
 template <int FMT, int BM, int BN, int WM, int WN, bool NN>
 __global__ __launch_bounds__(256, 2) void gemm_any(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                      void* __restrict__ C, int64_t M, int64_t N, int64_t kbytes,
-                                                     int64_t lda, int64_t ldb, int64_t ldc, Epilogue e, Split sp) {
+                                                     int64_t lda, int64_t ldb, int64_t ldc, Epilogue e, int parts) {
   typedef Mfma<FMT> Unit;
   typedef typename Unit::Acc Acc;
   constexpr int BKB = 128, TM = BM / WM / 32, TN = BN / WN / 32, STEP = Unit::kBytes, CH = STEP / 32;
@@ -80,7 +80,7 @@ __global__ __launch_bounds__(256, 2) void gemm_any(const uint8_t* __restrict__ A
   // all whole
   const int slices = (int)((kbytes + BKB - 1) / BKB), whole = (int)(kbytes / BKB);
   const int part = blockIdx.y;
-  const int first = (int)((int64_t)slices * part / sp.parts), n = (int)((int64_t)slices * (part + 1) / sp.parts) - first;
+  const int first = (int)((int64_t)slices * part / parts), n = (int)((int64_t)slices * (part + 1) / parts) - first;
   const bool tail = first + n > whole;
   const int kbase = tail ? first - 1 : first;
 
@@ -222,7 +222,7 @@ __global__ __launch_bounds__(256, 2) void gemm_any(const uint8_t* __restrict__ A
 #undef KRN_PUT
 #undef KRN_COMPUTE
 
-  store_blocks<FMT == FMT_I8>(acc, reinterpret_cast<uint32_t*>(lds), wave, C, sp, part, ldc, m0 + wm * (BM / WM),
+  store_blocks<FMT == FMT_I8>(acc, reinterpret_cast<uint32_t*>(lds), wave, C, part, ldc, m0 + wm * (BM / WM),
                               n0 + wn * (BN / WN), M, N, e, lane);
 }
 
@@ -256,7 +256,7 @@ __device__ __forceinline__ void tr_read(uint8_t* p, u32x4 (&f)[4]) {
 template <int FMT, int BM, int BN, int WM, int WN, int STAGES, bool NN>
 __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                      void* __restrict__ C, int64_t M, int64_t N, int64_t kbytes,
-                                                     int64_t lda, int64_t ldb, int64_t ldc, Epilogue e, Split sp) {
+                                                     int64_t lda, int64_t ldb, int64_t ldc, Epilogue e, int parts) {
   typedef Mfma<FMT> Unit;
   typedef typename Unit::Acc Acc;
   constexpr int BKB = 128, TM = BM / WM / 32, TN = BN / WN / 32, STEP = Unit::kBytes, CH = STEP / 32, KS = BKB / STEP;
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
   const int wm = wave / WN, wn = wave % WN, half = lane >> 5, r32 = lane & 31;
   const int slices = (int)((kbytes + BKB - 1) / BKB), whole = (int)(kbytes / BKB);
   const int part = blockIdx.y;
-  const int first = (int)((int64_t)slices * part / sp.parts), n = (int)((int64_t)slices * (part + 1) / sp.parts) - first;
+  const int first = (int)((int64_t)slices * part / parts), n = (int)((int64_t)slices * (part + 1) / parts) - first;
   const bool tail = first + n > whole;  // this part ends with the partial slice: it is taken first
   const int kbase = tail ? first - 1 : first;
 
@@ -380,7 +380,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
 #undef KRN_VMWAIT
 #undef KRN_SLICE
   __syncthreads();  // every wave is done with the ring before its LDS becomes the store patches
-  store_blocks<FMT == FMT_I8>(acc, reinterpret_cast<uint32_t*>(lds), wave, C, sp, part, ldc, m0 + wm * (BM / WM),
+  store_blocks<FMT == FMT_I8>(acc, reinterpret_cast<uint32_t*>(lds), wave, C, part, ldc, m0 + wm * (BM / WM),
                               n0 + wn * (BN / WN), M, N, e, lane);
 }
 
@@ -388,16 +388,16 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
 // parts have just left in the caches (256 x 4096, four parts: 17 MB).
 template <bool INT>
 __global__ __launch_bounds__(256) void split_reduce(const uint8_t* __restrict__ planes, void* __restrict__ C, int64_t M,
-                                                    int64_t N, Split sp, Epilogue e) {
-  const int64_t per_row = sp.ld / 8, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
+                                                    int64_t N, int64_t ld, int parts, Epilogue e) {
+  const int64_t per_row = ld / 8, at = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t m = at / per_row, n = at % per_row * 8;
   if (m >= M) return;
   typedef std::conditional_t<INT, i32x4, f32x4> V;
-  const uint8_t* from = planes + (m * sp.ld + n) * 4;
+  const uint8_t* from = planes + (m * ld + n) * 4;
   V lo = *reinterpret_cast<const V*>(from), hi = *reinterpret_cast<const V*>(from + 16);
 #pragma unroll 4
-  for (int p = 1; p < sp.parts; ++p) {
-    from += sp.plane;
+  for (int p = 1; p < parts; ++p) {
+    from += M * ld * 4;
     lo += *reinterpret_cast<const V*>(from);
     hi += *reinterpret_cast<const V*>(from + 16);
   }
@@ -470,35 +470,35 @@ static int launched(const char* what) {
 }
 
 int krn::launch_reduce(int fmt, int parts, const SplitCall& g) {
-  const Split sp{parts, split_plane(g.m, g.n), split_ld(g.n)};
-  const dim3 blocks((unsigned)((g.m * (sp.ld / 8) + 255) / 256));
+  const int64_t ld = split_ld(g.n);
+  const dim3 blocks((unsigned)((g.m * (ld / 8) + 255) / 256));
   if (fmt == FMT_I8)
     hipLaunchKernelGGL(split_reduce<true>, blocks, dim3(256), 0, g.stream, (const uint8_t*)g.workspace, g.c, g.m, g.n,
-                       sp, g.e);
+                       ld, parts, g.e);
   else
     hipLaunchKernelGGL(split_reduce<false>, blocks, dim3(256), 0, g.stream, (const uint8_t*)g.workspace, g.c, g.m, g.n,
-                       sp, g.e);
+                       ld, parts, g.e);
   return launched("gemm reduction");
 }
 
 template <int FMT, int BM, int BN, int WM, int WN, int STAGES, bool NN>
 static int launch(const SplitCall& g, int parts) {  // STAGES = 0: the loader for any alignment
   const int64_t tiles = ((g.m + BM - 1) / BM) * ((g.n + BN - 1) / BN);
-  Split sp{parts, 0, g.n};
+  int64_t ldc = g.n;
   Epilogue e = g.e;
   void* c = g.c;
   if (parts > 1) {
     c = g.workspace;
-    sp = Split{parts, split_plane(g.m, g.n), split_ld(g.n)};
+    ldc = split_ld(g.n);
     e = plane_epilogue(FMT);
   }
   const dim3 grid((unsigned)tiles, (unsigned)parts), block(WM * WN * 64);
   if constexpr (STAGES > 0)
     hipLaunchKernelGGL((gemm_ring<FMT, BM, BN, WM, WN, STAGES, NN>), grid, block, 0, g.stream, (const uint8_t*)g.a,
-                       (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, sp.ld, e, sp);
+                       (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, ldc, e, parts);
   else
     hipLaunchKernelGGL((gemm_any<FMT, BM, BN, WM, WN, NN>), grid, block, 0, g.stream, (const uint8_t*)g.a,
-                       (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, sp.ld, e, sp);
+                       (const uint8_t*)g.b, c, g.m, g.n, g.kbytes, g.lda, g.ldb, ldc, e, parts);
   const int rc = launched("gemm");
   return rc != 0 || parts == 1 ? rc : launch_reduce(FMT, parts, g);
 }

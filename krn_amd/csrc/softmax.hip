@@ -8,108 +8,95 @@
 // past its tile) are neither read nor written; a row is a run of valid lanes, so no padding value enters the
 // maximum or the sum.
 //
-// Layout (HBM-bound: one read, one write per element). One wave per row, four rows per workgroup, no LDS and no
-// barriers (or, for at most 4096 rows longer than 2048 columns, four waves per row): lane l owns the 8-element
-// chunks l, l + 64, ...; it keeps a running maximum m and sum s of its chunks (s rescaled by exp(m_old - m_new)
-// when m grows), the wave combines the 64 pairs by shuffles, and a second pass writes exp(x - m) * (1 / s). Up to
-// CACHE chunks per lane stay in registers between the passes, so those rows are read from HBM once; longer rows
-// are read again (from L2).
+// Layout (HBM-bound: one read, one write per element). A row belongs to one wave (four rows per workgroup), four waves
+// or sixteen: thread l owns the 16-byte chunks l, l + T, ... of its row. Up to CACHE chunks per thread stay in registers
+// as they were read, so rows of up to 65536 16-bit columns are read from HBM once; longer rows are read again (from
+// L2). A thread keeps a running maximum m and sum s of exp(x - m) over its chunks as they arrive (the maximum of all of
+// them first: f16 8192 x 2048 12.6 -> 13.1 us), the threads' pairs meet by shuffles and in LDS, and a second pass writes
+// exp(x - m) * (1 / s).
+//
+// Rows may start at any element: the chunks are loaded and stored 16 bytes at a time at any alignment, and only a chunk
+// that crosses the end of its row goes element by element (bf16 1024 x 50001, rows at every alignment, element by
+// element before: 145 -> 59 us; the copy of as many bytes takes 31).
 #include "common.h"
 
 namespace krn {
 
 constexpr float LOG2E = 1.4426950408889634f;
+typedef u32x4 u32x4_any __attribute__((aligned(1)));  // a 16-byte access at any address
 
-// Eight elements of row `row` from chunk `c` as float32; lanes at or past `width` read -infinity (they then add
-// exp(-inf) = 0 to the sum and never win the maximum)
 template <int KIND>
-__device__ __forceinline__ void load8(const void* X, int64_t row, int64_t ld, int64_t c, int64_t width, bool vec,
-                                      float* v) {
-  const int64_t col = c * 8;
-  if (vec && col + 8 <= width) {
-    if constexpr (KIND == F32) {
-      const f32x4* p = reinterpret_cast<const f32x4*>(static_cast<const float*>(X) + row * ld + col);
-      const f32x4 a = p[0], b = p[1];
-      v[0] = a[0], v[1] = a[1], v[2] = a[2], v[3] = a[3], v[4] = b[0], v[5] = b[1], v[6] = b[2], v[7] = b[3];
-    } else {
-      const u32x4 w = *reinterpret_cast<const u32x4*>(static_cast<const uint16_t*>(X) + row * ld + col);
+struct Chunk {  // 16 bytes of a row
+  static constexpr int N = KIND == F32 ? 4 : 8;
+  static constexpr int BYTES = KIND == F32 ? 4 : 2;
+  __device__ static float value(const u32x4& w, int e) {
+    if constexpr (KIND == F32) return __uint_as_float(w[e]);
+    const uint16_t h = (uint16_t)(w[e >> 1] >> ((e & 1) * 16));
+    return KIND == F16 ? h2f(h) : bf2f(h);
+  }
+  __device__ static void set(u32x4& w, int e, float v) {  // into a zeroed chunk
+    if constexpr (KIND == F32) w[e] = __float_as_uint(v);
+    else w[e >> 1] |= (uint32_t)(KIND == F16 ? f2h(v) : f2bf(v)) << ((e & 1) * 16);
+  }
+  static constexpr uint32_t LOWEST = KIND == F32 ? 0xff800000u : KIND == F16 ? 0xfc00fc00u : 0xff80ff80u;  // -infinity
+};
+
+// Chunk c of a row; elements at or past `width` are -infinity (they add exp(-inf) = 0 to the sum and never win the
+// maximum), and so is a chunk past the row
+template <int KIND>
+__device__ __forceinline__ u32x4 load_chunk(const uint8_t* row, int64_t c, int64_t width) {
+  typedef Chunk<KIND> C;
+  const int64_t col = c * C::N;
+  if (col + C::N <= width) return *reinterpret_cast<const u32x4_any*>(row + col * C::BYTES);
+  u32x4 w = {C::LOWEST, C::LOWEST, C::LOWEST, C::LOWEST};
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint16_t lo = (uint16_t)(w[q] & 0xffff), hi = (uint16_t)(w[q] >> 16);
-        v[2 * q] = KIND == F16 ? h2f(lo) : bf2f(lo);
-        v[2 * q + 1] = KIND == F16 ? h2f(hi) : bf2f(hi);
+  for (int e = 0; e < C::N; ++e)
+    if (col + e < width) {
+      if constexpr (KIND == F32) {
+        w[e] = reinterpret_cast<const uint32_t*>(row)[col + e];
+      } else {
+        const uint32_t h = reinterpret_cast<const uint16_t*>(row)[col + e];
+        w[e >> 1] = (e & 1) ? (w[e >> 1] & 0xffffu) | h << 16 : (w[e >> 1] & 0xffff0000u) | h;
       }
     }
+  return w;
+}
+
+// NaN if an element of the chunk is (the maximum passes over NaN), otherwise 0
+template <int KIND>
+__device__ __forceinline__ float nan_of(const u32x4& w) {
+  float s = 0.0f;
+#pragma unroll
+  for (int e = 0; e < Chunk<KIND>::N; ++e) {
+    const float x = Chunk<KIND>::value(w, e);
+    s = x != x ? x : s;
+  }
+  return s;
+}
+
+// exp(x - m) * inv of a chunk, rounded once, to the output. Chunks at 16-byte addresses are stored non-temporally: the
+// output is not read again, and a wave's store covers whole lines (f16 32768 x 4096: 5.0 -> 6.5 TB/s). Unaligned ones
+// share their first and last lines with their neighbours and keep ordinary stores, which the L2 joins.
+template <int KIND, bool ALIGNED>
+__device__ __forceinline__ void store_chunk(uint8_t* row, int64_t c, int64_t width, const u32x4& x, float m, float inv) {
+  typedef Chunk<KIND> C;
+  const int64_t col = c * C::N;
+  u32x4 w = {0, 0, 0, 0};
+#pragma unroll
+  for (int e = 0; e < C::N; ++e) C::set(w, e, __builtin_amdgcn_exp2f((C::value(x, e) - m) * LOG2E) * inv);
+  if (col + C::N <= width) {
+    if constexpr (ALIGNED) __builtin_nontemporal_store(w, reinterpret_cast<u32x4*>(row + col * C::BYTES));
+    else *reinterpret_cast<u32x4_any*>(row + col * C::BYTES) = w;
     return;
   }
 #pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int64_t at = col + e;
-    if (at < width) {
-      if constexpr (KIND == F32) v[e] = static_cast<const float*>(X)[row * ld + at];
-      else {
-        const uint16_t h = static_cast<const uint16_t*>(X)[row * ld + at];
-        v[e] = KIND == F16 ? h2f(h) : bf2f(h);
-      }
-    } else {
-      v[e] = -INFINITY;
+  for (int e = 0; e < C::N; ++e)
+    if (col + e < width) {
+      if constexpr (KIND == F32) reinterpret_cast<uint32_t*>(row)[col + e] = w[e];
+      else reinterpret_cast<uint16_t*>(row)[col + e] = (uint16_t)(w[e >> 1] >> ((e & 1) * 16));
     }
-  }
 }
 
-// Whole 16-bit chunks (one 16-byte store per lane, lanes contiguous) are stored non-temporally: the output is not read
-// again by this kernel, and keeping it out of the caches' way lifts f16 32768 x 4096 from 5.0 to 6.5 TB/s. float32
-// chunks are two 16-byte stores 32 bytes apart per lane, half lines per instruction, which are slower non-temporal
-// (8192 x 4096: 0.047 -> 0.067 ms), so they keep ordinary stores.
-template <int KIND>
-__device__ __forceinline__ void store8(void* Y, int64_t row, int64_t ld, int64_t c, int64_t width, bool vec,
-                                       const float* v) {
-  const int64_t col = c * 8;
-  if (vec && col + 8 <= width) {
-    if constexpr (KIND == F32) {
-      f32x4* p = reinterpret_cast<f32x4*>(static_cast<float*>(Y) + row * ld + col);
-      p[0] = f32x4{v[0], v[1], v[2], v[3]};
-      p[1] = f32x4{v[4], v[5], v[6], v[7]};
-    } else {
-      uint32_t w[4];
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const uint32_t lo = KIND == F16 ? f2h(v[2 * q]) : f2bf(v[2 * q]);
-        const uint32_t hi = KIND == F16 ? f2h(v[2 * q + 1]) : f2bf(v[2 * q + 1]);
-        w[q] = lo | (hi << 16);
-      }
-      __builtin_nontemporal_store(u32x4{w[0], w[1], w[2], w[3]},
-                                  reinterpret_cast<u32x4*>(static_cast<uint16_t*>(Y) + row * ld + col));
-    }
-    return;
-  }
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const int64_t at = col + e;
-    if (at < width) {
-      if constexpr (KIND == F32) static_cast<float*>(Y)[row * ld + at] = v[e];
-      else static_cast<uint16_t*>(Y)[row * ld + at] = KIND == F16 ? f2h(v[e]) : f2bf(v[e]);
-    }
-  }
-}
-
-// (m, s) += the eight values: m the running maximum, s the sum of exp(x - m)
-__device__ __forceinline__ void accumulate(float& m, float& s, const float* v) {
-  float top = v[0];
-#pragma unroll
-  for (int e = 1; e < 8; ++e) top = fmaxf(top, v[e]);
-  const float m_new = fmaxf(m, top);
-  if (m_new == -INFINITY) return;  // nothing valid yet
-  float add = 0.0f;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) add += __builtin_amdgcn_exp2f((v[e] - m_new) * LOG2E);
-  s = s * __builtin_amdgcn_exp2f((m - m_new) * LOG2E) + add;
-  m = m_new;
-}
-
-// SPLIT waves share one row (4 / SPLIT rows per workgroup): lane t of the row's 64 * SPLIT owns chunks t, t + 64 *
-// SPLIT, ...; with SPLIT > 1 the waves' (m, s) pairs meet in LDS. One wave per row fills the chip when rows are
-// many; a whole workgroup per row keeps enough loads in flight when few long rows are all there is.
 // (m, s) and (m2, s2) merged: both sums rescaled to the larger maximum
 __device__ __forceinline__ void combine(float& m, float& s, float m2, float s2) {
   const float m_new = fmaxf(m, m2);
@@ -118,86 +105,118 @@ __device__ __forceinline__ void combine(float& m, float& s, float m2, float s2) 
   m = m_new;
 }
 
-template <int KIND, int CACHE, int SPLIT>
-__global__ __launch_bounds__(256) void softmax_rows(const void* __restrict__ X, void* __restrict__ Y, int64_t rows,
-                                                   int64_t width, int64_t ldx, int64_t ldy) {
-  constexpr int STRIDE = 64 * SPLIT;
-  const int lane = threadIdx.x % STRIDE;
-  const int64_t row = (int64_t)blockIdx.x * (4 / SPLIT) + threadIdx.x / STRIDE;
-  if constexpr (SPLIT == 1) {
+// One wave per row fills the chip when rows are many and fit its registers; more waves keep long rows in registers and
+// enough loads in flight when rows are few.
+template <int KIND, int CACHE, int WAVES, bool ALIGNED>
+__global__ __launch_bounds__(WAVES == 1 ? 256 : WAVES * 64) void softmax_rows(const uint8_t* __restrict__ X,
+                                                                               uint8_t* __restrict__ Y, int64_t rows,
+                                                                               int64_t width, int64_t ldx, int64_t ldy) {
+  typedef Chunk<KIND> C;
+  constexpr int T = WAVES * 64;
+  const int lane = threadIdx.x % T;
+  const int64_t row = WAVES == 1 ? (int64_t)blockIdx.x * 4 + threadIdx.x / 64 : blockIdx.x;
+  if constexpr (WAVES == 1) {
     if (row >= rows) return;  // a whole wave leaves together; no barrier follows
   }
-  const int64_t chunks = (width + 7) / 8;
-  const int esize = KIND == F32 ? 4 : 2;
-  const bool vec = (ldx * esize) % 16 == 0 && (ldy * esize) % 16 == 0 && (uintptr_t)X % 16 == 0 &&
-                   (uintptr_t)Y % 16 == 0;
+  const int64_t chunks = (width + C::N - 1) / C::N;
+  const uint8_t* x = X + row * ldx * C::BYTES;
+  uint8_t* y = Y + row * ldy * C::BYTES;
+  u32x4 kept[CACHE];
+#pragma unroll
+  for (int i = 0; i < CACHE; ++i) kept[i] = load_chunk<KIND>(x, lane + T * i, width);
   float m = -INFINITY, s = 0.0f;
-  float kept[CACHE][8];
+  // before the second pass: the chunks stay as they were read (the compiler would keep all their float32 values, twice
+  // the registers)
+#define KRN_OPAQUE() _Pragma("unroll") for (int i = 0; i < CACHE; ++i) asm volatile("" : "+v"(kept[i]))
 #pragma unroll
   for (int i = 0; i < CACHE; ++i) {
-    const int64_t c = lane + STRIDE * i;
-    if (c < chunks) load8<KIND>(X, row, ldx, c, width, vec, kept[i]);
+    float top = m;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) kept[i][e] = c < chunks ? kept[i][e] : -INFINITY;
-    accumulate(m, s, kept[i]);
+    for (int e = 0; e < C::N; ++e) top = fmaxf(top, C::value(kept[i], e));
+    if (top == -INFINITY) {  // nothing valid yet, or NaN
+      s += nan_of<KIND>(kept[i]);
+      continue;
+    }
+    float add = 0.0f;
+#pragma unroll
+    for (int e = 0; e < C::N; ++e) add += __builtin_amdgcn_exp2f((C::value(kept[i], e) - top) * LOG2E);
+    s = s * __builtin_amdgcn_exp2f((m - top) * LOG2E) + add;
+    m = top;
   }
-  for (int64_t c = lane + STRIDE * CACHE; c < chunks; c += STRIDE) {
-    float v[8];
-    load8<KIND>(X, row, ldx, c, width, vec, v);
-    accumulate(m, s, v);
+  for (int64_t c = lane + T * CACHE; c < chunks; c += T) {
+    const u32x4 w = load_chunk<KIND>(x, c, width);
+    float top = C::value(w, 0), add = 0.0f;
+#pragma unroll
+    for (int e = 1; e < C::N; ++e) top = fmaxf(top, C::value(w, e));
+    if (!(top > -INFINITY)) {
+      s += nan_of<KIND>(w);
+      continue;
+    }
+#pragma unroll
+    for (int e = 0; e < C::N; ++e) add += __builtin_amdgcn_exp2f((C::value(w, e) - top) * LOG2E);
+    combine(m, s, top, add);
   }
-  // the wave's maximum and sum: pairs combined by shuffles
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) combine(m, s, __shfl_xor(m, off), __shfl_xor(s, off));
-  if constexpr (SPLIT > 1) {
-    __shared__ float part[2][4];
+  if constexpr (WAVES > 1) {
+    __shared__ float part[2][WAVES];
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) part[0][wave] = m, part[1][wave] = s;
     __syncthreads();
     m = part[0][0], s = part[1][0];
 #pragma unroll
-    for (int w = 1; w < SPLIT; ++w) combine(m, s, part[0][w], part[1][w]);
+    for (int w = 1; w < WAVES; ++w) combine(m, s, part[0][w], part[1][w]);
   }
   const float inv = 1.0f / s;
+  KRN_OPAQUE();
+#undef KRN_OPAQUE
 #pragma unroll
-  for (int i = 0; i < CACHE; ++i) {
-    const int64_t c = lane + STRIDE * i;
-    if (c < chunks) {
-      float y[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = __builtin_amdgcn_exp2f((kept[i][e] - m) * LOG2E) * inv;
-      store8<KIND>(Y, row, ldy, c, width, vec, y);
-    }
-  }
-  for (int64_t c = lane + STRIDE * CACHE; c < chunks; c += STRIDE) {
-    float v[8], y[8];
-    load8<KIND>(X, row, ldx, c, width, vec, v);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) y[e] = __builtin_amdgcn_exp2f((v[e] - m) * LOG2E) * inv;
-    store8<KIND>(Y, row, ldy, c, width, vec, y);
-  }
+  for (int i = 0; i < CACHE; ++i)
+    if (lane + T * i < chunks) store_chunk<KIND, ALIGNED>(y, lane + T * i, width, kept[i], m, inv);
+  for (int64_t c = lane + T * CACHE; c < chunks; c += T)
+    store_chunk<KIND, ALIGNED>(y, c, width, load_chunk<KIND>(x, c, width), m, inv);
 }
 
 }  // namespace krn
 
 using namespace krn;
 
+template <int KIND, int CACHE, int WAVES>
+static void launch_rows(bool aligned, const void* x, void* y, int64_t rows, int64_t width, int64_t ldx, int64_t ldy,
+                        hipStream_t stream) {
+  const dim3 grid((unsigned)(WAVES == 1 ? (rows + 3) / 4 : rows)), block(WAVES == 1 ? 256 : WAVES * 64);
+  if (aligned)
+    hipLaunchKernelGGL((softmax_rows<KIND, CACHE, WAVES, true>), grid, block, 0, stream, (const uint8_t*)x, (uint8_t*)y,
+                       rows, width, ldx, ldy);
+  else
+    hipLaunchKernelGGL((softmax_rows<KIND, CACHE, WAVES, false>), grid, block, 0, stream, (const uint8_t*)x, (uint8_t*)y,
+                       rows, width, ldx, ldy);
+}
+
 template <int KIND>
 static int launch_softmax(const void* x, void* y, int64_t rows, int64_t width, int64_t ldx, int64_t ldy,
                           hipStream_t stream) {
-  const dim3 block(256);
-  if (rows <= 4096 && width > 2048) {
-    // few long rows: a workgroup per row; up to 16384 columns stay in registers between the passes
-    hipLaunchKernelGGL((softmax_rows<KIND, 8, 4>), dim3((unsigned)rows), block, 0, stream, x, y, rows, width, ldx,
-                       ldy);
+  constexpr int N = Chunk<KIND>::N;
+  const bool aligned = (ldy * Chunk<KIND>::BYTES) % 16 == 0 && (uintptr_t)y % 16 == 0;
+  const int64_t chunks = (width + N - 1) / N;
+#define KRN_ROWS(CACHE, WAVES) launch_rows<KIND, CACHE, WAVES>(aligned, x, y, rows, width, ldx, ldy, stream)
+  // chunks per thread that stay in registers (no more than the row needs: bf16 20000 x 1000 on two 14.9 us, on four
+  // 18.4): a wave's row up to 512 chunks (4096 16-bit columns), four waves' up to
+  // 2048, sixteen waves' up to 8192; longer rows are read again. Few rows of more than 256 chunks take four waves for
+  // the loads in flight.
+  if (chunks <= 512 && !(rows <= 4096 && chunks > 256)) {
+    if (chunks <= 64) KRN_ROWS(1, 1);
+    else if (chunks <= 128) KRN_ROWS(2, 1);
+    else if (chunks <= 256) KRN_ROWS(4, 1);
+    else KRN_ROWS(8, 1);
+  } else if (chunks <= 1024) {
+    KRN_ROWS(4, 4);
+  } else if (chunks <= 2048) {
+    KRN_ROWS(8, 4);
   } else {
-    // a wave per row; up to 2048 (4096) columns stay in registers, longer rows are read again from L2
-    const dim3 grid((unsigned)((rows + 3) / 4));
-    if (width <= 8 * 64 * 4)
-      hipLaunchKernelGGL((softmax_rows<KIND, 4, 1>), grid, block, 0, stream, x, y, rows, width, ldx, ldy);
-    else
-      hipLaunchKernelGGL((softmax_rows<KIND, 8, 1>), grid, block, 0, stream, x, y, rows, width, ldx, ldy);
+    KRN_ROWS(8, 16);
   }
+#undef KRN_ROWS
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {
     krn_set_error("softmax launch: %s", hipGetErrorString(err));

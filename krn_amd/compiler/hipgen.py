@@ -1,12 +1,12 @@
 """Generic lowering of any captured tile program to HIP C++ for gfx950, compiled at run time with hiprtc.
 
 This is the path for tile programs that are not one of the contraction shapes the hand-written MFMA kernels serve
-(`cdna4.lower` decides). One workgroup of 256 threads runs one block; every tile lives in LDS with a validity byte
-per lane; each tile statement is an element loop strided over the workgroup followed by a barrier. Its arithmetic is
+(`cdna4.lower` decides). One workgroup of 256 threads runs one block; tile variables live in LDS with a validity byte
+per lane; a tile statement is one loop over its elements, strided over the workgroup. Its arithmetic is
 the tile semantics of krn's C-family lowering (reference src/krn/compiler/emit.py): a product stages both operands
 as float32 (invalid lanes zero) and runs one fused multiply-add per k in k order for each output element
-(emit.py:788-796), a reduction walks its axis over the valid lanes from the first one (emit.py:997-1034), stores
-skip invalid lanes and elements outside the tensor. The kernel ABI is krn's generated-kernel ABI
+(emit.py:788-796), a reduction takes the valid lanes of its axis from the first one (emit.py:997-1034; float32 sums in
+up to 64 interleaved parts), stores skip invalid lanes and elements outside the tensor. The kernel ABI is krn's generated-kernel ABI
 (reference src/krn/compiler/cuda.py:319 and ir.py:441-452): `extern "C" __global__`, a tensor is a pointer plus one
 `long long` extent per axis, scalars by value.
 """
@@ -157,52 +157,125 @@ def products(kernel: ir.Kernel) -> list[str]:
     return found
 
 
+Access = tuple[tuple, str]  # a resource (("lds", first byte, end byte) or ("tensor", name)) and how it is indexed
+
+
 class Emitter:
+    """The source of one kernel. A statement's elementwise operations run fused, in one loop over its elements, each
+    operation one rounded line; tile variables live in LDS, and so do the intermediate tiles that other threads read
+    (reductions, staged product operands, transposed loads), in memory that the next statement reuses: a program's
+    footprint is its variables and the largest statement, not every operation (flash attention with 64 x 64 tiles and
+    d = 32: 321 KiB, in global scratch, before; 16 heads of 512 took 1270 us).
+
+    Loops over the same elements need no barrier between them when each reads only what its own thread wrote: `sync`
+    keeps what has been read and written since the last barrier and puts one only before a conflict."""
+
     def __init__(self, kernel: ir.Kernel, entry: str) -> None:
         self.kernel, self.entry = kernel, entry
         self.mfma_products = 0
         self.lines: list[str] = []
-        self.buffers: list[tuple[str, str, int]] = []
         self.depth = 1
         self.count = 0
+        self.names: dict[str, tuple[str, int, int]] = {}  # buffer -> element type, offset, bytes
+        self.order: list[str] = []  # buffers in the order of their declaration
+        self.top = self.peak = 0  # the statement's end of used memory, and the most any statement uses
         self.tile_vars: dict[str, tuple[str, str]] = {}
+        self.node: dict[int, object] = {}  # what a statement has prepared for its expressions, by identity
+        self.memo: dict[tuple, tuple[str, str]] = {}
+        self.reads: list[Access] = []
+        self.writes: list[Access] = []
+        self.pending: list[tuple[Access, bool]] = []  # since the last barrier: access, whether it wrote
 
     def put(self, text: str) -> None:
         self.lines.append("  " * self.depth + text)
 
+    def fresh(self, stem: str) -> str:
+        self.count += 1
+        return f"_{stem}{self.count}"
+
+    # ---- memory
+
+    def reserve(self, name: str, element: str, size: int) -> str:
+        nbytes = (SIZES[element] * max(size, 1) + 15) // 16 * 16
+        self.names[name] = (element, self.top, nbytes)
+        self.order.append(name)
+        self.top += nbytes
+        self.peak = max(self.peak, self.top)
+        return name
+
     def buffer(self, dtype: Dtype, shape: tuple[int, ...], stem: str = "t") -> tuple[str, str]:
         self.count += 1
         size = math.prod(shape) if shape else 1
-        value, valid = f"{stem}{self.count}", f"{stem}{self.count}_v"
-        self.buffers.append((value, ctype(dtype), size))
-        self.buffers.append((valid, "unsigned char", size))
-        return value, valid
+        return (self.reserve(f"{stem}{self.count}", ctype(dtype), size),
+                self.reserve(f"{stem}{self.count}_v", "unsigned char", size))
 
-    def loop(self, shape: tuple[int, ...], body) -> None:
-        size = math.prod(shape)
-        self.put(f"for (int _e = threadIdx.x; _e < {size}; _e += {THREADS}) {{")
-        self.depth += 1
-        names = []
-        for a in range(len(shape)):
-            self.put(f"const int _i{a} = _e / {math.prod(shape[a + 1:])} % {shape[a]};")
-            names.append(f"_i{a}")
-        body(names)
-        self.depth -= 1
-        self.put("}")
-        self.put("__syncthreads();")
+    def access(self, name: str, pattern: str, write: bool = False) -> None:
+        """Note that the loop being emitted touches buffer `name` at `pattern`: "e<size>" is the element of the
+        thread's own index in a loop over <size> elements, "any" everything else."""
+        _, start, nbytes = self.names[name]
+        (self.writes if write else self.reads).append((("lds", start, start + nbytes), pattern))
 
     @staticmethod
-    def index(idx: list[str], of: tuple[int, ...]) -> str:
-        """Linear index into a tile of shape `of` broadcast numpy-style (aligned from the right) to the loop `idx`."""
-        if not of:
-            return "0"
+    def conflict(a: Access, b: Access) -> bool:
+        (ra, pa), (rb, pb) = a, b
+        if ra[0] != rb[0] or (ra[0] == "tensor" and ra[1] != rb[1]):
+            return False
+        if ra[0] == "lds" and (ra[2] <= rb[1] or rb[2] <= ra[1]):
+            return False
+        return pa == "any" or pa != pb or ra != rb
+
+    def sync(self, reads: list[Access], writes: list[Access]) -> None:
+        """A barrier if these accesses meet one since the last barrier that another thread may have made."""
+        if any(self.conflict(w, old) for w in writes for old, _ in self.pending) or any(
+                self.conflict(r, old) for r in reads for old, wrote in self.pending if wrote):
+            self.barrier()
+        self.pending += [(r, False) for r in reads] + [(w, True) for w in writes]
+
+    def barrier(self) -> None:
+        self.put("__syncthreads();")
+        self.pending = []
+
+    def region(self, emit) -> None:
+        """The lines `emit` puts, after the barrier their accesses need."""
+        outer, reads, writes = self.lines, self.reads, self.writes
+        self.lines, self.reads, self.writes, self.memo = [], [], [], {}
+        emit()
+        inner, self.lines = self.lines, outer
+        self.sync(self.reads, self.writes)
+        self.lines += inner
+        self.reads, self.writes, self.memo = reads, writes, {}
+
+    def loop(self, shape: tuple[int, ...], body) -> None:
+        """`body(index names)` for every element of `shape`, strided over the workgroup."""
+        def emit() -> None:
+            self.put(f"for (int _e = threadIdx.x; _e < {math.prod(shape)}; _e += {THREADS}) {{")
+            self.depth += 1
+            names = []
+            for a in range(len(shape)):
+                self.put(f"const int _i{a} = _e / {math.prod(shape[a + 1:])} % {shape[a]};")
+                names.append(f"_i{a}")
+            body(names)
+            self.depth -= 1
+            self.put("}")
+
+        self.region(emit)
+
+    @staticmethod
+    def aligned(idx: list[str], of: tuple[int, ...]) -> list[str]:
+        """The indices of a tile of shape `of` broadcast numpy-style (aligned from the right) to the loop `idx`."""
         skip = len(idx) - len(of)
-        terms = [f"{idx[a + skip]} * {math.prod(of[a + 1:])}" for a, extent in enumerate(of) if extent != 1]
-        return " + ".join(terms) or "0"
+        return ["0" if extent == 1 else idx[a + skip] for a, extent in enumerate(of)]
+
+    @staticmethod
+    def linear(idx: list[str], of: tuple[int, ...]) -> str:
+        return " + ".join(f"{i} * {math.prod(of[a + 1:])}" for a, i in enumerate(idx) if i != "0") or "0"
+
+    # ---- the kernel
 
     def emit(self) -> tuple[str, int]:
         for var in self.kernel.tiles:
             self.tile_vars[var.name] = self.buffer(var.dtype, var.shape, stem=f"v_{var.name.strip('_')}_")
+        self.fixed = self.top  # bytes of the variables; the statements' temporaries follow
         self.body(self.kernel.body)
         params = []
         for name, kind in self.kernel.params:
@@ -211,7 +284,7 @@ class Emitter:
                     params.append(f"{storage(dtype)}* __restrict__ {slot}")
                 else:
                     params.append(f"{ctype(dtype if dtype != I64 else PY_INT)} {slot}")
-        total = sum((SIZES[c] * n + 15) // 16 * 16 for _, c, n in self.buffers)
+        total = self.peak
         scratch = total > LDS_LIMIT  # tiles beyond one CU's LDS live in a per-block slice of global scratch
         if scratch:
             params.append("char* __restrict__ _scratch")
@@ -219,12 +292,15 @@ class Emitter:
         if scratch:
             head.append(f"  char* _block = _scratch + ((long long)blockIdx.x + (long long)blockIdx.y * gridDim.x + "
                         f"(long long)blockIdx.z * gridDim.x * gridDim.y) * {total}LL;")
-            offset = 0
-            for name, c, n in self.buffers:
-                head.append(f"  {c}* __restrict__ {name} = ({c}*)(_block + {offset});")
-                offset += (SIZES[c] * n + 15) // 16 * 16
         else:
-            head += [f"  __shared__ __attribute__((aligned(16))) {c} {name}[{n}];" for name, c, n in self.buffers]
+            head.append(f"  __shared__ __attribute__((aligned(16))) char _block[{max(total - self.fixed, 16)}];")
+        for name in self.order:
+            element, offset, nbytes = self.names[name]
+            if offset < self.fixed and not scratch:
+                # a variable is an array of its own, which the compiler can tell from the others
+                head.append(f"  __shared__ __attribute__((aligned(16))) {element} {name}[{nbytes // SIZES[element]}];")
+            else:
+                head.append(f"  {element}* {name} = ({element}*)(_block + {offset - (0 if scratch else self.fixed)});")
         self.scratch_bytes = total if scratch else 0
         head += ["  const long long bx = blockIdx.x, by = blockIdx.y, bz = blockIdx.z;",
                  "  (void)bx; (void)by; (void)bz;"]
@@ -232,149 +308,476 @@ class Emitter:
 
     def body(self, statements) -> None:
         for s in statements:
+            mark, self.node = self.top, {}
             getattr(self, f"stmt_{type(s).__name__}")(s)
+            self.top = mark  # the statement's temporaries are dead
+
+    # ---- expressions: `prepare` before the loop, `value` inside it
+
+    def prepare(self, e: ir.Expr, product: bool = False) -> None:
+        """What an expression's elements need before a loop can compute them: the starts of its loads, the results of
+        its reductions, a transposed load turned through LDS (in a product the staging loop turns it)."""
+        if id(e) in self.node or not e.shape or isinstance(e, ir.Var):
+            return
+        match e:
+            case ir.TileLoad(slices=slices):
+                starts = [self.fresh("s") for _ in slices]
+                for name, sl in zip(starts, slices):
+                    self.put(f"const long long {name} = {self.scalar(sl.start)};")
+                self.node[id(e)] = starts
+            case ir.Arange(start=start):
+                name = self.fresh("s")
+                self.put(f"const long long {name} = {self.scalar(start)};")
+                self.node[id(e)] = name
+            case ir.Reduce():
+                self.prepare(e.operand)
+                self.node[id(e)] = self.reduce(e)
+            case ir.Transpose(operand=o) if not product and self.loads(o):
+                self.prepare(o)
+                self.node[id(e)] = self.materialise(o)
+            case _:
+                for child in ir.children(e):
+                    self.prepare(child, product)
+                self.node.setdefault(id(e), None)
+
+    @staticmethod
+    def loads(e: ir.Expr, tensor: str | None = None) -> bool:
+        """Whether evaluating `e` loads from a tensor (from `tensor`)."""
+        if isinstance(e, ir.TileLoad):
+            return tensor is None or e.tensor.name == tensor
+        return any(Emitter.loads(child, tensor) for child in ir.children(e))
+
+    def materialise(self, e: ir.Expr) -> tuple[str, str]:
+        value, valid = self.buffer(e.dtype, e.shape)
+
+        def body(idx):
+            x, ok = self.value(e, idx)
+            self.store(value, valid, "_e", x, ok, f"e{math.prod(e.shape)}")
+
+        self.loop(e.shape, body)
+        return value, valid
+
+    def store(self, value: str, valid: str, at: str, x: str, ok: str, pattern: str) -> None:
+        self.put(f"{value}[{at}] = {x}; {valid}[{at}] = {ok};")
+        self.access(value, pattern, write=True)
+        self.access(valid, pattern, write=True)
+
+    def fetch(self, buffers: tuple[str, str], idx: list[str], shape: tuple[int, ...], own: bool) -> tuple[str, str]:
+        """An element of a tile in LDS; `own`: it is the loop's own element."""
+        at = "_e" if own else self.linear(idx, shape)
+        for name in buffers:
+            self.access(name, f"e{math.prod(shape)}" if own else "any")
+        return f"{buffers[0]}[{at}]", f"{buffers[1]}[{at}]"
+
+    def line(self, dtype: Dtype, text: str) -> str:
+        name = self.fresh("x")
+        self.put(f"const {ctype(dtype)} {name} = {text};")
+        return name
+
+    @staticmethod
+    def both(checks: list[str]) -> str:
+        kept = list(dict.fromkeys(c for c in checks if c != "1"))
+        return " & ".join(kept) or "1"
+
+    def value(self, e: ir.Expr, idx: list[str]) -> tuple[str, str]:
+        """The element of `e` at `idx` (its value and its validity), computed in the current loop."""
+        if not e.shape:
+            return self.scalar(e), "1"
+        idx = self.aligned(idx, e.shape)
+        key = (id(e), *idx)
+        if key not in self.memo:
+            self.memo[key] = self.compute(e, idx)
+        return self.memo[key]
+
+    def own(self, idx: list[str], shape: tuple[int, ...]) -> bool:
+        """Whether `idx` is the element of the surrounding `loop`, whose shape is `shape`."""
+        return self.loop_shape == shape and idx == self.aligned([f"_i{a}" for a in range(len(shape))], shape)
+
+    loop_shape: tuple[int, ...] | None = None
+
+    def compute(self, e: ir.Expr, idx: list[str]) -> tuple[str, str]:
+        match e:
+            case ir.Var(name=n):
+                return self.fetch(self.tile_vars[n], idx, e.shape, self.own(idx, e.shape))
+            case ir.Reduce():
+                return self.fetch(self.node[id(e)], idx, e.shape, False)
+            case ir.Zeros():
+                return f"(({ctype(e.dtype)})0)", "1"
+            case ir.Arange():
+                return self.line(e.dtype, f"({ctype(e.dtype)})({self.node[id(e)]} + {idx[e.axis]})"), "1"
+            case ir.Transpose(operand=o):
+                if self.node.get(id(e)):
+                    return self.fetch(self.node[id(e)], [idx[1], idx[0]], o.shape, False)
+                return self.value(o, [idx[1], idx[0]])
+            case ir.TileLoad():
+                return self.load(e, idx)
+        operands = [self.value(child, idx) for child in ir.children(e)]
+        texts, valid = [v for v, _ in operands], self.both([ok for _, ok in operands])
+        match e:
+            case ir.Cast(operand=o):
+                text = self.cast(texts[0], o.dtype, e.dtype)
+            case ir.Unary():
+                text = self.rounded(f"-{texts[0]}", e.dtype)
+            case ir.Binary():
+                text = self.binary(e, texts)
+            case ir.Math(fn=fn):
+                template = MATH[fn]
+                if e.dtype == F64:
+                    template = template.replace("f(", "(")
+                text = self.rounded(template.format(*texts), e.dtype)
+            case ir.Select():
+                text = f"({texts[0]} ? {texts[1]} : {texts[2]})"
+            case _:
+                raise LoweringError(f"tile {type(e).__name__} is not lowered")
+        if valid.count("&") > 2:
+            valid = self.line(BOOL, valid)
+        return self.line(e.dtype, text), valid
+
+    def cells(self, starts: list[str], slices, tensor: str, idx: list[str]) -> tuple[str, str]:
+        """The linear index of a tile element in its tensor, and whether it lies inside."""
+        axes = iter(idx)
+        cells = [st if sl.squeeze else f"({st} + {next(axes)})" for st, sl in zip(starts, slices)]
+        inside = " && ".join(f"{c} >= 0 && {c} < {tensor}_n{a}" for a, c in enumerate(cells))
+        linear = " + ".join(c + "".join(f" * {tensor}_n{b}" for b in range(a + 1, len(cells)))
+                            for a, c in enumerate(cells))
+        return linear, inside
+
+    def load(self, e: ir.TileLoad, idx: list[str]) -> tuple[str, str]:
+        tensor = e.tensor.name
+        # a tile axis of extent 1 that the loop broadcasts is element 0 of its slice
+        linear, inside = self.cells(self.node[id(e)], e.slices, tensor, idx)
+        ok = self.line(BOOL, inside)
+        element = f"{tensor}[{linear}]"
+        if e.dtype == BF16:
+            element = f"kb16_load({element})"
+        self.reads.append((("tensor", tensor), "any"))
+        return self.line(e.dtype, f"{ok} ? {element} : ({ctype(e.dtype)})0"), ok
+
+    def binary(self, e: ir.Binary, t: list[str]) -> str:
+        op = {ir.Op.AND: "&", ir.Op.OR: "|"}.get(e.op, e.op.value)
+        if e.op is ir.Op.MOD and e.lhs.dtype.is_float:
+            return f"fmodf({t[0]}, {t[1]})"
+        if e.op in ir.COMPARISONS:
+            return f"({t[0]} {op} {t[1]})"
+        if e.op is ir.Op.DIV and e.lhs.dtype.is_int:
+            return f"({t[1]} ? {t[0]} / {t[1]} : 0)"
+        return self.rounded(f"{t[0]} {op} {t[1]}", e.dtype)
+
+    def reduce(self, e: ir.Reduce) -> tuple[str, str]:
+        """A reduction over one axis, valid lanes only. float32 and integer ones share an output among up to 64
+        neighbouring threads, each from its first valid lane, joined by shuffles; the 16-bit types, which round after
+        every step, keep one thread and the order of the axis."""
+        value, valid = self.buffer(e.dtype, e.shape)
+        shape, axis = e.operand.shape, e.axis
+        outputs, extent = math.prod(shape) // shape[axis], shape[axis]
+        join = {
+            ir.Reduction.MAX: "_acc = (_y > _acc || _y != _y) ? _y : _acc;",
+            ir.Reduction.MIN: "_acc = (_y < _acc || _y != _y) ? _y : _acc;",
+            ir.Reduction.SUM: "_acc = _acc + _y;",
+        }[e.op]
+        if e.dtype == BF16:
+            join = join.replace("_acc + _y", "kb16(_acc + _y)")
+        group = 1
+        if e.dtype in (F32, I32) or (e.op is not ir.Reduction.SUM and e.dtype == BF16):
+            while group < 64 and 2 * group <= extent and outputs * group < THREADS:
+                group *= 2
+        kept = [s for a, s in enumerate(shape) if a != axis]
+        acc = ctype(e.dtype)
+
+        def emit() -> None:
+            self.put(f"for (int _t = threadIdx.x; _t < {outputs * group}; _t += {THREADS}) {{")
+            self.depth += 1
+            self.put(f"const int _o = _t / {group};")
+            idx, position = [], 0
+            for a in range(len(shape)):
+                if a == axis:
+                    idx.append("_r")
+                else:
+                    idx.append(f"(_o / {math.prod(kept[position + 1:])} % {kept[position]})")
+                    position += 1
+            self.put(f"{acc} _acc = 0; unsigned char _seen = 0;")
+            self.put(f"for (int _r = _t % {group}; _r < {extent}; _r += {group}) {{")
+            self.depth += 1
+            x, ok = self.value(e.operand, idx)
+            take = f"{acc} _y = {x}; if (_seen) {{ {join} }} else {{ _acc = _y; _seen = 1; }}"
+            self.put(f"{{ {take} }}" if ok == "1" else f"if ({ok}) {{ {take} }}")
+            self.depth -= 1
+            self.put("}")
+            if group > 1:
+                self.put(f"for (int _g = {group // 2}; _g; _g >>= 1) {{")
+                self.put(f"  const {acc} _y = __shfl_xor(_acc, _g); const int _other = __shfl_xor((int)_seen, _g);")
+                self.put(f"  if (_other) {{ if (_seen) {{ {join} }} else _acc = _y; _seen = 1; }}")
+                self.put("}")
+            self.put(f"if (_t % {group} == 0) {{ {value}[_o] = _acc; {valid}[_o] = _seen; }}")
+            self.depth -= 1
+            self.put("}")
+            for name in (value, valid):
+                self.access(name, "any", write=True)
+
+        self.region(emit)
+        return value, valid
+
+    # ---- statements
 
     def stmt_TileAssign(self, s: ir.TileAssign) -> None:
-        value, valid = self.tile(s.value)
-        target, target_v = self.tile_vars[s.var.name]
-        if (value, valid) == (target, target_v):
+        if s.value == s.var:
             return
-        # a value that reads the variable it assigns is computed into a temporary first (one barrier between)
-        self.loop(s.var.shape, lambda idx: self.put(
-            f"{target}[_e] = {value}[{self.index(idx, s.value.shape)}]; "
-            f"{target_v}[_e] = {valid}[{self.index(idx, s.value.shape)}];"))
+        self.prepare(s.value)
+        target = self.tile_vars[s.var.name]
+        if self.reads_elsewhere(s.value, s.var, s.var.shape):
+            temporary = self.materialise(s.value)  # other threads' elements of the variable: computed before it changes
+            shape = s.value.shape
+            self.loop(s.var.shape, lambda idx: self.store(
+                *target, "_e", *self.fetch(temporary, self.aligned(idx, shape), shape, False),
+                f"e{math.prod(s.var.shape)}"))
+            return
+
+        def body(idx):
+            x, ok = self.value(s.value, idx)
+            self.store(*target, "_e", x, ok, f"e{math.prod(s.var.shape)}")
+
+        self.elements(s.var.shape, body)
+
+    def elements(self, shape: tuple[int, ...], body) -> None:
+        """`loop` whose index is the thread's own element of every tile of this shape."""
+        self.loop_shape = shape
+        self.loop(shape, body)
+        self.loop_shape = None
+
+    @staticmethod
+    def reads_elsewhere(e: ir.Expr, var: ir.Var, shape: tuple[int, ...] | None) -> bool:
+        """Whether computing `e` at an element reads `var` at another one (through a transpose or a broadcast)."""
+        if isinstance(e, ir.Var):
+            return e.name == var.name and e.shape != shape
+        if isinstance(e, ir.Reduce):
+            return False  # computed before the loop
+        inner = None if isinstance(e, ir.Transpose) else shape
+        return any(Emitter.reads_elsewhere(child, var, inner) for child in ir.children(e))
 
     def stmt_TileStore(self, s: ir.TileStore) -> None:
-        value, valid = self.tile(s.value)
-        tensor = s.tensor.name
-        starts = [f"_s{a}" for a in range(len(s.slices))]
-        for a, sl in enumerate(s.slices):
-            self.put(f"{{ const long long _s{a} = {self.scalar(sl.start)};")
+        self.prepare(s.value)
+        tensor, starts = s.tensor.name, [self.fresh("s") for _ in s.slices]
+        for name, sl in zip(starts, s.slices):
+            self.put(f"const long long {name} = {self.scalar(sl.start)};")
+        # a value loaded from the tensor it is stored to is complete before any of it is stored
+        temporary = self.materialise(s.value) if self.loads(s.value, tensor) else None
 
         def store(idx):
-            axes = iter(idx)
-            cells = [st if sl.squeeze else f"({st} + {next(axes)})" for st, sl in zip(starts, s.slices)]
-            inside = " && ".join(f"{c} >= 0 && {c} < {tensor}_n{a}" for a, c in enumerate(cells))
-            linear = " + ".join(c + "".join(f" * {tensor}_n{b}" for b in range(a + 1, len(cells)))
-                                for a, c in enumerate(cells))
-            element = f"{value}[_e]"
-            if s.tensor.type.dtype == BF16:
-                element = f"kb16_word({element})"
-            self.put(f"if ({valid}[_e] && {inside}) {tensor}[{linear}] = {element};")
+            linear, inside = self.cells(starts, s.slices, tensor, idx)
+            if temporary is not None:
+                x, ok = self.fetch(temporary, idx, s.value.shape, False)
+            else:
+                x, ok = self.value(s.value, idx)
+            element = f"kb16_word({x})" if s.tensor.type.dtype == BF16 else x
+            self.put(f"if ({'' if ok == '1' else f'({ok}) && '}{inside}) {tensor}[{linear}] = {element};")
+            self.writes.append((("tensor", tensor), "any"))
 
-        self.loop(s.value.shape, store)
-        self.put("}" * len(s.slices))
+        self.elements(s.value.shape, store)
 
     def stmt_Accumulate(self, s: ir.Accumulate) -> None:
-        acc, acc_v = self.tile_vars[s.acc.name]
-        (m, k), n = s.lhs.shape, s.rhs.shape[1]
-        integer = s.acc.dtype == I32
-        stage = "int" if integer else "float"
-        a, av = self.tile(s.lhs)
-        b, bv = self.tile(s.rhs)
+        self.prepare(s.lhs, product=True)
+        self.prepare(s.rhs, product=True)
         form = mfma_form(s)
         if form is not None:
-            self.mfma_product(s, form, (a, av), (b, bv), (acc, acc_v))
-            return
-        af, bf = self.staged(stage, a, av, s.lhs), self.staged(stage, b, bv, s.rhs)
-        self.put(f"for (int _e = threadIdx.x; _e < {m * n}; _e += {THREADS}) {{")
-        self.put(f"  const int _i = _e / {n}, _j = _e % {n};")
-        if integer:
-            self.put(f"  unsigned _s = (unsigned){acc}[_e];")
-            self.put(f"  for (int _k = 0; _k < {k}; ++_k) _s += (unsigned)({af}[_i * {k} + _k] * {bf}[_k * {n} + _j]);")
-            self.put(f"  {acc}[_e] = (int)_s;")
+            self.mfma_product(s, form)
         else:
-            self.put(f"  float _s = {acc}[_e];")
-            self.put(f"  for (int _k = 0; _k < {k}; ++_k) _s = fmaf({af}[_i * {k} + _k], {bf}[_k * {n} + _j], _s);")
-            self.put(f"  {acc}[_e] = _s;")
-        self.put(f"  unsigned char _row = 0, _col = 0;")
-        self.put(f"  for (int _k = 0; _k < {k}; ++_k) {{ _row |= {av}[_i * {k} + _k]; _col |= {bv}[_k * {n} + _j]; }}")
-        self.put(f"  {acc_v}[_e] = {acc_v}[_e] & _row & _col;")
-        self.put("}")
-        self.put("__syncthreads();")
+            self.scalar_product(s)
+        self.product_validity(s)
 
-    def mfma_product(self, s: ir.Accumulate, form: "MfmaForm", lhs, rhs, accumulator) -> None:
+    def product_validity(self, s: ir.Accumulate) -> None:
+        """An accumulator element stays valid when its row of lhs and its column of rhs have a valid lane each."""
+        (m, k), n = s.lhs.shape, s.rhs.shape[1]
+        flags = [self.any_valid(s.lhs, m, k, False), self.any_valid(s.rhs, n, k, True)]
+        valid = self.tile_vars[s.acc.name][1]
+
+        def body(idx):
+            checks = [flag[0] if isinstance(flag, tuple) else f"{flag}[{i}]" for flag, i in zip(flags, idx)]
+            for flag in flags:
+                if isinstance(flag, str):
+                    self.access(flag, "any")
+            checks = [self.line(BOOL, flag[1](i)) if isinstance(flag, tuple) else c
+                      for flag, i, c in zip(flags, idx, checks)]
+            self.access(valid, f"e{m * n}")
+            self.access(valid, f"e{m * n}", write=True)
+            self.put(f"{valid}[_e] = {valid}[_e] & {self.both(checks)};")
+
+        self.elements((m, n), body)
+
+    def any_valid(self, e: ir.Expr, rows: int, k: int, transposed: bool):
+        """Whether row i of an operand (column i of a (k, n) one) has a valid lane: the name of a flag per row, or, for
+        a load, whose lanes are valid in a block, ("load", the condition as a function of i)."""
+        turned = isinstance(e, ir.Transpose)
+        load = e.operand if turned else e
+        if isinstance(load, ir.TileLoad):
+            starts, tensor = self.node[id(load)], load.tensor.name
+            kept = [a for a, sl in enumerate(load.slices) if not sl.squeeze]
+            row_axis, k_axis = (kept[1], kept[0]) if transposed != turned else (kept[0], kept[1])
+
+            def condition(i: str) -> str:
+                checks = [f"{st} >= 0 && {st} < {tensor}_n{a}" for a, (st, sl) in enumerate(zip(starts, load.slices))
+                          if sl.squeeze]
+                checks.append(f"{starts[k_axis]} < {tensor}_n{k_axis} && {starts[k_axis]} + {k} > 0")
+                checks.append(f"{starts[row_axis]} + {i} >= 0 && {starts[row_axis]} + {i} < {tensor}_n{row_axis}")
+                return " && ".join(checks)
+
+            return ("load", condition)
+        flag = self.reserve(self.fresh("any"), "unsigned char", rows)
+
+        def emit() -> None:
+            self.put(f"for (int _t = threadIdx.x; _t < {rows}; _t += {THREADS}) {{")
+            self.depth += 1
+            self.put("unsigned char _any = 0;")
+            self.put(f"for (int _k = 0; _k < {k}; ++_k) {{")
+            self.depth += 1
+            self.put(f"_any |= {self.value(e, ['_k', '_t'] if transposed else ['_t', '_k'])[1]};")
+            self.depth -= 1
+            self.put("}")
+            self.put(f"{flag}[_t] = _any;")
+            self.access(flag, "any", write=True)
+            self.depth -= 1
+            self.put("}")
+
+        self.region(emit)
+        return flag
+
+    def scalar_product(self, s: ir.Accumulate) -> None:
+        """One fused multiply-add per k in k order for each output. Both operands are staged k-major, and a thread keeps
+        a block of outputs in registers over the whole k: of 4 x 4 two 16-byte LDS reads per 16 multiply-adds (one
+        output at a time, two reads each, 256^3 took 38 us)."""
+        (m, k), n = s.lhs.shape, s.rhs.shape[1]
+        acc = self.tile_vars[s.acc.name][0]
+        integer = s.acc.dtype == I32
+        stage = "int" if integer else "float"
+        a, b = self.staged(stage, s.lhs, m, k, False), self.staged(stage, s.rhs, n, k, True)
+        rm, rn = next((r for r in ((4, 4), (2, 4), (1, 4), (2, 2), (1, 2), (1, 1))
+                       if m % r[0] == 0 and n % r[1] == 0 and (m // r[0]) * (n // r[1]) >= min(THREADS, m * n)), (1, 1))
+
+        def emit() -> None:
+            self.put(f"for (int _t = threadIdx.x; _t < {(m // rm) * (n // rn)}; _t += {THREADS}) {{")
+            self.depth += 1
+            self.put(f"const int _i = _t / {n // rn} * {rm}, _j = _t % {n // rn} * {rn};")
+            kind = "unsigned" if integer else "float"
+            self.put(f"{kind} _s[{rm}][{rn}];")
+            each = f"for (int _y = 0; _y < {rm}; ++_y) for (int _x = 0; _x < {rn}; ++_x)"
+            self.put(f"_Pragma(\"unroll\") {each} _s[_y][_x] = ({kind}){acc}[(_i + _y) * {n} + _j + _x];")
+            self.put(f"_Pragma(\"unroll 4\") for (int _k = 0; _k < {k}; ++_k) {{")
+            self.put(f"  {stage} _p[{rm}], _q[{rn}];")
+            self.put(f"  for (int _y = 0; _y < {rm}; ++_y) _p[_y] = {a}[_k * {m + 4} + _i + _y];")
+            self.put(f"  for (int _x = 0; _x < {rn}; ++_x) _q[_x] = {b}[_k * {n + 4} + _j + _x];")
+            step = ("_s[_y][_x] += (unsigned)(_p[_y] * _q[_x]);" if integer
+                    else "_s[_y][_x] = fmaf(_p[_y], _q[_x], _s[_y][_x]);")
+            self.put(f"  _Pragma(\"unroll\") {each} {step}")
+            self.put("}")
+            self.put(f"_Pragma(\"unroll\") {each} {acc}[(_i + _y) * {n} + _j + _x] = ({stage})_s[_y][_x];")
+            self.depth -= 1
+            self.put("}")
+            for name in (a, b, acc):
+                self.access(name, "any")
+            self.access(acc, "any", write=True)
+
+        self.region(emit)
+
+    def staged(self, stage: str, e: ir.Expr, rows: int, k: int, transposed: bool) -> str:
+        """An operand of a scalar product in LDS as `k` rows of `rows` elements (and four more, so that a column of
+        them is not in one bank), invalid lanes zero; `transposed` reads
+        a (k, rows) tile. The loop runs along the operand's own rows, so that loads from a tensor are contiguous."""
+        name = self.reserve(self.fresh("st"), stage, (rows + 4) * k)
+        along_rows = transposed != isinstance(e, ir.Transpose)
+
+        def body(idx):
+            kk, rr = (idx[0], idx[1]) if along_rows else (idx[1], idx[0])
+            x, ok = self.value(e, [kk, rr] if transposed else [rr, kk])
+            element = f"k8dec({x})" if e.dtype.is_narrow else f"({stage}){x}"
+            self.put(f"{name}[{kk} * {rows + 4} + {rr}] = {element if ok == '1' else f'({ok}) ? {element} : ({stage})0'};")
+            self.access(name, "any", write=True)
+
+        self.loop((k, rows) if along_rows else (rows, k), body)
+        return name
+
+    def mfma_product(self, s: ir.Accumulate, form: "MfmaForm") -> None:
         """acc[m, n] += lhs[m, k] @ rhs[k, n] on the matrix cores: both operands staged into LDS K-contiguous as the
         instruction's operand type (invalid lanes 0, so they add nothing), then each of the 4 waves takes 16 x 16
         output blocks in turn, loads the block's accumulators, runs k / K_STEP MFMAs and writes them back. Lane l of
         a 16x16xK MFMA holds operand row (or column) l % 16 and K_STEP / 4 consecutive k from (l / 16) * K_STEP / 4,
         and accumulators rows 4 (l / 16) + i, column l % 16 (reference compiler/hip.py:70-97 `AMDMFMA.product`,
-        compiler/emit.py:924-955 `matrix_stage`). The validity of the accumulator is the scalar path's."""
-        (a, av), (b, bv), (acc, acc_v) = lhs, rhs, accumulator
+        compiler/emit.py:924-955 `matrix_stage`). Staged rows are 16 bytes longer than K: 16 rows of a multiple of 128
+        bytes would meet in one bank."""
+        acc = self.tile_vars[s.acc.name][0]
         (m, k), n = s.lhs.shape, s.rhs.shape[1]
         per = form.k_step // 4  # operand elements per lane per instruction
-        at = self.mfma_stage(form, a, av, s.lhs, m, k, transposed=False)
-        bt = self.mfma_stage(form, b, bv, s.rhs, n, k, transposed=True)
+        pitch = k + 16 // SIZES[form.element]
+        at = self.mfma_stage(form, s.lhs, m, k, pitch, transposed=False)
+        bt = self.mfma_stage(form, s.rhs, n, k, pitch, transposed=True)
         acc_t = "int" if form.integer else "float"
-        self.put("{")
-        self.put("  const int _w = threadIdx.x >> 6, _l = threadIdx.x & 63, _r = _l & 15, _q = _l >> 4;")
-        self.put(f"  for (int _blk = _w; _blk < {(m // 16) * (n // 16)}; _blk += {THREADS // 64}) {{")
-        self.put(f"    const int _m0 = (_blk / {n // 16}) * 16, _n0 = (_blk % {n // 16}) * 16;")
-        self.put(f"    {form.acc_vec} _c;")
-        self.put(f"    for (int _i = 0; _i < 4; ++_i) _c[_i] = {acc}[(_m0 + 4 * _q + _i) * {n} + _n0 + _r];")
-        self.put(f"    for (int _k = 0; _k < {k}; _k += {form.k_step}) {{")
-        self.put(f"      const {form.operand_vec} _a = *(const {form.operand_vec}*)&{at}[(_m0 + _r) * {k} + _k + _q * {per}];")
-        self.put(f"      const {form.operand_vec} _b = *(const {form.operand_vec}*)&{bt}[(_n0 + _r) * {k} + _k + _q * {per}];")
-        self.put(f"      _c = {form.builtin}(_a, _b, _c, 0, 0, 0);")
-        self.put("    }")
-        self.put(f"    for (int _i = 0; _i < 4; ++_i) {acc}[(_m0 + 4 * _q + _i) * {n} + _n0 + _r] = ({acc_t})_c[_i];")
-        self.put("  }")
-        self.put("}")
-        self.put(f"for (int _e = threadIdx.x; _e < {m * n}; _e += {THREADS}) {{")
-        self.put(f"  const int _i = _e / {n}, _j = _e % {n};")
-        self.put(f"  unsigned char _row = 0, _col = 0;")
-        self.put(f"  for (int _k = 0; _k < {k}; ++_k) {{ _row |= {av}[_i * {k} + _k]; _col |= {bv}[_k * {n} + _j]; }}")
-        self.put(f"  {acc_v}[_e] = {acc_v}[_e] & _row & _col;")
-        self.put("}")
-        self.put("__syncthreads();")
+
+        def emit() -> None:
+            self.put("{")
+            self.put("  const int _w = threadIdx.x >> 6, _l = threadIdx.x & 63, _r = _l & 15, _q = _l >> 4;")
+            self.put(f"  for (int _blk = _w; _blk < {(m // 16) * (n // 16)}; _blk += {THREADS // 64}) {{")
+            self.put(f"    const int _m0 = (_blk / {n // 16}) * 16, _n0 = (_blk % {n // 16}) * 16;")
+            self.put(f"    {form.acc_vec} _c;")
+            self.put(f"    for (int _i = 0; _i < 4; ++_i) _c[_i] = {acc}[(_m0 + 4 * _q + _i) * {n} + _n0 + _r];")
+            self.put(f"    for (int _k = 0; _k < {k}; _k += {form.k_step}) {{")
+            vec = form.operand_vec
+            self.put(f"      const {vec} _a = *(const {vec}*)&{at}[(_m0 + _r) * {pitch} + _k + _q * {per}];")
+            self.put(f"      const {vec} _b = *(const {vec}*)&{bt}[(_n0 + _r) * {pitch} + _k + _q * {per}];")
+            self.put(f"      _c = {form.builtin}(_a, _b, _c, 0, 0, 0);")
+            self.put("    }")
+            self.put(f"    for (int _i = 0; _i < 4; ++_i) {acc}[(_m0 + 4 * _q + _i) * {n} + _n0 + _r] = ({acc_t})_c[_i];")
+            self.put("  }")
+            self.put("}")
+            for name in (at, bt, acc):
+                self.access(name, "any")
+            self.access(acc, "any", write=True)
+
+        self.region(emit)
         self.mfma_products += 1
 
-    def mfma_stage(self, form: "MfmaForm", value: str, valid: str, e: ir.Expr, rows: int, k: int,
-                   transposed: bool) -> str:
+    def mfma_stage(self, form: "MfmaForm", e: ir.Expr, rows: int, k: int, pitch: int, transposed: bool) -> str:
         """An operand in LDS as `rows` K-contiguous rows of the instruction's element bits; `transposed` reads a
-        (k, rows) tile."""
-        self.count += 1
-        name = f"mf{self.count}"
-        self.buffers.append((name, form.element, rows * k))
-        source = f"{value}[_kk * {rows} + _rr]" if transposed else f"{value}[_rr * {k} + _kk]"
-        check = f"{valid}[_kk * {rows} + _rr]" if transposed else f"{valid}[_rr * {k} + _kk]"
-        bits = {"f16": f"__builtin_bit_cast(unsigned short, (_Float16){source})",
-                "bf16": f"(unsigned short)(__float_as_uint({source}) >> 16)",
-                "fp8": f"(unsigned char){source}",  # the e4m3 code as the tile holds it
-                "i8": f"(signed char){source}"}[form.name]
-        self.put(f"for (int _e = threadIdx.x; _e < {rows * k}; _e += {THREADS}) {{")
-        self.put(f"  const int _rr = _e / {k}, _kk = _e % {k};")
-        self.put(f"  {name}[_e] = {check} ? {bits} : ({form.element})0;")
-        self.put("}")
-        self.put("__syncthreads();")
-        return name
+        (k, rows) tile. The loop runs along the operand's own rows, so that loads from a tensor are contiguous."""
+        name = self.reserve(self.fresh("mf"), form.element, rows * pitch)
+        along_rows = transposed != isinstance(e, ir.Transpose)
 
-    def staged(self, stage: str, value: str, valid: str, e: ir.Expr) -> str:
-        self.count += 1
-        name = f"st{self.count}"
-        self.buffers.append((name, stage, math.prod(e.shape)))
-        element = f"k8dec({value}[_e])" if e.dtype.is_narrow else f"({stage}){value}[_e]"
-        self.put(f"for (int _e = threadIdx.x; _e < {math.prod(e.shape)}; _e += {THREADS}) "
-                 f"{name}[_e] = {valid}[_e] ? {element} : ({stage})0;")
-        self.put("__syncthreads();")
+        def body(idx):
+            kk, rr = (idx[0], idx[1]) if along_rows else (idx[1], idx[0])
+            x, ok = self.value(e, [kk, rr] if transposed else [rr, kk])
+            bits = {"f16": f"__builtin_bit_cast(unsigned short, (_Float16){x})",
+                    "bf16": f"(unsigned short)(__float_as_uint({x}) >> 16)",
+                    "fp8": f"(unsigned char){x}",  # the e4m3 code as the tile holds it
+                    "i8": f"(signed char){x}"}[form.name]
+            self.put(f"{name}[{rr} * {pitch} + {kk}] = {bits if ok == '1' else f'({ok}) ? {bits} : ({form.element})0'};")
+            self.access(name, "any", write=True)
+
+        self.loop((k, rows) if along_rows else (rows, k), body)
         return name
 
     def stmt_For(self, s: ir.For) -> None:
         var = s.var.name
+        if self.pending:
+            self.barrier()  # the body's first accesses are checked against its own last ones only
         self.put(f"for (long long {var} = {self.scalar(s.lo)}; {var} < {self.scalar(s.hi)}; {var} += {s.step}) {{")
         self.depth += 1
         self.body(s.body)
+        if self.pending:
+            self.barrier()
         self.depth -= 1
         self.put("}")
 
     def stmt_If(self, s: ir.If) -> None:
+        if self.pending:
+            self.barrier()
         self.put(f"if ({self.scalar(s.cond)}) {{")
         self.depth += 1
         self.body(s.then)
+        if self.pending:
+            self.barrier()
         self.depth -= 1
         self.put("} else {")
         self.depth += 1
         self.body(s.orelse)
+        if self.pending:
+            self.barrier()
         self.depth -= 1
         self.put("}")
 
@@ -417,121 +820,8 @@ class Emitter:
             return f"(({text}) != 0)"
         return f"(({ctype(dst)})({text}))"
 
-    def tile(self, e: ir.Expr) -> tuple[str, str]:
-        if isinstance(e, ir.Var):
-            return self.tile_vars[e.name]
-        if not e.shape:
-            value, valid = self.buffer(e.dtype, ())
-            self.put(f"if (threadIdx.x == 0) {{ {value}[0] = {self.scalar(e)}; {valid}[0] = 1; }}")
-            self.put("__syncthreads();")
-            return value, valid
-        return getattr(self, f"tile_{type(e).__name__}")(e)
-
-    def tile_Zeros(self, e: ir.Zeros):
-        value, valid = self.buffer(e.dtype, e.shape)
-        self.loop(e.shape, lambda idx: self.put(f"{value}[_e] = 0; {valid}[_e] = 1;"))
-        return value, valid
-
-    def tile_TileLoad(self, e: ir.TileLoad):
-        value, valid = self.buffer(e.dtype, e.shape)
-        tensor = e.tensor.name
-        starts = [f"_s{a}" for a in range(len(e.slices))]
-        for a, sl in enumerate(e.slices):
-            self.put(f"{{ const long long _s{a} = {self.scalar(sl.start)};")
-
-        def load(idx):
-            axes = iter(idx)
-            cells = [st if sl.squeeze else f"({st} + {next(axes)})" for st, sl in zip(starts, e.slices)]
-            inside = " && ".join(f"{c} >= 0 && {c} < {tensor}_n{a}" for a, c in enumerate(cells))
-            linear = " + ".join(c + "".join(f" * {tensor}_n{b}" for b in range(a + 1, len(cells)))
-                                for a, c in enumerate(cells))
-            element = f"{tensor}[{linear}]"
-            if e.dtype == BF16:
-                element = f"kb16_load({element})"
-            self.put(f"if ({inside}) {{ {value}[_e] = {element}; {valid}[_e] = 1; }} "
-                     f"else {{ {value}[_e] = 0; {valid}[_e] = 0; }}")
-
-        self.loop(e.shape, load)
-        self.put("}" * len(e.slices))
-        return value, valid
-
-    def tile_Transpose(self, e: ir.Transpose):
-        a, av = self.tile(e.operand)
-        value, valid = self.buffer(e.dtype, e.shape)
-        cols = e.operand.shape[1]
-        self.loop(e.shape, lambda idx: self.put(
-            f"{value}[_e] = {a}[{idx[1]} * {cols} + {idx[0]}]; {valid}[_e] = {av}[{idx[1]} * {cols} + {idx[0]}];"))
-        return value, valid
-
-    def tile_Arange(self, e: ir.Arange):
-        value, valid = self.buffer(e.dtype, e.shape)
-        start = self.scalar(e.start)
-        self.loop(e.shape, lambda idx: self.put(f"{value}[_e] = (int)({start} + {idx[e.axis]}); {valid}[_e] = 1;"))
-        return value, valid
-
-    def elementwise(self, e: ir.Expr, operands: list[ir.Expr], make) -> tuple[str, str]:
-        parts = [self.tile(o) for o in operands]
-        value, valid = self.buffer(e.dtype, e.shape)
-
-        def body(idx):
-            texts = [f"{v}[{self.index(idx, o.shape)}]" for (v, _), o in zip(parts, operands)]
-            checks = [f"{vv}[{self.index(idx, o.shape)}]" for (_, vv), o in zip(parts, operands)]
-            self.put(f"{value}[_e] = {make(texts)}; {valid}[_e] = {' & '.join(checks)};")
-
-        self.loop(e.shape, body)
-        return value, valid
-
     def rounded(self, text: str, dtype: Dtype) -> str:
         return f"kb16({text})" if dtype == BF16 else f"({ctype(dtype)})({text})"
-
-    def tile_Cast(self, e: ir.Cast):
-        return self.elementwise(e, [e.operand], lambda t: self.cast(t[0], e.operand.dtype, e.dtype))
-
-    def tile_Unary(self, e: ir.Unary):
-        return self.elementwise(e, [e.operand], lambda t: self.rounded(f"-{t[0]}", e.dtype))
-
-    def tile_Binary(self, e: ir.Binary):
-        op = {ir.Op.AND: "&", ir.Op.OR: "|"}.get(e.op, e.op.value)
-        if e.op is ir.Op.MOD and e.lhs.dtype.is_float:
-            return self.elementwise(e, [e.lhs, e.rhs], lambda t: f"fmodf({t[0]}, {t[1]})")
-        if e.op in ir.COMPARISONS:
-            return self.elementwise(e, [e.lhs, e.rhs], lambda t: f"({t[0]} {op} {t[1]})")
-        if e.op is ir.Op.DIV and e.lhs.dtype.is_int:
-            return self.elementwise(e, [e.lhs, e.rhs], lambda t: f"({t[1]} ? {t[0]} / {t[1]} : 0)")
-        return self.elementwise(e, [e.lhs, e.rhs], lambda t: self.rounded(f"{t[0]} {op} {t[1]}", e.dtype))
-
-    def tile_Math(self, e: ir.Math):
-        template = MATH[e.fn]
-        if e.dtype == F64:
-            template = template.replace("f(", "(")
-        return self.elementwise(e, list(e.args), lambda t: self.rounded(template.format(*t), e.dtype))
-
-    def tile_Select(self, e: ir.Select):
-        return self.elementwise(e, [e.cond, e.then, e.orelse], lambda t: f"({t[0]} ? {t[1]} : {t[2]})")
-
-    def tile_Reduce(self, e: ir.Reduce):
-        a, av = self.tile(e.operand)
-        value, valid = self.buffer(e.dtype, e.shape)
-        shape, axis = e.operand.shape, e.axis
-        reducer = {
-            ir.Reduction.MAX: "_acc = (_x > _acc || _x != _x) ? _x : _acc;",
-            ir.Reduction.MIN: "_acc = (_x < _acc || _x != _x) ? _x : _acc;",
-            ir.Reduction.SUM: "_acc = _acc + _x;",
-        }[e.op]
-        if e.dtype == BF16:
-            reducer = reducer.replace("_acc + _x", "kb16(_acc + _x)")
-
-        def run(idx):
-            full = list(idx) if e.keepdims else [*idx[:axis], "0", *idx[axis:]]
-            full[axis] = "_r"
-            at = self.index(full, shape)
-            self.put(f"{ctype(e.dtype)} _acc = 0; unsigned char _seen = 0;")
-            self.put(f"for (int _r = 0; _r < {shape[axis]}; ++_r) {{ if (!{av}[{at}]) continue; "
-                     f"{ctype(e.dtype)} _x = {a}[{at}]; if (_seen) {{ {reducer} }} else {{ _acc = _x; _seen = 1; }} }}")
-            self.put(f"{value}[_e] = _acc; {valid}[_e] = _seen;")
-
-        self.loop(e.shape, run)
-        return value, valid
 
 
 def emit(kernel: ir.Kernel, entry: str) -> tuple[str, int]:

@@ -292,6 +292,7 @@ class Launch:
 
     def __init__(self, kernel: ir.Kernel, plan) -> None:
         self.kernel, self.plan = kernel, plan
+        self._program: Program | None = None  # the generic lowering's, once a launch has needed it
 
     def prepare(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The launch of these argument values on this grid as one call per stream: the plan's checks and argument
@@ -411,7 +412,9 @@ class Launch:
 
     def _generic(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The hiprtc program of this kernel, compiled (or found) once, with its kernelParams table built once."""
-        program = generic_program(self.kernel)
+        program = self._program
+        if program is None:  # writing the source to look the program up takes 0.8 ms
+            program = self._program = generic_program(self.kernel)
         params: list = []
         for (name, kind), value in zip(self.kernel.params, values):
             if isinstance(kind, ir.TensorType):

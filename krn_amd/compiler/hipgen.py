@@ -17,7 +17,6 @@ from dataclasses import dataclass
 from krn_amd.compiler import ir
 from krn_amd.dtypes import BF16, BOOL, F8E4M3, F16, F32, F64, I8, I32, I64, PY_FLOAT, PY_INT, Dtype, Kind
 
-THREADS = 256
 LDS_LIMIT = 160 * 1024
 
 
@@ -141,6 +140,16 @@ def mfma_form(s: ir.Accumulate) -> MfmaForm | None:
     return None
 
 
+def threads(kernel: ir.Kernel) -> int:
+    """Threads of one block: 256, and 1024 for programs whose tiles have 4096 elements and more and whose products, if
+    any, run on the matrix cores. Their LDS leaves room for one or two blocks on a CU, and 256 threads would be one
+    wave per SIMD with nothing to cover its LDS latency (flash attention, 64 x 64 tiles, d = 32: 16 x 512: 100 us with 256 threads, 51 with 1024). A scalar
+    product keeps 256: fewer outputs per thread are more LDS reads per multiply-add."""
+    large = max((math.prod(v.shape) for v in kernel.tiles), default=1) >= 4096
+    scalar = any(isinstance(s, ir.Accumulate) and mfma_form(s) is None for s in ir.walk(kernel.body))
+    return 1024 if large and not scalar else 256
+
+
 def products(kernel: ir.Kernel) -> list[str]:
     """How the generic lowering runs each product of `kernel`: "mfma 16x16x<K> <type>" or "scalar fma"."""
     found: list[str] = []
@@ -172,6 +181,7 @@ class Emitter:
 
     def __init__(self, kernel: ir.Kernel, entry: str) -> None:
         self.kernel, self.entry = kernel, entry
+        self.threads = threads(kernel)
         self.mfma_products = 0
         self.lines: list[str] = []
         self.depth = 1
@@ -185,6 +195,7 @@ class Emitter:
         self.reads: list[Access] = []
         self.writes: list[Access] = []
         self.pending: list[tuple[Access, bool]] = []  # since the last barrier: access, whether it wrote
+        self.open: tuple[tuple[int, ...], int, int] | None = None  # the last `elements` loop: shape, first and last line
 
     def put(self, text: str) -> None:
         self.lines.append("  " * self.depth + text)
@@ -248,7 +259,7 @@ class Emitter:
     def loop(self, shape: tuple[int, ...], body) -> None:
         """`body(index names)` for every element of `shape`, strided over the workgroup."""
         def emit() -> None:
-            self.put(f"for (int _e = threadIdx.x; _e < {math.prod(shape)}; _e += {THREADS}) {{")
+            self.put(f"for (int _e = threadIdx.x; _e < {math.prod(shape)}; _e += {self.threads}) {{")
             self.depth += 1
             names = []
             for a in range(len(shape)):
@@ -288,7 +299,7 @@ class Emitter:
         scratch = total > LDS_LIMIT  # tiles beyond one CU's LDS live in a per-block slice of global scratch
         if scratch:
             params.append("char* __restrict__ _scratch")
-        head = [PRELUDE, f'extern "C" __global__ __launch_bounds__({THREADS}) void {self.entry}({", ".join(params)}) {{']
+        head = [PRELUDE, f'extern "C" __global__ __launch_bounds__({self.threads}) void {self.entry}({", ".join(params)}) {{']
         if scratch:
             head.append(f"  char* _block = _scratch + ((long long)blockIdx.x + (long long)blockIdx.y * gridDim.x + "
                         f"(long long)blockIdx.z * gridDim.x * gridDim.y) * {total}LL;")
@@ -307,10 +318,29 @@ class Emitter:
         return "\n".join([*head, *self.lines, "}", ""]), self.scratch_bytes
 
     def body(self, statements) -> None:
-        for s in statements:
+        self.open = None
+        for s, following in zip(statements, [*statements[1:], None]):
+            # `acc = zeros` right before `acc += a @ b`: the product starts from zero itself
+            self.fresh_acc = isinstance(s, ir.Accumulate) and self.skipped is s.acc
+            self.skipped = None
+            if (isinstance(s, ir.TileAssign) and isinstance(s.value, ir.Zeros) and isinstance(following, ir.Accumulate)
+                    and following.acc == s.var and not self.reads_var(following, s.var)):
+                self.skipped = following.acc
+                continue
             mark, self.node = self.top, {}
             getattr(self, f"stmt_{type(s).__name__}")(s)
             self.top = mark  # the statement's temporaries are dead
+        self.open = None
+
+    fresh_acc = False
+    skipped: ir.Var | None = None
+
+    @staticmethod
+    def reads_var(s: ir.Accumulate, var: ir.Var) -> bool:
+        def within(e: ir.Expr) -> bool:
+            return (isinstance(e, ir.Var) and e.name == var.name) or any(within(child) for child in ir.children(e))
+
+        return within(s.lhs) or within(s.rhs)
 
     # ---- expressions: `prepare` before the loop, `value` inside it
 
@@ -479,13 +509,13 @@ class Emitter:
             join = join.replace("_acc + _y", "kb16(_acc + _y)")
         group = 1
         if e.dtype in (F32, I32) or (e.op is not ir.Reduction.SUM and e.dtype == BF16):
-            while group < 64 and 2 * group <= extent and outputs * group < THREADS:
+            while group < 64 and 2 * group <= extent and outputs * group < self.threads:
                 group *= 2
         kept = [s for a, s in enumerate(shape) if a != axis]
         acc = ctype(e.dtype)
 
         def emit() -> None:
-            self.put(f"for (int _t = threadIdx.x; _t < {outputs * group}; _t += {THREADS}) {{")
+            self.put(f"for (int _t = threadIdx.x; _t < {outputs * group}; _t += {self.threads}) {{")
             self.depth += 1
             self.put(f"const int _o = _t / {group};")
             idx, position = [], 0
@@ -539,10 +569,23 @@ class Emitter:
         self.elements(s.var.shape, body)
 
     def elements(self, shape: tuple[int, ...], body) -> None:
-        """`loop` whose index is the thread's own element of every tile of this shape."""
+        """`loop` whose index is the thread's own element of every tile of this shape. It joins the loop just before it
+        when that one runs over the same elements and nothing but the starts of slices stands between them."""
+        before = len(self.lines)
         self.loop_shape = shape
         self.loop(shape, body)
         self.loop_shape = None
+        added = self.lines[before:]
+        if self.open is not None and self.open[0] == shape and "__syncthreads();" not in added[0]:
+            _, first, last = self.open
+            between = self.lines[last + 1:before]
+            if all(line.lstrip().startswith("const long long _s") for line in between):
+                inner = added[1 + len(shape):-1]  # without the loop's head, index names and end
+                self.lines[first:] = [*between, *self.lines[first:last], *inner, self.lines[last]]
+                self.open = (shape, first + len(between), len(self.lines) - 1)
+                return
+        start = before + (1 if "__syncthreads();" in added[0] else 0)
+        self.open = (shape, start, len(self.lines) - 1)
 
     @staticmethod
     def reads_elsewhere(e: ir.Expr, var: ir.Var, shape: tuple[int, ...] | None) -> bool:
@@ -588,7 +631,7 @@ class Emitter:
         """An accumulator element stays valid when its row of lhs and its column of rhs have a valid lane each."""
         (m, k), n = s.lhs.shape, s.rhs.shape[1]
         flags = [self.any_valid(s.lhs, m, k, False), self.any_valid(s.rhs, n, k, True)]
-        valid = self.tile_vars[s.acc.name][1]
+        valid, zero = self.tile_vars[s.acc.name][1], self.fresh_acc
 
         def body(idx):
             checks = [flag[0] if isinstance(flag, tuple) else f"{flag}[{i}]" for flag, i in zip(flags, idx)]
@@ -597,9 +640,11 @@ class Emitter:
                     self.access(flag, "any")
             checks = [self.line(BOOL, flag[1](i)) if isinstance(flag, tuple) else c
                       for flag, i, c in zip(flags, idx, checks)]
-            self.access(valid, f"e{m * n}")
+            if not zero:
+                self.access(valid, f"e{m * n}")
+                checks = [f"{valid}[_e]", *checks]
             self.access(valid, f"e{m * n}", write=True)
-            self.put(f"{valid}[_e] = {valid}[_e] & {self.both(checks)};")
+            self.put(f"{valid}[_e] = {self.both(checks)};")
 
         self.elements((m, n), body)
 
@@ -624,7 +669,7 @@ class Emitter:
         flag = self.reserve(self.fresh("any"), "unsigned char", rows)
 
         def emit() -> None:
-            self.put(f"for (int _t = threadIdx.x; _t < {rows}; _t += {THREADS}) {{")
+            self.put(f"for (int _t = threadIdx.x; _t < {rows}; _t += {self.threads}) {{")
             self.depth += 1
             self.put("unsigned char _any = 0;")
             self.put(f"for (int _k = 0; _k < {k}; ++_k) {{")
@@ -648,18 +693,20 @@ class Emitter:
         acc = self.tile_vars[s.acc.name][0]
         integer = s.acc.dtype == I32
         stage = "int" if integer else "float"
+        zero = self.fresh_acc
         a, b = self.staged(stage, s.lhs, m, k, False), self.staged(stage, s.rhs, n, k, True)
         rm, rn = next((r for r in ((4, 4), (2, 4), (1, 4), (2, 2), (1, 2), (1, 1))
-                       if m % r[0] == 0 and n % r[1] == 0 and (m // r[0]) * (n // r[1]) >= min(THREADS, m * n)), (1, 1))
+                       if m % r[0] == 0 and n % r[1] == 0 and (m // r[0]) * (n // r[1]) >= min(self.threads, m * n)), (1, 1))
 
         def emit() -> None:
-            self.put(f"for (int _t = threadIdx.x; _t < {(m // rm) * (n // rn)}; _t += {THREADS}) {{")
+            self.put(f"for (int _t = threadIdx.x; _t < {(m // rm) * (n // rn)}; _t += {self.threads}) {{")
             self.depth += 1
             self.put(f"const int _i = _t / {n // rn} * {rm}, _j = _t % {n // rn} * {rn};")
             kind = "unsigned" if integer else "float"
             self.put(f"{kind} _s[{rm}][{rn}];")
+            start = "0" if zero else f"({kind}){acc}[(_i + _y) * {n} + _j + _x]"
             each = f"for (int _y = 0; _y < {rm}; ++_y) for (int _x = 0; _x < {rn}; ++_x)"
-            self.put(f"_Pragma(\"unroll\") {each} _s[_y][_x] = ({kind}){acc}[(_i + _y) * {n} + _j + _x];")
+            self.put(f"_Pragma(\"unroll\") {each} _s[_y][_x] = {start};")
             self.put(f"_Pragma(\"unroll 4\") for (int _k = 0; _k < {k}; ++_k) {{")
             self.put(f"  {stage} _p[{rm}], _q[{rn}];")
             self.put(f"  for (int _y = 0; _y < {rm}; ++_y) _p[_y] = {a}[_k * {m + 4} + _i + _y];")
@@ -671,7 +718,7 @@ class Emitter:
             self.put(f"_Pragma(\"unroll\") {each} {acc}[(_i + _y) * {n} + _j + _x] = ({stage})_s[_y][_x];")
             self.depth -= 1
             self.put("}")
-            for name in (a, b, acc):
+            for name in (a, b, *(() if zero else (acc,))):
                 self.access(name, "any")
             self.access(acc, "any", write=True)
 
@@ -705,7 +752,7 @@ class Emitter:
         acc = self.tile_vars[s.acc.name][0]
         (m, k), n = s.lhs.shape, s.rhs.shape[1]
         per = form.k_step // 4  # operand elements per lane per instruction
-        pitch = k + 16 // SIZES[form.element]
+        pitch, zero = k + 16 // SIZES[form.element], self.fresh_acc
         at = self.mfma_stage(form, s.lhs, m, k, pitch, transposed=False)
         bt = self.mfma_stage(form, s.rhs, n, k, pitch, transposed=True)
         acc_t = "int" if form.integer else "float"
@@ -713,10 +760,11 @@ class Emitter:
         def emit() -> None:
             self.put("{")
             self.put("  const int _w = threadIdx.x >> 6, _l = threadIdx.x & 63, _r = _l & 15, _q = _l >> 4;")
-            self.put(f"  for (int _blk = _w; _blk < {(m // 16) * (n // 16)}; _blk += {THREADS // 64}) {{")
+            self.put(f"  for (int _blk = _w; _blk < {(m // 16) * (n // 16)}; _blk += {self.threads // 64}) {{")
             self.put(f"    const int _m0 = (_blk / {n // 16}) * 16, _n0 = (_blk % {n // 16}) * 16;")
             self.put(f"    {form.acc_vec} _c;")
-            self.put(f"    for (int _i = 0; _i < 4; ++_i) _c[_i] = {acc}[(_m0 + 4 * _q + _i) * {n} + _n0 + _r];")
+            start = "0" if zero else f"{acc}[(_m0 + 4 * _q + _i) * {n} + _n0 + _r]"
+            self.put(f"    for (int _i = 0; _i < 4; ++_i) _c[_i] = {start};")
             self.put(f"    for (int _k = 0; _k < {k}; _k += {form.k_step}) {{")
             vec = form.operand_vec
             self.put(f"      const {vec} _a = *(const {vec}*)&{at}[(_m0 + _r) * {pitch} + _k + _q * {per}];")
@@ -726,7 +774,7 @@ class Emitter:
             self.put(f"    for (int _i = 0; _i < 4; ++_i) {acc}[(_m0 + 4 * _q + _i) * {n} + _n0 + _r] = ({acc_t})_c[_i];")
             self.put("  }")
             self.put("}")
-            for name in (at, bt, acc):
+            for name in (at, bt, *(() if zero else (acc,))):
                 self.access(name, "any")
             self.access(acc, "any", write=True)
 
@@ -742,10 +790,7 @@ class Emitter:
         def body(idx):
             kk, rr = (idx[0], idx[1]) if along_rows else (idx[1], idx[0])
             x, ok = self.value(e, [kk, rr] if transposed else [rr, kk])
-            bits = {"f16": f"__builtin_bit_cast(unsigned short, (_Float16){x})",
-                    "bf16": f"(unsigned short)(__float_as_uint({x}) >> 16)",
-                    "fp8": f"(unsigned char){x}",  # the e4m3 code as the tile holds it
-                    "i8": f"(signed char){x}"}[form.name]
+            bits = self.mfma_bits(form, x)
             self.put(f"{name}[{rr} * {pitch} + {kk}] = {bits if ok == '1' else f'({ok}) ? {bits} : ({form.element})0'};")
             self.access(name, "any", write=True)
 
@@ -753,6 +798,8 @@ class Emitter:
         return name
 
     def stmt_For(self, s: ir.For) -> None:
+        if self.pipelined_product(s):
+            return
         var = s.var.name
         if self.pending:
             self.barrier()  # the body's first accesses are checked against its own last ones only
@@ -763,6 +810,186 @@ class Emitter:
             self.barrier()
         self.depth -= 1
         self.put("}")
+
+    def pipelined_product(self, s: ir.For) -> bool:
+        """The loop of a matrix product, `acc += a[.., ks] @ b[ks, ..]` (or the transpose of b[.., ks]) alone in its body:
+        the accumulators stay in registers over the whole loop, the next step's elements are loaded while this one
+        multiplies, and two LDS stages leave one barrier per step (f32 256^3 with 32 x 32 tiles, 16 steps of one load's
+        latency each: 21.6 us before, 13.4 now). Anything else (other statements in the body, computed operands, tiles with more
+        outputs than the threads hold) is False, and runs statement by statement."""
+        if len(s.body) != 1 or not isinstance(s.body[0], ir.Accumulate):
+            return False
+        product = s.body[0]
+        lhs, rhs = product.lhs, product.rhs
+        turned = isinstance(rhs, ir.Transpose)
+        loads = (lhs, rhs.operand if turned else rhs)
+        if not all(isinstance(e, ir.TileLoad) and len(e.shape) == 2 for e in loads):
+            return False
+        (m, k), n, var = lhs.shape, rhs.shape[1], s.var.name
+        axes = [[a for a, sl in enumerate(e.slices) if not sl.squeeze] for e in loads]
+        k_axes = [axes[0][1], axes[1][1] if turned else axes[1][0]]
+        if any(self.mentions(sl.start, var) for e, ka in zip(loads, k_axes) for a, sl in enumerate(e.slices) if a != ka):
+            return False
+        form, integer = mfma_form(product), product.acc.dtype == I32
+        acc, valid = self.tile_vars[product.acc.name]
+        waves = self.threads // 64
+        if form is not None:
+            element, pitches = form.element, (k + 16 // SIZES[form.element],) * 2
+            sizes = (m * pitches[0], n * pitches[1])
+            held = -(-(m // 16) * (n // 16) // waves)
+            if held > 16:
+                return False
+        else:
+            element, pitches = ("int" if integer else "float"), (m + 4, n + 4)
+            sizes = (k * pitches[0], k * pitches[1])
+            shape = next((r for r in ((1, 1), (1, 2), (2, 2), (2, 4), (4, 4), (4, 8), (8, 8))
+                          if m % r[0] == 0 and n % r[1] == 0 and (m // r[0]) * (n // r[1]) <= self.threads), None)
+            if shape is None:
+                return False
+        if self.top + 2 * sum(sizes) * SIZES[element] + 64 > LDS_LIMIT:
+            return False
+        stages = [self.reserve(self.fresh("st"), element, 2 * size) for size in sizes]
+        counts = [-(-m * k // self.threads), -(-n * k // self.threads)]
+        regs = [self.fresh("r"), self.fresh("r")]
+
+        def each(body) -> None:
+            """`body(stage, registers, index, expression, row, k position)` for every element a thread moves."""
+            for i, (e, rows) in enumerate(((lhs, m), (rhs, n))):
+                along_rows = i == 1 and not turned
+                inner = rows if along_rows else k
+                self.put(f'_Pragma("unroll") for (int _u = 0; _u < {counts[i]}; ++_u) {{')
+                self.depth += 1
+                self.put(f"const int _e = threadIdx.x + _u * {self.threads}, _i0 = _e / {inner}, _i1 = _e % {inner};")
+                whole = rows * k % self.threads == 0
+                self.put("{" if whole else f"if (_e < {rows * k}) {{")
+                self.memo = {}
+                row, at = ("_i1", "_i0") if along_rows else ("_i0", "_i1")
+                body(i, e, row, at)
+                self.put("}")
+                self.depth -= 1
+                self.put("}")
+
+        def fetch() -> None:
+            self.node, reads = {}, self.reads
+            for e in (lhs, rhs):
+                self.prepare(e, product=True)
+
+            def one(i, e, row, at):
+                x, ok = self.value(e, [row, at] if i == 0 else [at, row])
+                if form is None:
+                    x = f"k8dec({x})" if e.dtype.is_narrow else f"({element}){x}"
+                else:
+                    x = self.mfma_bits(form, x)
+                self.put(f"{regs[i]}[_u] = ({ok}) ? {x} : ({element})0;")
+
+            each(one)
+            self.reads, self.memo = reads, {}
+
+        def stage(i, e, row, at):
+            place = f"{row} * {pitches[i]} + {at}" if form is not None else f"{at} * {pitches[i]} + {row}"
+            self.put(f"{stages[i]}[_p * {sizes[i]} + {place}] = {regs[i]}[_u];")
+
+        if self.pending:
+            self.barrier()
+        hi = self.scalar(s.hi)
+        self.put(f"long long {var} = {self.scalar(s.lo)};")
+        self.put(f"if ({var} < {hi}) {{")
+        self.depth += 1
+        for name, count in zip(regs, counts):
+            self.put(f"{element} {name}[{count}];")
+        self.put("int _p = 0; unsigned char _kok = 1;")
+        kind = "unsigned" if integer else "float"
+        if form is not None:
+            at16 = f"[(_m0 + 4 * _q + _i) * {n} + _n0 + _r]"
+            self.put("const int _w = threadIdx.x >> 6, _l = threadIdx.x & 63, _r = _l & 15, _q = _l >> 4;")
+            self.put(f"{form.acc_vec} _c[{held}];")
+            blocks = (f'_Pragma("unroll") for (int _b = 0; _b < {held}; ++_b) {{ const int _blk = _w + _b * {waves}, '
+                      f"_m0 = _blk / {n // 16} * 16, _n0 = _blk % {n // 16} * 16; "
+                      f"if (_blk < {(m // 16) * (n // 16)}) {{")
+            self.put(f"{blocks} for (int _i = 0; _i < 4; ++_i) _c[_b][_i] = {acc}{at16}; }} }}")
+        else:
+            rm, rn = shape
+            live = f"if (threadIdx.x < {(m // rm) * (n // rn)})"
+            self.put(f"const int _i = threadIdx.x / {n // rn} * {rm}, _j = threadIdx.x % {n // rn} * {rn};")
+            self.put(f"{kind} _s[{rm}][{rn}];")
+            cell = (f'_Pragma("unroll") for (int _y = 0; _y < {rm}; ++_y) _Pragma("unroll") '
+                    f"for (int _x = 0; _x < {rn}; ++_x)")
+            self.put(f"{live} {{ {cell} _s[_y][_x] = ({kind}){acc}[(_i + _y) * {n} + _j + _x]; }}")
+        self.put("{")
+        self.depth += 1
+        fetch()
+        self.depth -= 1
+        self.put("}")
+        self.put("for (;;) {")
+        self.depth += 1
+        each(stage)
+        self.put("__syncthreads();")  # the other stage's readers are a whole step behind
+        self.put(f"const long long _next = {var} + {s.step};")
+        self.put(f"if (_next < {hi}) {{")
+        self.depth += 1
+        self.put(f"const long long {var} = _next;")
+        fetch()
+        self.depth -= 1
+        self.put("}")
+        for e, ka in zip(loads, k_axes):
+            start = self.scalar(e.slices[ka].start)
+            self.put(f"_kok &= ({start}) < {e.tensor.name}_n{ka} && ({start}) + {k} > 0;")
+        if form is not None:
+            per, vec = form.k_step // 4, form.operand_vec
+            self.put(f"{blocks} _Pragma(\"unroll\") for (int _k = 0; _k < {k}; _k += {form.k_step}) {{")
+            for name, stem, origin, i in (("_a", stages[0], "_m0", 0), ("_b2", stages[1], "_n0", 1)):
+                self.put(f"  const {vec} {name} = *(const {vec}*)&{stem}[_p * {sizes[i]} + ({origin} + _r) * {pitches[i]}"
+                         f" + _k + _q * {per}];")
+            self.put(f"  _c[_b] = {form.builtin}(_a, _b2, _c[_b], 0, 0, 0);")
+            self.put("} } }")
+            self.mfma_products += 1
+        else:
+            self.put(f"{live} {{")
+            self.put(f'  _Pragma("unroll 8") for (int _k = 0; _k < {k}; ++_k) {{')
+            self.put(f"    {element} _f[{rm}], _g[{rn}];")
+            self.put(f"    for (int _y = 0; _y < {rm}; ++_y) _f[_y] = "
+                     f"{stages[0]}[_p * {sizes[0]} + _k * {pitches[0]} + _i + _y];")
+            self.put(f"    for (int _x = 0; _x < {rn}; ++_x) _g[_x] = "
+                     f"{stages[1]}[_p * {sizes[1]} + _k * {pitches[1]} + _j + _x];")
+            step = ("_s[_y][_x] += (unsigned)(_f[_y] * _g[_x]);" if integer
+                    else "_s[_y][_x] = fmaf(_f[_y], _g[_x], _s[_y][_x]);")
+            self.put(f"    {cell} {step}")
+            self.put("  }")
+            self.put("}")
+        self.put(f"if (_next >= {hi}) break;")
+        self.put(f"{var} = _next; _p ^= 1;")
+        self.depth -= 1
+        self.put("}")
+        if form is not None:
+            cast = "int" if form.integer else "float"
+            self.put(f"{blocks} for (int _i = 0; _i < 4; ++_i) {acc}{at16} = ({cast})_c[_b][_i]; }} }}")
+        else:
+            self.put(f"{live} {{ {cell} {acc}[(_i + _y) * {n} + _j + _x] = ({element})_s[_y][_x]; }}")
+        self.node = {}
+        for e in (lhs, rhs):
+            self.prepare(e, product=True)
+        rows, cols = self.any_valid(lhs, m, k, False)[1], self.any_valid(rhs, n, k, True)[1]
+        self.put(f"for (int _e = threadIdx.x; _e < {m * n}; _e += {self.threads}) {{")
+        self.put(f"  const int _i0 = _e / {n}, _i1 = _e % {n};")
+        self.put(f"  {valid}[_e] = {valid}[_e] & _kok & ({rows('_i0')}) & ({cols('_i1')});")
+        self.put("}")
+        self.depth -= 1
+        self.put("}")
+        self.barrier()
+        return True
+
+    @staticmethod
+    def mentions(e: ir.Expr, name: str) -> bool:
+        return (isinstance(e, (ir.Var, ir.Param)) and e.name == name) or any(
+            Emitter.mentions(child, name) for child in ir.children(e))
+
+    @staticmethod
+    def mfma_bits(form: "MfmaForm", x: str) -> str:
+        """An element as the bits of a matrix-core operand."""
+        return {"f16": f"__builtin_bit_cast(unsigned short, (_Float16){x})",
+                "bf16": f"(unsigned short)(__float_as_uint({x}) >> 16)",
+                "fp8": f"(unsigned char){x}",  # the e4m3 code as the tile holds it
+                "i8": f"(signed char){x}"}[form.name]
 
     def stmt_If(self, s: ir.If) -> None:
         if self.pending:

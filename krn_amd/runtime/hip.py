@@ -250,8 +250,8 @@ def _kind(argument: object) -> object:
 class Program:
     """A hiprtc-compiled module with one entry point."""
 
-    def __init__(self, source: str, entry: str, scratch: int = 0) -> None:
-        self.source, self.entry, self.scratch = source, entry, scratch
+    def __init__(self, source: str, entry: str, threads: int, scratch: int = 0) -> None:
+        self.source, self.entry, self.threads, self.scratch = source, entry, threads, scratch
         self.code = hipapi.rtc().compile(source, entry, HIPRTC_OPTIONS)
         module = c_void_p()
         buffer = ctypes.create_string_buffer(self.code, len(self.code))
@@ -283,7 +283,7 @@ def generic_program(kernel: ir.Kernel) -> Program:
     digest = hashlib.sha256(source.encode()).hexdigest()
     with _programs_lock:
         if digest not in _programs:
-            _programs[digest] = Program(source, entry, scratch)
+            _programs[digest] = Program(source, entry, hipgen.threads(kernel), scratch)
         return _programs[digest]
 
 
@@ -436,7 +436,7 @@ class Launch:
             return lambda stream: None  # a zero-extent grid launches nothing (reference cuda_backend.py:377-383)
         if not program.scratch:
             table = Program.table(params)
-            return lambda stream: program.launch(dims, hipgen.THREADS, table, stream.handle)
+            return lambda stream: program.launch(dims, program.threads, table, stream.handle)
         scratch = StreamScratch(blocks * program.scratch)
         slot = c_void_p(0)
         table = Program.table([*params, slot])
@@ -444,7 +444,7 @@ class Launch:
         def run(stream: HIPStream) -> None:
             memory = scratch.on(stream)
             slot.value = memory.pointer
-            program.launch(dims, hipgen.THREADS, table, stream.handle)
+            program.launch(dims, program.threads, table, stream.handle)
             stream.note(self.kernel.name, (memory,))
 
         return run

@@ -143,8 +143,9 @@ def mfma_form(s: ir.Accumulate) -> MfmaForm | None:
 def threads(kernel: ir.Kernel) -> int:
     """Threads of one block: 256, and 1024 for programs whose tiles have 4096 elements and more and whose products, if
     any, run on the matrix cores. Their LDS leaves room for one or two blocks on a CU, and 256 threads would be one
-    wave per SIMD with nothing to cover its LDS latency (flash attention, 64 x 64 tiles, d = 32: 16 x 512: 100 us with 256 threads, 51 with 1024). A scalar
-    product keeps 256: fewer outputs per thread are more LDS reads per multiply-add."""
+    wave per SIMD with nothing to cover its LDS latency (flash attention, 64 x 64 tiles, d = 32, 16 x 512:
+    100 us with 256 threads, 51 with 1024). A scalar product keeps 256: fewer outputs per thread are more LDS reads per
+    multiply-add."""
     large = max((math.prod(v.shape) for v in kernel.tiles), default=1) >= 4096
     scalar = any(isinstance(s, ir.Accumulate) and mfma_form(s) is None for s in ir.walk(kernel.body))
     return 1024 if large and not scalar else 256

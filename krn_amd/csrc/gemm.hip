@@ -1144,10 +1144,12 @@ static bool nn_direct(const void* a, const void* b, int64_t m, int64_t n, int64_
 // Estimated microseconds of a split-kernel launch beyond its fixed cost, from sweeps of each tile over 10 to 1500
 // workgroups (bf16 unless noted): a 128-byte K slice takes a CU `slice` us, with `more` us for every workgroup the
 // busiest CU holds once that is larger. 256 x 4096 x 4096 on 64 x 64 tiles 16.6 us (one workgroup per CU), 512 rows
-// 26 us (two); 128 x 128 tiles 44 us at 1024 x 4096 x 4096; unaligned 1024 x 4096 x 4097 60 us on 128 x 128.
+// 26 us (two); 128 x 128 tiles, operands from HBM: two workgroups per CU 56.8 us at 256 x 4096 x 14336 in eight parts,
+// one with four stages 51.3 in four, 78 at 512 x 8192 x 8192 (the four-wave loop 95);
+// unaligned 1024 x 4096 x 4097 60 us on 128 x 128.
 static double split_cost(int shape, bool nn, int64_t m, int64_t n, int64_t slices, int parts) {
   static const struct { int bm, bn; double slice, more, more_nn; } T[] = {
-      {32, 64, 0.23, 0.15, 0.17},   {64, 64, 0.28, 0.22, 0.25},   {128, 128, 0.62, 0.43, 0.52}, {128, 128, 0.70, 0.70, 0.75},
+      {32, 64, 0.23, 0.15, 0.17},   {64, 64, 0.28, 0.22, 0.25},   {128, 128, 0.80, 0.60, 0.52}, {128, 128, 0.62, 0.62, 0.82},
       {32, 128, 0.70, 0.75, 0.75},  {64, 64, 0.43, 0.35, 0.38},   {128, 128, 0.92, 0.92, 0.95}};
   const int64_t wgs = ((m + T[shape].bm - 1) / T[shape].bm) * ((n + T[shape].bn - 1) / T[shape].bn) * parts;
   const double per_cu = (double)((wgs + 255) / 256);
@@ -1192,7 +1194,7 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
     if (m <= 64 || elem == 1) return best;
     least -= 2.0;  // near ties stay (89 x 1536 x 2560 f16: 11.0 us, 32 x 64 tiles 11.7)
   } else if (piped && 128 * kbytes <= 0x7fffffff) {
-    if (t128 <= 256) best = {MID, 0, 1, 0}, least = 0.60 * (double)slices;
+    if (t128 <= 256) best = {MID, 0, 1, 0}, least = 0.66 * (double)slices;
     else if (fmt != FMT_FP8 && 256 * kbytes <= 0x7fffffff)
       best = {BAND, 0, 1, 0},
       least = 0.95 * (double)slices * (double)((((m + 127) / 128) * ((n + 255) / 256) + 255) / 256);

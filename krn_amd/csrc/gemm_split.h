@@ -15,7 +15,7 @@ __device__ __forceinline__ int kn_slot(int k, int c) {
 }
 
 // Tile and loader: the ring of direct-to-LDS slices needs 16-byte aligned rows, the other takes any alignment. DEEP:
-// four stages instead of two, for one workgroup per CU.
+// four stages instead of two, for one workgroup per CU (NT: fragments read a slice ahead).
 enum SplitShape : int {
   RING_32x64, RING_64x64, RING_128x128, RING_128x128_DEEP, ANY_32x128, ANY_64x64, ANY_128x128
 };

@@ -29,6 +29,15 @@ def test_int8_products_of_every_split_and_alignment_are_bit_exact(device, m, n, 
     np.testing.assert_array_equal(c.to_host(), want.astype(np.int32))
 
 
+@pytest.mark.parametrize("k", [16, 128, 144, 272, 400, 512, 528, 640, 656, 1040])
+def test_int8_products_of_one_to_nine_slices_on_128_by_128_tiles_are_bit_exact(device, k):
+    rng = np.random.default_rng(k)
+    a, w = rng.integers(-127, 128, (2000, k), dtype=np.int8), rng.integers(-127, 128, (2010, k), dtype=np.int8)
+    c = device.empty(T.i32, 2000, 2010)
+    programs.gemm_i8_i32[programs.Tiling(bm=64, bn=64, bk=64)](device.to_device(a), device.to_device(w), c)
+    np.testing.assert_array_equal(c.to_host(), (a.astype(np.float64) @ w.astype(np.float64).T).astype(np.int32))
+
+
 @pytest.mark.parametrize("m,n,k", [(129, 130, 8192), (128, 520, 16384), (257, 100, 5000)])
 def test_w8a8_scales_apply_once_to_the_sum_of_the_parts(device, m, n, k):
     rng = np.random.default_rng(m + n + k)

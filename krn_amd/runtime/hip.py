@@ -113,6 +113,9 @@ class HIPEvent(Event):
 KEEP_LIMIT = 256  # launches a stream holds before it records a marker of its own (reference completion.py:19)
 
 
+WORKSPACE_KEPT = 256 << 20  # bytes of scratch a stream keeps for its launches: sixteen K parts of 1024 x 4096 sums
+
+
 class HIPStream(Stream):
     """An in-order queue of device work. A launch's arguments are held until a marker event recorded after it has
     completed (the `Keeper` of reference runtime/completion.py:99-131): `record()` closes the open launches under its
@@ -129,8 +132,9 @@ class HIPStream(Stream):
         """At least `nbytes` of device scratch for one launch on this stream. Launches on a stream run in order, so they
         share one buffer, which grows to the largest request and is freed with the stream; a launch holds it until
         it has completed, so a buffer outgrown meanwhile (by another thread, too) is freed after its last use. A
-        launch that a graph records gets memory of its own, which the graph keeps: its replays run on any stream."""
-        if self.capturing:
+        request above WORKSPACE_KEPT is that launch's own and goes back after it. A launch that a graph records gets
+        memory of its own, which the graph keeps: its replays run on any stream."""
+        if self.capturing or nbytes > WORKSPACE_KEPT:
             return self.device.empty_on(self, D.U8, nbytes)
         held = self._workspace
         if held is None or held.nbytes < nbytes:

@@ -101,3 +101,17 @@ def test_a_split_product_replays_from_a_graph_between_eager_calls_and_on_two_str
         device.sync()
         for (_, _, c), want in zip(inputs, wants):
             np.testing.assert_array_equal(c.to_host(), want)
+
+
+@pytest.mark.parametrize("kept", [0, 1 << 30])
+def test_a_workspace_above_what_a_stream_keeps_is_the_launches_own(device, monkeypatch, kept):
+    monkeypatch.setattr("krn_amd.runtime.hip.WORKSPACE_KEPT", kept)
+    rng = np.random.default_rng(kept)
+    a, w = rng.integers(-127, 128, (129, 8192), dtype=np.int8), rng.integers(-127, 128, (31, 8192), dtype=np.int8)
+    want = a.astype(np.int64) @ w.astype(np.int64).T
+    with device.stream() as stream:
+        c = device.empty(T.i32, 129, 31)
+        for _ in range(3):
+            programs.gemm_i8_i32[programs.Tiling(bm=64, bn=64, bk=64)](device.to_device(a), device.to_device(w), c)
+            np.testing.assert_array_equal(c.to_host(), want.astype(np.int32))
+        assert (stream._workspace is None) == (kept == 0)

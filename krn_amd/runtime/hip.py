@@ -127,6 +127,7 @@ class HIPStream(Stream):
         self._open: list[tuple[str, tuple[object, ...]]] = []
         self._marks: deque[tuple[HIPEvent, list[tuple[str, tuple[object, ...]]]]] = deque()
         self._workspace: HIPTensor | None = None
+        self.workspace_lock = threading.Lock()  # held while a call that uses the workspace puts its kernels on the stream
 
     def workspace(self, nbytes: int) -> "HIPTensor":
         """At least `nbytes` of device scratch for one launch on this stream. Launches on a stream run in order, so they
@@ -371,12 +372,15 @@ class Launch:
         return self._with_workspace(product, need)
 
     def _with_workspace(self, call: Callable[[int, int], None], nbytes: int) -> Callable[[HIPStream], None]:
-        """`call(workspace, stream)` with the stream's workspace, held until the launch has completed."""
+        """`call(workspace, stream)` with the stream's workspace, held until the launch has completed. The call puts
+        two kernels on the stream, the second reading what the first left in the workspace, and runs without the
+        interpreter's lock: another thread's call must not put its own between them."""
 
         def run(stream: HIPStream) -> None:
-            workspace = stream.workspace(nbytes)
-            call(workspace.pointer, stream.handle)
-            stream.note(self.kernel.name, (workspace,))
+            with stream.workspace_lock:
+                workspace = stream.workspace(nbytes)
+                call(workspace.pointer, stream.handle)
+                stream.note(self.kernel.name, (workspace,))
 
         return run
 

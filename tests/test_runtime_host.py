@@ -191,3 +191,31 @@ def test_a_kernel_parameter_table_keeps_its_parameters_alive():
     gc.collect()
     _ = [ctypes.c_int64(-1) for _ in range(1000)]  # reuse of freed memory would show here
     assert [ctypes.c_int64.from_address(a).value for a in table] == [1111 * i for i in range(6)] + [0xABC]
+
+
+def test_threads_sharing_a_stream_do_not_interleave_calls_on_its_workspace(fake):
+    """A call that uses the stream's workspace launches two kernels, the second reading what the first wrote there;
+    the library runs without the interpreter's lock, so a second thread's call could otherwise launch between them."""
+    import threading
+    import time
+
+    def empty(stream, dtype, nbytes):
+        return SimpleNamespace(nbytes=nbytes, pointer=16)
+
+    stream = hip.HIPStream(SimpleNamespace(empty_on=empty), 1)
+    order = []
+
+    def call(workspace, handle):
+        order.append((threading.get_ident(), "write"))
+        time.sleep(0.02)  # as in the library: the other thread may run here
+        order.append((threading.get_ident(), "read"))
+
+    launch = hip.Launch(SimpleNamespace(name="split"), None)
+    runs = [launch._with_workspace(call, nbytes) for nbytes in (64, 128)]
+    threads = [threading.Thread(target=lambda r=r: [r(stream) for _ in range(3)]) for r in runs]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert len(order) == 12 and len(stream.pending_launches()) == 6
+    assert all(order[i][0] == order[i + 1][0] for i in range(0, 12, 2))

@@ -181,16 +181,23 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : WAVES * 64) void softmax_rows(co
 
 using namespace krn;
 
+// A workgroup per row takes the rows in runs of 2^21: a launch holds fewer than 2^32 threads, which 2^22 rows of sixteen
+// waves reach. A wave per row needs 2^26 rows for that.
 template <int KIND, int CACHE, int WAVES>
 static void launch_rows(bool aligned, const void* x, void* y, int64_t rows, int64_t width, int64_t ldx, int64_t ldy,
                         hipStream_t stream) {
-  const dim3 grid((unsigned)(WAVES == 1 ? (rows + 3) / 4 : rows)), block(WAVES == 1 ? 256 : WAVES * 64);
-  if (aligned)
-    hipLaunchKernelGGL((softmax_rows<KIND, CACHE, WAVES, true>), grid, block, 0, stream, (const uint8_t*)x, (uint8_t*)y,
-                       rows, width, ldx, ldy);
-  else
-    hipLaunchKernelGGL((softmax_rows<KIND, CACHE, WAVES, false>), grid, block, 0, stream, (const uint8_t*)x, (uint8_t*)y,
-                       rows, width, ldx, ldy);
+  constexpr int64_t BYTES = Chunk<KIND>::BYTES;
+  const int64_t most = WAVES == 1 ? rows : (int64_t)1 << 21;
+  for (int64_t r0 = 0; r0 < rows; r0 += most) {
+    const int64_t n = rows - r0 < most ? rows - r0 : most;
+    const dim3 grid((unsigned)(WAVES == 1 ? (n + 3) / 4 : n)), block(WAVES == 1 ? 256 : WAVES * 64);
+    const uint8_t* xr = (const uint8_t*)x + r0 * ldx * BYTES;
+    uint8_t* yr = (uint8_t*)y + r0 * ldy * BYTES;
+    if (aligned)
+      hipLaunchKernelGGL((softmax_rows<KIND, CACHE, WAVES, true>), grid, block, 0, stream, xr, yr, n, width, ldx, ldy);
+    else
+      hipLaunchKernelGGL((softmax_rows<KIND, CACHE, WAVES, false>), grid, block, 0, stream, xr, yr, n, width, ldx, ldy);
+  }
 }
 
 template <int KIND>

@@ -391,7 +391,7 @@ static void launch_attention(const void* q, const void* k, const void* v, void* 
 // the shorter taken. A workgroup above takes 1.8 us (d = 64: 1.35) per 64 keys, whatever its rows, and the launch 4
 // more; a wave of the key-split kernel 1.6 us per 32 keys (d = 64: 0.93 alone on its CU, 1.15 in twos), a workgroup
 // 2.6, a launch 3, the reduction of several parts 3 and the planes' bytes. Measured, both sides: 128 heads x 1 query x
-// 4096 keys, d = 128: 113 -> 57 us (two parts; 268 MB of K and V); 32 x 1 x 8192: 203 -> 29 (eight); 16 x 1000 x 1000,
+// 4096 keys, d = 128: 113 -> 52 us (two parts; 268 MB of K and V); 32 x 1 x 8192: 203 -> 29 (eight); 16 x 1000 x 1000,
 // d = 64: 25.9 -> 13.0; causal 32 x 512 x 512, d = 128: 19.4 -> 15.6; causal 32 x 1024 x 1024: 33.3 against 41.0, so
 // launches that fill the chip with 256-row workgroups stay there.
 static int attention_parts(int64_t bh, int64_t sq, int64_t sk, int64_t d, int causal, int64_t workspace) {

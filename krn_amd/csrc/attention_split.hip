@@ -31,7 +31,7 @@ __device__ __forceinline__ void v_fragments(uint32_t at, u32x4 (&va)[2]) {
   va[1] = u32x4{w[2][0], w[2][1], w[3][0], w[3][1]};
 }
 
-template <bool BF, int D>
+template <bool BF, int D, bool ONCE>
 __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attention_split(
     const uint16_t* __restrict__ Q, const uint16_t* __restrict__ K, const uint16_t* __restrict__ V,
     uint16_t* __restrict__ O, float* __restrict__ planes, int64_t sq, int64_t sk, float scale, int q_tiles, int causal,
@@ -81,8 +81,8 @@ __global__ __launch_bounds__(64 * SPLIT_WAVES, 2) void attention_split(
 #pragma unroll
     for (int j = 0; j < LOADS; ++j) {
       const bool out = ragged && key0 + j * ROWS_PER_LOAD + lrow >= sk;
-      buffer_to_lds16(k_rsrc, st + j * 1024, out ? OUTSIDE_HEAD : koff[j], soff);
-      buffer_to_lds16(v_rsrc, st + TILE + j * 1024, out ? OUTSIDE_HEAD : voff[j], soff);
+      buffer_to_lds16<ONCE>(k_rsrc, st + j * 1024, out ? OUTSIDE_HEAD : koff[j], soff);
+      buffer_to_lds16<ONCE>(v_rsrc, st + TILE + j * 1024, out ? OUTSIDE_HEAD : voff[j], soff);
     }
   };
 
@@ -230,11 +230,11 @@ __global__ __launch_bounds__(256) void attention_reduce(const float* __restrict_
 
 using namespace krn;
 
-template <bool BF, int D>
+template <bool BF, int D, bool ONCE>
 static int launch(const AttentionCall& c) {
   const int q_tiles = (int)((c.sq + 31) / 32);
   const dim3 grid((unsigned)(c.bh * q_tiles * c.parts));
-  hipLaunchKernelGGL((attention_split<BF, D>), grid, dim3(64 * SPLIT_WAVES), 0, c.stream, (const uint16_t*)c.q,
+  hipLaunchKernelGGL((attention_split<BF, D, ONCE>), grid, dim3(64 * SPLIT_WAVES), 0, c.stream, (const uint16_t*)c.q,
                      (const uint16_t*)c.k, (const uint16_t*)c.v, (uint16_t*)c.o, (float*)c.workspace, c.sq, c.sk,
                      c.scale, q_tiles, c.causal, c.parts, (int)c.bh);
   if (c.parts > 1) {
@@ -250,7 +250,15 @@ static int launch(const AttentionCall& c) {
   return 0;
 }
 
+// Up to 32 query rows a head are one row block, whose keys and values are read once. From 128 MiB of them, half of the
+// last-level cache, their loads are non-temporal, since little would be found there by a later launch anyway (d = 128,
+// one query, bf16: 128 heads x 4096 keys 57.4 -> 52.0 us, 4.7 -> 5.2 TB/s; 128 x 16384 190.9 -> 170.3; 32 x 8192, 128 MiB,
+// 34.7 -> 32.0). Smaller ones keep ordinary loads (8 heads x 16384 keys, 64 MiB: 24.3 us, non-temporally 27.8), and so do
+// longer prompts, whose row blocks share keys in L2 (16 x 1000 x 1000, d = 64: 11.9 us, non-temporally 13.2).
 int krn::launch_attention_split(bool bf, int d, const AttentionCall& c) {
-  if (bf) return d == 128 ? launch<true, 128>(c) : launch<true, 64>(c);
-  return d == 128 ? launch<false, 128>(c) : launch<false, 64>(c);
+  const bool once = c.sq <= 32 && c.bh * c.sk * d * 4 >= (int64_t)128 << 20;
+#define KRN_SPLIT(BFV, DV) (once ? launch<BFV, DV, true>(c) : launch<BFV, DV, false>(c))
+  if (bf) return d == 128 ? KRN_SPLIT(true, 128) : KRN_SPLIT(true, 64);
+  return d == 128 ? KRN_SPLIT(false, 128) : KRN_SPLIT(false, 64);
+#undef KRN_SPLIT
 }

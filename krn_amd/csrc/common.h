@@ -46,9 +46,12 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t panel_rsrc(const void* base, i
 }
 
 // 16 bytes per lane from resource offset voff + soff straight into LDS: the wave's 64 lanes fill 1 KiB at `dst`
-// (buffer_load_dwordx4 ... lds). A device function so that the host pass never sees the builtin.
+// (buffer_load_dwordx4 ... lds), non-temporally (the nt bit) with NT. A device function so that the host pass never sees
+// the builtin.
+template <bool NT = false>
 __device__ __forceinline__ void buffer_to_lds16(__amdgpu_buffer_rsrc_t r, void* dst, uint32_t voff, int soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, voff, soff, 0,
+                                           NT ? 2 : 0);
 }
 
 }  // namespace krn

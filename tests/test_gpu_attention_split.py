@@ -14,9 +14,10 @@ from oracle.numerics import bf16_values, bf16_words
 
 pytestmark = pytest.mark.gpu
 
-# one query, a few, one row more than a block; keys fewer than a tile, one more than a tile, several parts
+# one query, a few, a whole block, one row more than a block; keys fewer than a tile, one more than a tile, several parts;
+# 128 MiB of keys and values (d = 128), read non-temporally
 SHAPES = [(1, 1, 1), (2, 1, 33), (3, 5, 333), (8, 1, 16384), (32, 1, 8200), (128, 8, 2000), (2, 33, 31), (4, 100, 1000),
-          (16, 300, 300), (5, 31, 4097)]
+          (16, 300, 300), (5, 31, 4097), (3, 32, 500), (32, 3, 8193)]
 
 
 def attend(device, dtype, q, k, v, scale, causal, workspace=True):

@@ -167,6 +167,19 @@ def products(kernel: ir.Kernel) -> list[str]:
     return found
 
 
+# A program's own names in the source: prefixed, so that neither a parameter nor a name that capture gives a loop variable
+# (`_i1` for the first `i`) can be one of the emitter's (`_i1` is a loop's column index), of the prelude's or of HIP's
+
+
+def user(name: str) -> str:
+    return f"u_{name}"
+
+
+def dim(tensor: str, axis: int) -> str:
+    """`tensor.shape[axis]`; no parameter can have this name (`user` begins with u, and no local with n)."""
+    return f"n{axis}_{tensor}"
+
+
 Access = tuple[tuple, str]  # a resource (("lds", first byte, end byte) or ("tensor", name)) and how it is indexed
 
 
@@ -291,11 +304,11 @@ class Emitter:
         self.body(self.kernel.body)
         params = []
         for name, kind in self.kernel.params:
-            for slot, dtype, role in ir.slots(name, kind):
-                if role == "ptr":
-                    params.append(f"{storage(dtype)}* __restrict__ {slot}")
-                else:
-                    params.append(f"{ctype(dtype if dtype != I64 else PY_INT)} {slot}")
+            if isinstance(kind, ir.TensorType):
+                params.append(f"{storage(kind.dtype)}* __restrict__ {user(name)}")
+                params += [f"long long {dim(name, a)}" for a in range(kind.rank)]
+            else:
+                params.append(f"{ctype(kind if kind != I64 else PY_INT)} {user(name)}")
         total = self.peak
         scratch = total > LDS_LIMIT  # tiles beyond one CU's LDS live in a per-block slice of global scratch
         if scratch:
@@ -468,8 +481,8 @@ class Emitter:
         """The linear index of a tile element in its tensor, and whether it lies inside."""
         axes = iter(idx)
         cells = [st if sl.squeeze else f"({st} + {next(axes)})" for st, sl in zip(starts, slices)]
-        inside = " && ".join(f"{c} >= 0 && {c} < {tensor}_n{a}" for a, c in enumerate(cells))
-        linear = " + ".join(c + "".join(f" * {tensor}_n{b}" for b in range(a + 1, len(cells)))
+        inside = " && ".join(f"{c} >= 0 && {c} < {dim(tensor, a)}" for a, c in enumerate(cells))
+        linear = " + ".join(c + "".join(f" * {dim(tensor, b)}" for b in range(a + 1, len(cells)))
                             for a, c in enumerate(cells))
         return linear, inside
 
@@ -478,7 +491,7 @@ class Emitter:
         # a tile axis of extent 1 that the loop broadcasts is element 0 of its slice
         linear, inside = self.cells(self.node[id(e)], e.slices, tensor, idx)
         ok = self.line(BOOL, inside)
-        element = f"{tensor}[{linear}]"
+        element = f"{user(tensor)}[{linear}]"
         if e.dtype == BF16:
             element = f"kb16_load({element})"
         self.reads.append((("tensor", tensor), "any"))
@@ -613,7 +626,7 @@ class Emitter:
             else:
                 x, ok = self.value(s.value, idx)
             element = f"kb16_word({x})" if s.tensor.type.dtype == BF16 else x
-            self.put(f"if ({'' if ok == '1' else f'({ok}) && '}{inside}) {tensor}[{linear}] = {element};")
+            self.put(f"if ({'' if ok == '1' else f'({ok}) && '}{inside}) {user(tensor)}[{linear}] = {element};")
             self.writes.append((("tensor", tensor), "any"))
 
         self.elements(s.value.shape, store)
@@ -660,10 +673,10 @@ class Emitter:
             row_axis, k_axis = (kept[1], kept[0]) if transposed != turned else (kept[0], kept[1])
 
             def condition(i: str) -> str:
-                checks = [f"{st} >= 0 && {st} < {tensor}_n{a}" for a, (st, sl) in enumerate(zip(starts, load.slices))
+                checks = [f"{st} >= 0 && {st} < {dim(tensor, a)}" for a, (st, sl) in enumerate(zip(starts, load.slices))
                           if sl.squeeze]
-                checks.append(f"{starts[k_axis]} < {tensor}_n{k_axis} && {starts[k_axis]} + {k} > 0")
-                checks.append(f"{starts[row_axis]} + {i} >= 0 && {starts[row_axis]} + {i} < {tensor}_n{row_axis}")
+                checks.append(f"{starts[k_axis]} < {dim(tensor, k_axis)} && {starts[k_axis]} + {k} > 0")
+                checks.append(f"{starts[row_axis]} + {i} >= 0 && {starts[row_axis]} + {i} < {dim(tensor, row_axis)}")
                 return " && ".join(checks)
 
             return ("load", condition)
@@ -801,7 +814,7 @@ class Emitter:
     def stmt_For(self, s: ir.For) -> None:
         if self.pipelined_product(s):
             return
-        var = s.var.name
+        var = user(s.var.name)
         if self.pending:
             self.barrier()  # the body's first accesses are checked against its own last ones only
         self.put(f"for (long long {var} = {self.scalar(s.lo)}; {var} < {self.scalar(s.hi)}; {var} += {s.step}) {{")
@@ -826,10 +839,10 @@ class Emitter:
         loads = (lhs, rhs.operand if turned else rhs)
         if not all(isinstance(e, ir.TileLoad) and len(e.shape) == 2 for e in loads):
             return False
-        (m, k), n, var = lhs.shape, rhs.shape[1], s.var.name
+        (m, k), n, var = lhs.shape, rhs.shape[1], user(s.var.name)
         axes = [[a for a, sl in enumerate(e.slices) if not sl.squeeze] for e in loads]
         k_axes = [axes[0][1], axes[1][1] if turned else axes[1][0]]
-        if any(self.mentions(sl.start, var) for e, ka in zip(loads, k_axes) for a, sl in enumerate(e.slices) if a != ka):
+        if any(self.mentions(sl.start, s.var.name) for e, ka in zip(loads, k_axes) for a, sl in enumerate(e.slices) if a != ka):
             return False
         form, integer = mfma_form(product), product.acc.dtype == I32
         acc, valid = self.tile_vars[product.acc.name]
@@ -934,7 +947,7 @@ class Emitter:
         self.put("}")
         for e, ka in zip(loads, k_axes):
             start = self.scalar(e.slices[ka].start)
-            self.put(f"_kok &= ({start}) < {e.tensor.name}_n{ka} && ({start}) + {k} > 0;")
+            self.put(f"_kok &= ({start}) < {dim(e.tensor.name, ka)} && ({start}) + {k} > 0;")
         if form is not None:
             per, vec = form.k_step // 4, form.operand_vec
             self.put(f"{blocks} _Pragma(\"unroll\") for (int _k = 0; _k < {k}; _k += {form.k_step}) {{")
@@ -1010,7 +1023,7 @@ class Emitter:
         self.put("}")
 
     def stmt_Assign(self, s: ir.Assign) -> None:
-        self.put(f"const {ctype(s.var.dtype)} {s.var.name} = {self.scalar(s.value)};")
+        self.put(f"const {ctype(s.var.dtype)} {user(s.var.name)} = {self.scalar(s.value)};")
 
     def scalar(self, e: ir.Expr) -> str:
         match e:
@@ -1021,9 +1034,9 @@ class Emitter:
                     return f"(({ctype(e.dtype)}){float(v)!r})"
                 return f"(({ctype(e.dtype)}){int(v)}LL)"
             case ir.Var(name=n) | ir.Param(name=n):
-                return n
+                return user(n)
             case ir.Dim(tensor=t, axis=a):
-                return f"{t.name}_n{a}"
+                return dim(t.name, a)
             case ir.BlockIndex(axis=a):
                 return f"b{a}"
             case ir.Cast(operand=o):

@@ -191,10 +191,12 @@ class Emitter:
     d = 32: 321 KiB, in global scratch, before; 16 heads of 512 took 1270 us).
 
     Loops over the same elements need no barrier between them when each reads only what its own thread wrote: `sync`
-    keeps what has been read and written since the last barrier and puts one only before a conflict."""
+    keeps what has been read and written since the last barrier and puts one only before a conflict. Tensors are told
+    apart by their parameters' names, unless `overlapping`: then any two of them may share memory, and a statement's
+    loads are complete before it, or a later one, stores."""
 
-    def __init__(self, kernel: ir.Kernel, entry: str) -> None:
-        self.kernel, self.entry = kernel, entry
+    def __init__(self, kernel: ir.Kernel, entry: str, overlapping: bool = False) -> None:
+        self.kernel, self.entry, self.overlapping = kernel, entry, overlapping
         self.threads = threads(kernel)
         self.mfma_products = 0
         self.lines: list[str] = []
@@ -240,10 +242,9 @@ class Emitter:
         _, start, nbytes = self.names[name]
         (self.writes if write else self.reads).append((("lds", start, start + nbytes), pattern))
 
-    @staticmethod
-    def conflict(a: Access, b: Access) -> bool:
+    def conflict(self, a: Access, b: Access) -> bool:
         (ra, pa), (rb, pb) = a, b
-        if ra[0] != rb[0] or (ra[0] == "tensor" and ra[1] != rb[1]):
+        if ra[0] != rb[0] or (ra[0] == "tensor" and ra[1] != rb[1] and not self.overlapping):
             return False
         if ra[0] == "lds" and (ra[2] <= rb[1] or rb[2] <= ra[1]):
             return False
@@ -305,7 +306,8 @@ class Emitter:
         params = []
         for name, kind in self.kernel.params:
             if isinstance(kind, ir.TensorType):
-                params.append(f"{storage(kind.dtype)}* __restrict__ {user(name)}")
+                alone = "" if self.overlapping else "__restrict__ "
+                params.append(f"{storage(kind.dtype)}* {alone}{user(name)}")
                 params += [f"long long {dim(name, a)}" for a in range(kind.rank)]
             else:
                 params.append(f"{ctype(kind if kind != I64 else PY_INT)} {user(name)}")
@@ -616,8 +618,9 @@ class Emitter:
         tensor, starts = s.tensor.name, [self.fresh("s") for _ in s.slices]
         for name, sl in zip(starts, s.slices):
             self.put(f"const long long {name} = {self.scalar(sl.start)};")
-        # a value loaded from the tensor it is stored to is complete before any of it is stored
-        temporary = self.materialise(s.value) if self.loads(s.value, tensor) else None
+        # a value loaded from the memory it is stored to is complete before any of it is stored
+        shared = None if self.overlapping else tensor
+        temporary = self.materialise(s.value) if self.loads(s.value, shared) else None
 
         def store(idx):
             linear, inside = self.cells(starts, s.slices, tensor, idx)
@@ -1065,7 +1068,8 @@ class Emitter:
         return f"kb16({text})" if dtype == BF16 else f"({ctype(dtype)})({text})"
 
 
-def emit(kernel: ir.Kernel, entry: str) -> tuple[str, int]:
+def emit(kernel: ir.Kernel, entry: str, overlapping: bool = False) -> tuple[str, int]:
     """HIP source of `kernel` with the entry point `entry`, and the global scratch bytes each block needs (0 when
-    its tiles fit in LDS; otherwise the kernel takes a trailing `_scratch` pointer to blocks x that many bytes)."""
-    return Emitter(kernel, entry).emit()
+    its tiles fit in LDS; otherwise the kernel takes a trailing `_scratch` pointer to blocks x that many bytes).
+    `overlapping`: for launches in which a tensor the program stores to shares memory with another one."""
+    return Emitter(kernel, entry, overlapping).emit()

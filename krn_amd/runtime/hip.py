@@ -12,6 +12,7 @@ import asyncio
 import ctypes
 import hashlib
 import inspect
+import math
 import os
 import threading
 import time
@@ -20,7 +21,7 @@ from collections import deque
 from collections.abc import Callable, Sequence
 from ctypes import c_float, c_int, c_int64, c_void_p
 from dataclasses import is_dataclass
-from functools import lru_cache
+from functools import cached_property, lru_cache
 from pathlib import Path
 
 import numpy as np
@@ -282,9 +283,9 @@ _programs: dict[str, Program] = {}
 _programs_lock = threading.Lock()
 
 
-def generic_program(kernel: ir.Kernel) -> Program:
+def generic_program(kernel: ir.Kernel, overlapping: bool = False) -> Program:
     entry = f"krn_{kernel.name}"
-    source, scratch = hipgen.emit(kernel, entry)
+    source, scratch = hipgen.emit(kernel, entry, overlapping)
     digest = hashlib.sha256(source.encode()).hexdigest()
     with _programs_lock:
         if digest not in _programs:
@@ -297,7 +298,8 @@ class Launch:
 
     def __init__(self, kernel: ir.Kernel, plan) -> None:
         self.kernel, self.plan = kernel, plan
-        self._program: Program | None = None  # the generic lowering's, once a launch has needed it
+        # the generic lowering's, once a launch has needed them: for tensors apart, and for overlapping ones
+        self._generic_programs: dict[bool, Program] = {}
 
     def prepare(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The launch of these argument values on this grid as one call per stream: the plan's checks and argument
@@ -418,11 +420,23 @@ class Launch:
         return lambda stream: library.softmax_rows(plan.dtype, x.pointer, y.pointer, rows, width, cols, cols,
                                                    stream.handle)
 
+    @cached_property
+    def _stored(self) -> frozenset[str]:
+        return frozenset(s.tensor.name for s in ir.walk(self.kernel.body) if isinstance(s, ir.TileStore))
+
+    def _overlapping(self, values: list[object]) -> bool:
+        """Whether a tensor this program stores to shares memory with another of its tensors (an in-place call)."""
+        spans = [(name in self._stored, v.pointer, v.pointer + v.numpy.itemsize * math.prod(v.shape))
+                 for (name, _), v in zip(self.kernel.params, values) if isinstance(v, HIPTensor)]
+        return any((a_stored or b_stored) and max(a, b) < min(a_end, b_end)
+                   for i, (a_stored, a, a_end) in enumerate(spans) for b_stored, b, b_end in spans[:i])
+
     def _generic(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The hiprtc program of this kernel, compiled (or found) once, with its kernelParams table built once."""
-        program = self._program
+        overlapping = self._overlapping(values)
+        program = self._generic_programs.get(overlapping)
         if program is None:  # writing the source to look the program up takes 0.8 ms
-            program = self._program = generic_program(self.kernel)
+            program = self._generic_programs[overlapping] = generic_program(self.kernel, overlapping)
         params: list = []
         for (name, kind), value in zip(self.kernel.params, values):
             if isinstance(kind, ir.TensorType):

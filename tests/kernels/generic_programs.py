@@ -57,3 +57,26 @@ def product_scaled(t: Extent, a: Matrix[T.f32], b: Matrix[T.f32], c: Matrix[T.f3
         acc *= 0.5
         acc += (a[rows, k : k + 8] * 2.0) @ b[k : k + 8, cols]
     c[rows, cols] = acc
+
+
+@kernel
+def centred(t: Extent, x: Matrix[T.f32], y: Matrix[T.f32]) -> None:
+    """Every element of a row reads the row's first one."""
+    rows, cols = block.tile(t.rows, t.cols)
+    y[rows, 0 : t.cols] = x[rows, 0 : t.cols] - x[rows, 0:1]
+
+
+@kernel
+def moved(t: Extent, x: Matrix[T.f32], y: Matrix[T.f32]) -> None:
+    """A load of one statement, stored one column to the left by the next."""
+    rows, cols = block.tile(t.rows, t.cols)
+    tile = x[rows, 1 : t.cols + 1]
+    y[rows, 0 : t.cols] = tile
+
+
+@kernel
+def mirrored(t: Extent, x: Matrix[T.f32], y: Matrix[T.f32]) -> None:
+    """Two stores, the second of what the first statement's tensor held before."""
+    tile = x[0 : t.rows, 0 : t.rows]
+    y[0 : t.rows, 0 : t.rows] = tile.transpose() + x[0 : t.rows, 0:1]
+    y[0 : t.rows, 0:1] = y[0 : t.rows, 1:2] + x[0 : t.rows, 2:3]

@@ -428,7 +428,7 @@ class Emitter:
     def value(self, e: ir.Expr, idx: list[str]) -> tuple[str, str]:
         """The element of `e` at `idx` (its value and its validity), computed in the current loop."""
         if not e.shape:
-            return self.scalar(e), "1"
+            return f"(({ctype(e.dtype)}){self.scalar(e)})", "1"  # of its own type: C adds narrow integers as int
         idx = self.aligned(idx, e.shape)
         key = (id(e), *idx)
         if key not in self.memo:

@@ -1,6 +1,6 @@
 """Tile programs for the generic lowering alone: none is a product, softmax or attention that has a kernel of its own."""
 
-from krn_amd import Const, Matrix, T, block, kernel, struct, zeros
+from krn_amd import Const, Matrix, T, block, kernel, struct, where, zeros
 
 
 @struct
@@ -80,3 +80,9 @@ def mirrored(t: Extent, x: Matrix[T.f32], y: Matrix[T.f32]) -> None:
     tile = x[0 : t.rows, 0 : t.rows]
     y[0 : t.rows, 0 : t.rows] = tile.transpose() + x[0 : t.rows, 0:1]
     y[0 : t.rows, 0:1] = y[0 : t.rows, 1:2] + x[0 : t.rows, 2:3]
+
+
+@kernel
+def below(t: Extent, x: Matrix[T.i8], y: Matrix[T.i8], n: T.i8) -> None:
+    """A scalar sum of a type narrower than C's int: 100 + 100 is -56."""
+    y[0 : t.rows, 0 : t.cols] = where(x[0 : t.rows, 0 : t.cols] < n + n, T.i8(1), T.i8(0))

@@ -97,11 +97,11 @@ __device__ __forceinline__ void store_chunk(uint8_t* row, int64_t c, int64_t wid
     }
 }
 
-// (m, s) and (m2, s2) merged: both sums rescaled to the larger maximum
+// (m, s) and (m2, s2) merged: both sums rescaled to the larger maximum. Without one yet, a sum is 0, or NaN if a NaN was
+// read, which must reach both partners: exp(-inf - 0) = 0 keeps both.
 __device__ __forceinline__ void combine(float& m, float& s, float m2, float s2) {
-  const float m_new = fmaxf(m, m2);
-  if (m_new != -INFINITY)
-    s = s * __builtin_amdgcn_exp2f((m - m_new) * LOG2E) + s2 * __builtin_amdgcn_exp2f((m2 - m_new) * LOG2E);
+  const float m_new = fmaxf(m, m2), top = m_new == -INFINITY ? 0.0f : m_new;
+  s = s * __builtin_amdgcn_exp2f((m - top) * LOG2E) + s2 * __builtin_amdgcn_exp2f((m2 - top) * LOG2E);
   m = m_new;
 }
 

@@ -53,14 +53,18 @@ int krn_gemm_nt(int in_kind, const void* a, const void* b, void* c, int out_kind
  * operand is read as it lies or, where the transposed copy pays, transposed into it. krn_gemm_workspace gives the
  * bytes the call uses; with fewer, or none, another kernel runs (only a K x N operand with N < 8, K < 8 or 2 GiB and
  * more needs them, else an error). The workspace needs no preparation, is 16-byte aligned, and must not be touched by
- * other work until this call's work on `stream` has run; calls on one stream may share one. No counterpart in the
- * reference: its products need no caller memory. */
+ * other work until this call's work on `stream` has run; calls on one stream may share one. C may share memory with A
+ * or B if the workspace holds krn_gemm_workspace_in_place(m, n) bytes: C is then written after both have been read
+ * (K * element size of at least 16 bytes). No counterpart in the reference: its products need no caller memory. */
 int krn_gemm(int b_kn, int in_kind, const void* a, const void* b, void* c, int out_kind, int64_t m, int64_t n,
              int64_t k, int nops, const int* ops, const float* scalars, const void* const* vectors, void* workspace,
              int64_t workspace_bytes, void* stream);
 
 /* Bytes of workspace this krn_gemm call uses (a and b matter by their alignment; nothing is dereferenced). */
 int64_t krn_gemm_workspace(int b_kn, int in_kind, const void* a, const void* b, int64_t m, int64_t n, int64_t k);
+
+/* Bytes of workspace with which a krn_gemm call may write C over A or B. */
+int64_t krn_gemm_workspace_in_place(int64_t m, int64_t n);
 
 /* C[m, n] = epilogue(sum_k A[m, k] * B[k, n]), A: M x K, B: K x N (the NN form), C: M x N, bf16 or f16 operands;
  * out_kind and the epilogue as for krn_gemm_nt. Replaces krn's own GEMM tile program `acc += a[rows, ks] @

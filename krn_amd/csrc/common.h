@@ -37,6 +37,12 @@ __device__ __forceinline__ uint16_t f2h(float f) { return __builtin_bit_cast(uin
 
 __device__ __forceinline__ float h2f(uint16_t h) { return (float)__builtin_bit_cast(_Float16, h); }
 
+// Whether two ranges of memory have a byte in common (an output that is also an operand)
+inline bool share_memory(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+  const uintptr_t x = (uintptr_t)a, y = (uintptr_t)b;
+  return a_bytes > 0 && b_bytes > 0 && x < y + (uint64_t)b_bytes && y < x + (uint64_t)a_bytes;
+}
+
 // A buffer resource over `bytes` bytes from `base` (raw 32-bit offsets, no stride, no swizzle; at most 2^31 - 1).
 // Loads past the end return zeros instead of touching memory: that is how the whole-tile GEMMs read the ragged
 // last rows of an operand.

@@ -1162,18 +1162,22 @@ static double split_cost(int shape, bool nn, int64_t m, int64_t n, int64_t slice
 // included, K in whole 128-byte slices, 16-byte aligned rows) and those with at most 128 rows keep their kernels; what
 // is left is a choice between tiles by estimated time: the eight- and four-wave loops on 128 x 256 and 128 x 128
 // tiles (NT, whole slices), and the split kernels on smaller tiles, over K, or with unaligned rows. `workspace` bounds
-// the planes of K parts.
+// the planes of K parts. `in_place`: C shares memory with A or B. The parts then write to planes whatever the shape, and C
+// is written once all of them have read; without a workspace for two planes, no tile is smaller than 128 x 128 (a
+// product of one such tile column reads its rows before it writes them).
 static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, int64_t n, int64_t k, int64_t elem,
-                    int64_t workspace) {
+                    int64_t workspace, bool in_place = false) {
   const int64_t kbytes = k * elem, slices = (kbytes + 127) / 128;
   const bool aligned = kbytes % 16 == 0 && (uintptr_t)a % 16 == 0 && (uintptr_t)b % 16 == 0 && (!nn || n % 8 == 0);
   const int64_t t256 = ((m + 255) / 256) * ((n + 255) / 256), t128 = ((m + 127) / 128) * ((n + 127) / 128);
   const bool piped = !nn && aligned && kbytes % 128 == 0 && kbytes > 0 && m > 0 && n > 0;
-  if (nn && nn_direct(a, b, m, n, k)) return {NN_WHOLE, 0, 1, 0};
-  if (piped && t256 >= 128 && m > 128 && 256 * kbytes <= 0x7fffffff) return {WHOLE, 0, 1, 0};
   // the split kernels' 128-row panels (NN: all of B) are addressed by 31-bit offsets, rows hold a whole 16-byte load
   const bool split = kbytes >= 16 && m > 0 && n > 0 && 128 * kbytes <= 0x7fffffff &&
                      (!nn || (n >= 8 && kbytes / 2 * n * 2 <= 0x7fffffff));
+  if (in_place && split && 2 * split_plane(m, n) <= workspace)
+    return {SPLIT, aligned ? RING_128x128 : ANY_128x128, 2, 2 * split_plane(m, n)};
+  if (nn && nn_direct(a, b, m, n, k)) return {NN_WHOLE, 0, 1, 0};
+  if (piped && t256 >= 128 && m > 128 && 256 * kbytes <= 0x7fffffff) return {WHOLE, 0, 1, 0};
   Plan best{TILE, 0, 1, 0};
   double least = 1e30;
   if (piped && m <= 128) {
@@ -1207,7 +1211,7 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
   for (int shape = aligned ? RING_32x64 : ANY_32x128; shape <= (aligned ? RING_128x128_DEEP : ANY_128x128); ++shape)
     for (int parts = 1; parts <= 16 && (parts == 1 || slices / parts >= 8); ++parts) {
       const int64_t need = parts > 1 ? parts * split_plane(m, n) : 0;
-      if (need > workspace) break;
+      if (need > workspace || (in_place && shape != RING_128x128 && shape != RING_128x128_DEEP && shape != ANY_128x128)) break;
       const double us = split_cost(shape, nn, m, n, slices, parts);
       if (us < least) best = {SPLIT, shape, parts, need}, least = us;
     }
@@ -1256,7 +1260,9 @@ static int gemm_dispatch(int fmt, bool nn, const void* a, const void* b, void* c
                          int64_t elem, const Epilogue& e, void* workspace, int64_t workspace_bytes,
                          hipStream_t stream) {
   if (m == 0 || n == 0) return 0;
-  const Plan p = plan_of(fmt, nn, a, b, m, n, k, elem, workspace ? workspace_bytes : 0);
+  const int64_t c_bytes = m * n * (e.out_kind == F32 || e.out_kind == I32 ? 4 : 2);
+  const bool in_place = share_memory(c, c_bytes, a, m * k * elem) || share_memory(c, c_bytes, b, n * k * elem);
+  const Plan p = plan_of(fmt, nn, a, b, m, n, k, elem, workspace ? workspace_bytes : 0, in_place);
   const SplitCall g{a, b, c, m, n, k * elem, k * elem, nn ? n * 2 : k * elem, e, workspace, stream};
   if (p.route == NN_WHOLE) {
     const dim3 tiles((unsigned)(((m + 255) / 256) * (n / 256)));
@@ -1379,6 +1385,8 @@ int64_t krn_gemm_workspace(int b_kn, int in_kind, const void* a, const void* b, 
   if (m <= 0 || n <= 0 || k <= 0) return 0;
   return plan_of(fmt, b_kn != 0, a, b, m, n, k, fmt == FMT_BF16 || fmt == FMT_F16 ? 2 : 1, INT64_MAX).workspace;
 }
+
+int64_t krn_gemm_workspace_in_place(int64_t m, int64_t n) { return m <= 0 || n <= 0 ? 0 : 2 * split_plane(m, n); }
 
 }  // extern "C"
 

@@ -363,6 +363,10 @@ class Launch:
                 code = base + (1 if op.axis == "row" else 2) + library.VECTOR_KINDS[vector.dtype]
                 ops.append((code, 0.0, vector.pointer))
         need = library.gemm_workspace(plan.layout, plan.operand, a.pointer, b.pointer, m, n, k)
+        size, end = D.NUMPY[plan.operand].itemsize, c.pointer + D.NUMPY[plan.output].itemsize * m * n
+        if (c.pointer < a.pointer + size * m * k and a.pointer < end) or (
+                c.pointer < b.pointer + size * n * k and b.pointer < end):
+            need = max(need, library.gemm_workspace_in_place(m, n))
         if need == 0 and plan.layout == "nt":
             direct = library.gemm_nt_call(plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k, ops)
             return lambda stream: direct(stream.handle)

@@ -43,6 +43,8 @@ def lib() -> ctypes.CDLL:
     ]  # fmt: skip
     handle.krn_gemm_workspace.restype = c_int64
     handle.krn_gemm_workspace.argtypes = [c_int, c_int, c_void_p, c_void_p, c_int64, c_int64, c_int64]
+    handle.krn_gemm_workspace_in_place.restype = c_int64
+    handle.krn_gemm_workspace_in_place.argtypes = [c_int64, c_int64]
     handle.krn_attention_fwd.restype = c_int
     handle.krn_attention_fwd.argtypes = [
         c_int, c_void_p, c_void_p, c_void_p, c_void_p, c_int64, c_int64, c_int64, c_int64, c_float, c_int, c_void_p,
@@ -92,6 +94,11 @@ def kind(dtype: Dtype) -> int:
 def gemm_workspace(layout: str, in_dtype: Dtype, a: int, b: int, m: int, n: int, k: int) -> int:
     """Bytes of device workspace `gemm_call` of these arguments uses (`layout` "nt" or "nn")."""
     return lib().krn_gemm_workspace(int(layout == "nn"), kind(in_dtype), a, b, m, n, k)
+
+
+def gemm_workspace_in_place(m: int, n: int) -> int:
+    """Bytes of device workspace with which `gemm_call` may write its result over an operand."""
+    return lib().krn_gemm_workspace_in_place(m, n)
 
 
 def gemm_call(layout: str, in_dtype: Dtype, a: int, b: int, c: int, out_dtype: Dtype, m: int, n: int, k: int,

@@ -462,7 +462,14 @@ extern "C" int krn_attention_fwd_ws(int kind, const void* q, const void* k, cons
   if (bh == 0 || sq == 0) return 0;
   hipStream_t s = (hipStream_t)stream;
   const bool bf = kind == BF16;
-  const int parts = attention_parts(bh, sq, sk, d, causal != 0, workspace ? workspace_bytes : 0);
+  int parts = attention_parts(bh, sq, sk, d, causal != 0, workspace ? workspace_bytes : 0);
+  // an output in the keys' or values' memory: 32-row workgroups that share a head would store over what others still
+  // read (with several parts the reduction stores, after all have read); 256 rows of a head are one workgroup above
+  const int64_t q_bytes = bh * sq * d * 2, k_bytes = bh * sk * d * 2;
+  if (parts == 1 && sq > 32 &&
+      (share_memory(o, q_bytes, k, k_bytes) || share_memory(o, q_bytes, v, k_bytes) ||
+       (o != q && share_memory(o, q_bytes, q, q_bytes))))
+    parts = 0;
   if (parts > 0) {
     const AttentionCall c{q, k, v, o, workspace, bh, sq, sk, scale, causal != 0, parts, s};
     return launch_attention_split(bf, (int)d, c);

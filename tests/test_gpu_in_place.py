@@ -1,6 +1,8 @@
-"""Calls whose result is written over an operand: a product over A or B. The result is the one of separate tensors:
-products of small integers are exact in every order."""
+"""Calls whose result is written over an operand: a product over A or B, attention over its keys or values. The result is
+the one of separate tensors: products of small integers are exact in every order, attention is held to a float64
+softmax with the tolerance of the other attention tests (f16 3e-3)."""
 
+import math
 from types import SimpleNamespace
 
 import numpy as np
@@ -15,6 +17,7 @@ from krn_amd.runtime import hip, library
 from oracle.numerics import bf16_values, bf16_words
 from tests.conftest import KERNELS
 from tests.kernels import tile_programs as programs
+from tests.test_gpu_attention_split import reference
 
 
 @pytest.mark.gpu
@@ -42,6 +45,23 @@ def test_a_linear_layer_over_its_input(device, m, n):
     x = device.to_device(bf16_words(a), T.bf16)
     programs.gemm_nt[programs.Tiling(bm=64, bn=64, bk=32)](x, device.to_device(bf16_words(b), T.bf16), x)
     np.testing.assert_array_equal(bf16_values(x.to_host()), a @ b.T)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("over", ["q", "k", "v"])
+@pytest.mark.parametrize("bh,s", [(16, 200), (4, 256), (64, 33), (3, 31), (40, 100)])
+def test_attention_over_its_inputs(device, over, bh, s, d):
+    rng = np.random.default_rng(s + d)
+    words = {name: rng.standard_normal((bh, s, d)).astype(np.float16) for name in "qkv"}
+    scale = math.log2(math.e) / math.sqrt(d)
+    want = reference(*(w.astype(np.float64) for w in words.values()), scale, False)
+    tensors = {name: device.to_device(w) for name, w in words.items()}
+    need = library.attention_workspace(bh, s, s, d, False)
+    scratch = device.empty(T.u8, max(need, 1))
+    library.attention_call(F16, *(t.pointer for t in tensors.values()), tensors[over].pointer, bh, s, s, d, scale, False,
+                           need)(scratch.pointer if need else 0, device.default_stream.handle)
+    np.testing.assert_allclose(tensors[over].to_host().astype(np.float64), want, atol=3e-3)
 
 
 @pytest.mark.parametrize("c,in_place", [(1 << 20, True), ((1 << 20) + 2 * 512 * 128 - 2, True), (1 << 21, True),

@@ -1147,16 +1147,25 @@ static bool nn_direct(const void* a, const void* b, int64_t m, int64_t n, int64_
 // 26 us (two); 128 x 128 tiles, operands from HBM: two workgroups per CU 56.8 us at 256 x 4096 x 14336 in eight parts,
 // one with four stages 51.3 in four, 78 at 512 x 8192 x 8192 (the four-wave loop 95);
 // unaligned 1024 x 4096 x 4097 60 us on 128 x 128.
+static const struct { int bm, bn; double slice, more, more_nn; } SPLIT_TILES[] = {
+    {32, 64, 0.23, 0.15, 0.17},   {64, 64, 0.28, 0.22, 0.25},   {128, 128, 0.80, 0.60, 0.52}, {128, 128, 0.62, 0.62, 0.82},
+    {32, 128, 0.70, 0.75, 0.75},  {64, 64, 0.43, 0.35, 0.38},   {128, 128, 0.92, 0.92, 0.95}};
+static int64_t split_tiles(int shape, int64_t m, int64_t n) {
+  const auto& t = SPLIT_TILES[shape];
+  return ((m + t.bm - 1) / t.bm) * ((n + t.bn - 1) / t.bn);
+}
 static double split_cost(int shape, bool nn, int64_t m, int64_t n, int64_t slices, int parts) {
-  static const struct { int bm, bn; double slice, more, more_nn; } T[] = {
-      {32, 64, 0.23, 0.15, 0.17},   {64, 64, 0.28, 0.22, 0.25},   {128, 128, 0.80, 0.60, 0.52}, {128, 128, 0.62, 0.62, 0.82},
-      {32, 128, 0.70, 0.75, 0.75},  {64, 64, 0.43, 0.35, 0.38},   {128, 128, 0.92, 0.92, 0.95}};
-  const int64_t wgs = ((m + T[shape].bm - 1) / T[shape].bm) * ((n + T[shape].bn - 1) / T[shape].bn) * parts;
+  const auto& t = SPLIT_TILES[shape];
+  const int64_t wgs = split_tiles(shape, m, n) * parts;
   const double per_cu = (double)((wgs + 255) / 256);
-  double us = (double)((slices + parts - 1) / parts) * fmax(T[shape].slice, (nn ? T[shape].more_nn : T[shape].more) * per_cu);
+  double us = (double)((slices + parts - 1) / parts) * fmax(t.slice, (nn ? t.more_nn : t.more) * per_cu);
   if (parts > 1) us += 8.0 + (double)parts * (double)split_plane(m, n) / 5e6;  // the second launch reads the planes
   return us;
 }
+
+// Workgroups of a launch: of 256 threads, and a launch's threads along an axis stay below 2^32 (a launch past that runs
+// nothing: 2^30 rows of 64 x 64 tiles left C unwritten)
+constexpr int64_t MOST_TILES = ((int64_t)1 << 24) - 1;
 
 // Kernel choice on 256 CUs. Products that fill the chip with 256 x 256 tiles (at least 128 of them, ragged edges
 // included, K in whole 128-byte slices, 16-byte aligned rows) and those with at most 128 rows keep their kernels; what
@@ -1211,7 +1220,8 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
   for (int shape = aligned ? RING_32x64 : ANY_32x128; shape <= (aligned ? RING_128x128_DEEP : ANY_128x128); ++shape)
     for (int parts = 1; parts <= 16 && (parts == 1 || slices / parts >= 8); ++parts) {
       const int64_t need = parts > 1 ? parts * split_plane(m, n) : 0;
-      if (need > workspace || (in_place && shape != RING_128x128 && shape != RING_128x128_DEEP && shape != ANY_128x128)) break;
+      if (need > workspace || split_tiles(shape, m, n) > MOST_TILES) break;
+      if (in_place && shape != RING_128x128 && shape != RING_128x128_DEEP && shape != ANY_128x128) break;
       const double us = split_cost(shape, nn, m, n, slices, parts);
       if (us < least) best = {SPLIT, shape, parts, need}, least = us;
     }
@@ -1262,6 +1272,22 @@ static int gemm_dispatch(int fmt, bool nn, const void* a, const void* b, void* c
   if (m == 0 || n == 0) return 0;
   const int64_t c_bytes = m * n * (e.out_kind == F32 || e.out_kind == I32 ? 4 : 2);
   const bool in_place = share_memory(c, c_bytes, a, m * k * elem) || share_memory(c, c_bytes, b, n * k * elem);
+  // more rows than a launch of 128-row tiles holds (M of 2^31 and more): in runs of 2^30
+  constexpr int64_t RUN = (int64_t)1 << 30;
+  if (!in_place && m > RUN && (m + 127) / 128 * ((n + 127) / 128) > MOST_TILES) {
+    for (int64_t r0 = 0; r0 < m; r0 += RUN) {
+      Epilogue run = e;  // row vectors start at the run's first row
+      for (int i = 0; i < e.nops; ++i) {
+        const int op = e.op[i] & ((1 << VEC_KIND_SHIFT) - 1), kind = e.op[i] >> VEC_KIND_SHIFT;
+        if (op == MUL_ROW || op == ADD_ROW) run.vec[i] = static_cast<const uint8_t*>(e.vec[i]) + r0 * (kind == 0 ? 4 : 2);
+      }
+      const int rc = gemm_dispatch(fmt, nn, static_cast<const uint8_t*>(a) + r0 * k * elem, b,
+                                   static_cast<uint8_t*>(c) + c_bytes / m * r0, m - r0 < RUN ? m - r0 : RUN, n, k, elem,
+                                   run, workspace, workspace_bytes, stream);
+      if (rc != 0) return rc;
+    }
+    return 0;
+  }
   const Plan p = plan_of(fmt, nn, a, b, m, n, k, elem, workspace ? workspace_bytes : 0, in_place);
   const SplitCall g{a, b, c, m, n, k * elem, k * elem, nn ? n * 2 : k * elem, e, workspace, stream};
   if (p.route == NN_WHOLE) {

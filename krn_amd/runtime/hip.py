@@ -244,6 +244,12 @@ class HIPTensor(Tensor):
             self.pointer = 0
 
 
+def share_memory(x: object, y: object) -> bool:
+    """Whether two arguments are tensors with a byte of memory in common."""
+    return isinstance(x, HIPTensor) and isinstance(y, HIPTensor) and max(x.pointer, y.pointer) < min(
+        x.pointer + x.numpy.itemsize * math.prod(x.shape), y.pointer + y.numpy.itemsize * math.prod(y.shape))
+
+
 def _kind(argument: object) -> object:
     """What compiling depends on in one argument."""
     if isinstance(argument, HIPTensor):
@@ -363,9 +369,7 @@ class Launch:
                 code = base + (1 if op.axis == "row" else 2) + library.VECTOR_KINDS[vector.dtype]
                 ops.append((code, 0.0, vector.pointer))
         need = library.gemm_workspace(plan.layout, plan.operand, a.pointer, b.pointer, m, n, k)
-        size, end = D.NUMPY[plan.operand].itemsize, c.pointer + D.NUMPY[plan.output].itemsize * m * n
-        if (c.pointer < a.pointer + size * m * k and a.pointer < end) or (
-                c.pointer < b.pointer + size * n * k and b.pointer < end):
+        if share_memory(c, a) or share_memory(c, b):
             need = max(need, library.gemm_workspace_in_place(m, n))
         if need == 0 and plan.layout == "nt":
             direct = library.gemm_nt_call(plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k, ops)
@@ -430,10 +434,9 @@ class Launch:
 
     def _overlapping(self, values: list[object]) -> bool:
         """Whether a tensor this program stores to shares memory with another of its tensors (an in-place call)."""
-        spans = [(name in self._stored, v.pointer, v.pointer + v.numpy.itemsize * math.prod(v.shape))
-                 for (name, _), v in zip(self.kernel.params, values) if isinstance(v, HIPTensor)]
-        return any((a_stored or b_stored) and max(a, b) < min(a_end, b_end)
-                   for i, (a_stored, a, a_end) in enumerate(spans) for b_stored, b, b_end in spans[:i])
+        tensors = [(name in self._stored, v) for (name, _), v in zip(self.kernel.params, values)]
+        return any((x_stored or y_stored) and share_memory(x, y)
+                   for i, (x_stored, x) in enumerate(tensors) for y_stored, y in tensors[:i])
 
     def _generic(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The hiprtc program of this kernel, compiled (or found) once, with its kernelParams table built once."""

@@ -3,7 +3,6 @@ the one of separate tensors: products of small integers are exact in every order
 softmax with the tolerance of the other attention tests (f16 3e-3)."""
 
 import math
-from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -77,6 +76,6 @@ def test_a_launch_over_an_operand_asks_for_the_planes(monkeypatch, c, in_place):
     kernel = capture(KERNELS, "gemm_nt", consts={"t": {"bm": 64, "bn": 64, "bk": 32}})
     plan = cdna4.lower(kernel)
     tensor = {"a": ((512, 128), 1 << 20), "b": ((128, 128), 1 << 21), "c": ((512, 128), c)}
-    params = {name: SimpleNamespace(shape=shape, pointer=pointer, dtype=BF16) for name, (shape, pointer) in tensor.items()}
+    params = {name: hip.HIPTensor(None, pointer, BF16, shape, owner=object()) for name, (shape, pointer) in tensor.items()}
     assert hip.Launch(kernel, plan)._gemm(plan, params, Blocks(2, 8)) is not None
     assert asked == [2 * 512 * 128 * 4 if in_place else 0]

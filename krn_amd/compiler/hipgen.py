@@ -140,15 +140,18 @@ def mfma_form(s: ir.Accumulate) -> MfmaForm | None:
     return None
 
 
-def threads(kernel: ir.Kernel) -> int:
+MANY_BLOCKS = 1 << 22  # along x, of 1024 threads: 2^32
+
+
+def threads(kernel: ir.Kernel, blocks: int = 1) -> int:
     """Threads of one block: 256, and 1024 for programs whose tiles have 4096 elements and more and whose products, if
     any, run on the matrix cores. Their LDS leaves room for one or two blocks on a CU, and 256 threads would be one
     wave per SIMD with nothing to cover its LDS latency (flash attention, 64 x 64 tiles, d = 32, 16 x 512:
     100 us with 256 threads, 51 with 1024). A scalar product keeps 256: fewer outputs per thread are more LDS reads per
-    multiply-add."""
+    multiply-add. A launch's threads along an axis stay below 2^32, so MANY_BLOCKS take 256 as well."""
     large = max((math.prod(v.shape) for v in kernel.tiles), default=1) >= 4096
     scalar = any(isinstance(s, ir.Accumulate) and mfma_form(s) is None for s in ir.walk(kernel.body))
-    return 1024 if large and not scalar else 256
+    return 1024 if large and not scalar and blocks < MANY_BLOCKS else 256
 
 
 def products(kernel: ir.Kernel) -> list[str]:
@@ -195,9 +198,9 @@ class Emitter:
     apart by their parameters' names, unless `overlapping`: then any two of them may share memory, and a statement's
     loads are complete before it, or a later one, stores."""
 
-    def __init__(self, kernel: ir.Kernel, entry: str, overlapping: bool = False) -> None:
+    def __init__(self, kernel: ir.Kernel, entry: str, overlapping: bool = False, blocks: int = 1) -> None:
         self.kernel, self.entry, self.overlapping = kernel, entry, overlapping
-        self.threads = threads(kernel)
+        self.threads = threads(kernel, blocks)
         self.mfma_products = 0
         self.lines: list[str] = []
         self.depth = 1
@@ -1068,8 +1071,9 @@ class Emitter:
         return f"kb16({text})" if dtype == BF16 else f"({ctype(dtype)})({text})"
 
 
-def emit(kernel: ir.Kernel, entry: str, overlapping: bool = False) -> tuple[str, int]:
+def emit(kernel: ir.Kernel, entry: str, overlapping: bool = False, blocks: int = 1) -> tuple[str, int]:
     """HIP source of `kernel` with the entry point `entry`, and the global scratch bytes each block needs (0 when
     its tiles fit in LDS; otherwise the kernel takes a trailing `_scratch` pointer to blocks x that many bytes).
-    `overlapping`: for launches in which a tensor the program stores to shares memory with another one."""
-    return Emitter(kernel, entry, overlapping).emit()
+    `overlapping`: for launches in which a tensor the program stores to shares memory with another one; `blocks`: of
+    the launch's x axis, which only the threads of a block depend on."""
+    return Emitter(kernel, entry, overlapping, blocks).emit()

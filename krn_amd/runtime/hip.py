@@ -289,13 +289,13 @@ _programs: dict[str, Program] = {}
 _programs_lock = threading.Lock()
 
 
-def generic_program(kernel: ir.Kernel, overlapping: bool = False) -> Program:
+def generic_program(kernel: ir.Kernel, overlapping: bool = False, blocks: int = 1) -> Program:
     entry = f"krn_{kernel.name}"
-    source, scratch = hipgen.emit(kernel, entry, overlapping)
+    source, scratch = hipgen.emit(kernel, entry, overlapping, blocks)
     digest = hashlib.sha256(source.encode()).hexdigest()
     with _programs_lock:
         if digest not in _programs:
-            _programs[digest] = Program(source, entry, hipgen.threads(kernel), scratch)
+            _programs[digest] = Program(source, entry, hipgen.threads(kernel, blocks), scratch)
         return _programs[digest]
 
 
@@ -304,8 +304,8 @@ class Launch:
 
     def __init__(self, kernel: ir.Kernel, plan) -> None:
         self.kernel, self.plan = kernel, plan
-        # the generic lowering's, once a launch has needed them: for tensors apart, and for overlapping ones
-        self._generic_programs: dict[bool, Program] = {}
+        # the generic lowering's, once a launch has needed them: for many blocks or not, with tensors that overlap or not
+        self._generic_programs: dict[tuple[bool, bool], Program] = {}
 
     def prepare(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The launch of these argument values on this grid as one call per stream: the plan's checks and argument
@@ -441,9 +441,10 @@ class Launch:
     def _generic(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The hiprtc program of this kernel, compiled (or found) once, with its kernelParams table built once."""
         overlapping = self._overlapping(values)
-        program = self._generic_programs.get(overlapping)
+        form = (grid.x >= hipgen.MANY_BLOCKS, overlapping)
+        program = self._generic_programs.get(form)
         if program is None:  # writing the source to look the program up takes 0.8 ms
-            program = self._generic_programs[overlapping] = generic_program(self.kernel, overlapping)
+            program = self._generic_programs[form] = generic_program(self.kernel, overlapping, grid.x)
         params: list = []
         for (name, kind), value in zip(self.kernel.params, values):
             if isinstance(kind, ir.TensorType):

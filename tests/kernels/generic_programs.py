@@ -75,6 +75,13 @@ def moved(t: Extent, x: Matrix[T.f32], y: Matrix[T.f32]) -> None:
 
 
 @kernel
+def doubled(t: Extent, x: Matrix[T.f32], y: Matrix[T.f32]) -> None:
+    rows = block.tile(t.rows)
+    tile = x[rows, 0 : t.cols] * 2.0
+    y[rows, 0 : t.cols] = tile
+
+
+@kernel
 def mirrored(t: Extent, x: Matrix[T.f32], y: Matrix[T.f32]) -> None:
     """Two stores, the second of what the first statement's tensor held before."""
     tile = x[0 : t.rows, 0 : t.rows]

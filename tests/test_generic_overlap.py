@@ -49,7 +49,7 @@ def tensor(pointer, shape, dtype=F32):
 def test_the_launch_tells_overlapping_tensors_by_their_addresses(monkeypatch, x, y, shared):
     asked = []
 
-    def generic_program(kernel, overlapping=False):
+    def generic_program(kernel, overlapping=False, blocks=1):
         asked.append(overlapping)
         return SimpleNamespace(scratch=0, threads=256)
 

@@ -131,11 +131,11 @@ class HIPStream(Stream):
         self.workspace_lock = threading.Lock()  # held while a call that uses the workspace puts its kernels on the stream
 
     def workspace(self, nbytes: int) -> "HIPTensor":
-        """At least `nbytes` of device scratch for one launch on this stream. Launches on a stream run in order, so they
-        share one buffer, which grows to the largest request and is freed with the stream; a launch holds it until
-        it has completed, so a buffer outgrown meanwhile (by another thread, too) is freed after its last use. A
-        request above WORKSPACE_KEPT is that launch's own and goes back after it. A launch that a graph records gets
-        memory of its own, which the graph keeps: its replays run on any stream."""
+        """At least `nbytes` of device scratch for one launch on this stream, which the caller drops once the launch is
+        enqueued: it is stream ordered, so its free waits for the work queued before. Launches on a stream run in
+        order, so they share one buffer, which grows to the largest request; a request above WORKSPACE_KEPT is that
+        launch's own. A launch that a graph records gets memory of its own, which is not stream ordered and which
+        the graph keeps: its replays run on any stream."""
         if self.capturing or nbytes > WORKSPACE_KEPT:
             return self.device.empty_on(self, D.U8, nbytes)
         held = self._workspace
@@ -382,15 +382,16 @@ class Launch:
         return self._with_workspace(product, need)
 
     def _with_workspace(self, call: Callable[[int, int], None], nbytes: int) -> Callable[[HIPStream], None]:
-        """`call(workspace, stream)` with the stream's workspace, held until the launch has completed. The call puts
-        two kernels on the stream, the second reading what the first left in the workspace, and runs without the
-        interpreter's lock: another thread's call must not put its own between them."""
+        """`call(workspace, stream)` with the stream's workspace. The call puts two kernels on the stream, the second
+        reading what the first left in the workspace, and runs without the interpreter's lock: another thread's call
+        must not put its own between them."""
 
         def run(stream: HIPStream) -> None:
             with stream.workspace_lock:
                 workspace = stream.workspace(nbytes)
                 call(workspace.pointer, stream.handle)
-                stream.note(self.kernel.name, (workspace,))
+                recorded = workspace is not stream._workspace and stream.capturing
+                stream.note(self.kernel.name, (workspace,) if recorded else ())
 
         return run
 

@@ -121,10 +121,14 @@ class HIPStream(Stream):
     """An in-order queue of device work. A launch's arguments are held until a marker event recorded after it has
     completed (the `Keeper` of reference runtime/completion.py:99-131): `record()` closes the open launches under its
     event and releases every older marker that is done, and after KEEP_LIMIT unmarked launches the stream records a
-    marker itself, so a loop that never synchronizes holds a bounded number of them."""
+    marker itself, so a loop that never synchronizes holds a bounded number of them.
 
-    def __init__(self, device: "HIPDevice", handle: int) -> None:
-        self.device, self.handle = device, handle
+    A stream that its program drops frees its workspace (stream ordered) and leaves its handle, with what it still
+    holds, to `retire`: the handle is used again by a later stream, so nothing that keeps it (a tensor allocated on
+    it, a buffer of StreamScratch) ever has a destroyed one."""
+
+    def __init__(self, device: "HIPDevice", handle: int, retire: Callable[[int, tuple], None] | None = None) -> None:
+        self.device, self.handle, self._retire = device, handle, retire
         self._open: list[tuple[str, tuple[object, ...]]] = []
         self._marks: deque[tuple[HIPEvent, list[tuple[str, tuple[object, ...]]]]] = deque()
         self._workspace: HIPTensor | None = None
@@ -188,6 +192,29 @@ class HIPStream(Stream):
         self._open = []
         self._marks.clear()
 
+    def __del__(self) -> None:
+        if self._retire is not None:
+            self._retire(self.handle, (self._open, self._marks) if self._open or self._marks else ())
+
+
+class Retired:
+    """A dropped stream whose launches may not have completed: its handle, and the arguments they hold."""
+
+    def __init__(self, device: "HIPDevice", handle: int, held: tuple) -> None:
+        self.device, self.handle, self.held = device, handle, held
+        self._event: HIPEvent | None = None
+        self._recorded = hipapi.capturing(handle)  # into a graph, which reads the arguments at every replay
+
+    def done(self) -> bool:
+        """Whether its work has completed, by an event recorded after it when this is first asked."""
+        if self._recorded:
+            return False
+        if self._event is None:
+            event = HIPEvent(self.device, hipapi.event_create())
+            hipapi.api().hipEventRecord(c_void_p(event.handle), c_void_p(self.handle))
+            self._event = event
+        return self._event.done()
+
 
 class HIPTensor(Tensor):
     """C-contiguous device memory with its element type (bf16 as uint16 words, fp8 as uint8 codes) and shape.
@@ -204,7 +231,10 @@ class HIPTensor(Tensor):
         self.device, self.pointer, self.dtype, self.shape = device, pointer, dtype, tuple(int(s) for s in shape)
         self.numpy = D.NUMPY[dtype]
         self._owner = owner  # a view keeps the owner alive; an owner frees its memory
-        self._stream = stream  # the allocating stream (stream-ordered memory), or None for a plain allocation
+        # the allocating stream's handle (stream-ordered memory), or None for a plain allocation; the stream itself may
+        # hold this tensor (its workspace, a launch's argument)
+        self._stream = stream.handle if stream is not None else None
+
     @property
     def nbytes(self) -> int:
         return self.numpy.itemsize * int(np.prod(self.shape))
@@ -236,7 +266,7 @@ class HIPTensor(Tensor):
         if self._owner is None and self.pointer:
             try:
                 if self._stream is not None:
-                    hipapi.free_async(self.pointer, self._stream.handle)
+                    hipapi.free_async(self.pointer, self._stream)
                 else:
                     hipapi.free(self.pointer)
             except Exception:
@@ -644,22 +674,21 @@ class HIPGraph(Graph):
 
     def __init__(self, device: "HIPDevice", fn: Callable, args: tuple, kwargs: dict) -> None:
         self.device, self._fn, self._recorded = device, fn, (args, kwargs)
-        self._executable: int | None = None
-        self._keep: list[tuple[object, ...]] = []
+        self._recording: Recording | None = None
         if os.environ.get("KRN_GRAPHS", "1") != "0":
-            self._executable = self._capture(*args, **kwargs)
+            self._recording = self._capture(*args, **kwargs)
 
     def __call__(self, *args, **kwargs) -> None:
         recorded_args, recorded_kwargs = self._recorded
         same = (len(args) == len(recorded_args) and all(a is b for a, b in zip(args, recorded_args))
                 and kwargs.keys() == recorded_kwargs.keys()
                 and all(kwargs[name] is recorded_kwargs[name] for name in kwargs))
-        if self._executable is not None and same:
+        if self._recording is not None and same:
             stream = self.device.launch_stream()
-            hipapi.api().hipGraphLaunch(c_void_p(self._executable), c_void_p(stream.handle))
-            stream.note("graph", (self,))
+            hipapi.api().hipGraphLaunch(c_void_p(self._recording.executable), c_void_p(stream.handle))
+            stream.note("graph", (self._recording,))
             return
-        if self._executable is not None:
+        if self._recording is not None:
             raise TargetError("graph replay", self.device.arch,
                               "hipGraph nodes keep their recorded arguments; krn does not patch node parameters",
                               "record a new graph for these arguments or set KRN_GRAPHS=0")
@@ -669,7 +698,7 @@ class HIPGraph(Graph):
         self(*args, **kwargs)
         return self.device.launch_stream().record()
 
-    def _capture(self, *args, **kwargs) -> int:
+    def _capture(self, *args, **kwargs) -> "Recording":
         stream = self.device.capture_stream()
         handle = c_void_p(stream.handle)
         hipapi.api().hipStreamBeginCapture(handle, hipapi.CAPTURE_RELAXED)
@@ -689,10 +718,16 @@ class HIPGraph(Graph):
         except BaseException:
             hipapi.api().raw("hipGraphDestroy", graph)
             raise
-        # what the recorded launches hold (scratch tensors, arguments) now lives with the graph
-        self._keep = stream.take()
-        weakref.finalize(self, _release_graph, executable.value, graph.value)
-        return executable.value
+        return Recording(executable.value, graph.value, stream.take())
+
+
+class Recording:
+    """An instantiated graph with what its recorded launches hold (scratch tensors, arguments). Replays that may still
+    run hold it, and not the function that was recorded."""
+
+    def __init__(self, executable: int, graph: int, held: list[tuple[object, ...]]) -> None:
+        self.executable, self.held = executable, held
+        weakref.finalize(self, _release_graph, executable, graph)
 
 
 def _release_graph(executable: int, graph: int) -> None:
@@ -714,7 +749,10 @@ class HIPDevice(Device):
         library.lib()  # the kernel library must be present: there is no fallback path
         hipapi.keep_pool(ordinal)
         self._default = HIPStream(self, hipapi.stream_create())
-        self._streams: list[HIPStream] = [self._default]
+        self._streams: weakref.WeakSet[HIPStream] = weakref.WeakSet([self._default])
+        self._streams_lock = threading.Lock()
+        self._idle: deque[int] = deque()  # handles of dropped streams, their work done as far as launches hold arguments
+        self._retired: deque[Retired] = deque()  # dropped streams whose launches may still run
 
     @property
     def default_stream(self) -> HIPStream:
@@ -725,9 +763,38 @@ class HIPDevice(Device):
         return stream if isinstance(stream, HIPStream) else self._default
 
     def stream(self) -> HIPStream:
-        created = HIPStream(self, hipapi.stream_create())
-        self._streams.append(created)
+        for _ in range(len(self._retired)):
+            try:
+                retired = self._retired.popleft()
+            except IndexError:  # another thread's
+                break
+            done = False
+            try:
+                done = retired.done()
+            finally:
+                if done:
+                    self._idle.append(retired.handle)
+                else:
+                    self._retired.append(retired)
+        try:
+            handle = self._idle.popleft()
+            if hipapi.capturing(handle):  # dropped by a function that a graph is recording
+                self._idle.append(handle)
+                handle = hipapi.stream_create()
+        except IndexError:
+            handle = hipapi.stream_create()
+        created = HIPStream(self, handle, self._retire)
+        with self._streams_lock:
+            self._streams.add(created)
         return created
+
+    def _retire(self, handle: int, held: tuple) -> None:
+        """The handle of a dropped stream, and what its unfinished launches hold. Called when it is collected, in
+        whichever thread that happens, so it takes no lock."""
+        if held:
+            self._retired.append(Retired(self, handle, held))
+        else:
+            self._idle.append(handle)
 
     def capture_stream(self) -> HIPStream:
         """The stream graphs are recorded on (one per device, reused)."""
@@ -765,8 +832,23 @@ class HIPDevice(Device):
         return HIPGraph(self, fn, args, kwargs)
 
     def sync(self) -> None:
-        for stream in self._streams:
+        with self._streams_lock:
+            streams = list(self._streams)
+        for stream in streams:
             stream.sync()
+        for handle in list(self._idle):
+            hipapi.api().hipStreamSynchronize(c_void_p(handle))
+        while self._retired:
+            try:
+                retired = self._retired.popleft()
+            except IndexError:  # another thread's
+                break
+            try:
+                hipapi.api().hipStreamSynchronize(c_void_p(retired.handle))
+            except BaseException:
+                self._retired.append(retired)
+                raise
+            self._idle.append(retired.handle)
 
     async def synchronize(self) -> None:
         await asyncio.get_running_loop().run_in_executor(None, self.sync)

@@ -274,10 +274,17 @@ class HIPTensor(Tensor):
             self.pointer = 0
 
 
+def span(argument: object) -> tuple[int, int]:
+    """The first and the end address of a tensor's memory; empty for an argument that is none."""
+    if not isinstance(argument, HIPTensor):
+        return 0, 0
+    return argument.pointer, argument.pointer + argument.numpy.itemsize * math.prod(argument.shape)
+
+
 def share_memory(x: object, y: object) -> bool:
     """Whether two arguments are tensors with a byte of memory in common."""
-    return isinstance(x, HIPTensor) and isinstance(y, HIPTensor) and max(x.pointer, y.pointer) < min(
-        x.pointer + x.numpy.itemsize * math.prod(x.shape), y.pointer + y.numpy.itemsize * math.prod(y.shape))
+    (x, x_end), (y, y_end) = span(x), span(y)
+    return x < y_end and y < x_end and x < x_end and y < y_end
 
 
 def _kind(argument: object) -> object:
@@ -465,9 +472,13 @@ class Launch:
 
     def _overlapping(self, values: list[object]) -> bool:
         """Whether a tensor this program stores to shares memory with another of its tensors (an in-place call)."""
-        tensors = [(name in self._stored, v) for (name, _), v in zip(self.kernel.params, values)]
-        return any((x_stored or y_stored) and share_memory(x, y)
-                   for i, (x_stored, x) in enumerate(tensors) for y_stored, y in tensors[:i])
+        spans = [span(v) for v in values]
+        for (name, _), (x, x_end) in zip(self.kernel.params, spans):
+            if name in self._stored:
+                meeting = sum(1 for y, y_end in spans if x < y_end and y < x_end and y < y_end)
+                if meeting > 1:  # itself, and another
+                    return True
+        return False
 
     def _generic(self, values: list[object], grid: Blocks) -> Callable[[HIPStream], None]:
         """The hiprtc program of this kernel, compiled (or found) once, with its kernelParams table built once."""

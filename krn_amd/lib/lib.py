@@ -10,7 +10,6 @@ call falls to the next one.
 """
 
 import os
-import sys
 from abc import ABC, abstractmethod
 from dataclasses import dataclass
 from enum import Enum
@@ -117,6 +116,7 @@ class Host(Candidate):
 
 PREFERENCE: dict[Op, tuple[str, ...]] = {Op.MATMUL: ("hipblaslt", "ours", "host")}
 MODULES = {"hipblaslt": "krn_amd.lib.lib_hipblaslt", "ours": "krn_amd.lib.lib_ours"}
+_candidates: dict[str, Candidate] = {}
 
 
 def candidate(name: str) -> Candidate:
@@ -125,8 +125,9 @@ def candidate(name: str) -> Candidate:
         return Host()
     if name not in MODULES:
         raise KeyError(f"unknown matmul candidate {name!r}; known: {', '.join(PREFERENCE[Op.MATMUL])}")
-    module = sys.modules.get(MODULES[name]) or import_module(MODULES[name])  # import_module alone is 5 us a call
-    return module.CANDIDATE
+    if name not in _candidates:  # import_module, which waits for another thread's import of the module, is 5 us a call
+        _candidates[name] = import_module(MODULES[name]).CANDIDATE
+    return _candidates[name]
 
 
 def order(library: str | None = None) -> tuple[str, ...]:

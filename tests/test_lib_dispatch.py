@@ -126,3 +126,29 @@ def test_hipblaslt_plans_are_keyed_on_operand_alignment(monkeypatch):
     session.plan(p, lib.Operands(t(0x40000), t(0x50002), t(0x60000), None))
     assert len(made) == 2
     assert lt.alignments(lib.Operands(t(0x50002), t(0x50040), t(0x1000), None)) == (2, 64, 256, 0)
+
+
+def test_threads_that_make_the_first_call_together_wait_for_the_module(tmp_path, monkeypatch):
+    """A module that another thread is still importing has no CANDIDATE yet; the call waits for the import."""
+    import threading
+
+    (tmp_path / "slow_candidate.py").write_text("import time\ntime.sleep(0.3)\nCANDIDATE = object()\n")
+    monkeypatch.syspath_prepend(str(tmp_path))
+    monkeypatch.setitem(lib.MODULES, "slow", "slow_candidate")
+    found, failed, start = [], [], threading.Barrier(4)
+
+    def call(delay):
+        start.wait()
+        threading.Event().wait(delay)
+        try:
+            found.append(lib.candidate("slow"))
+        except AttributeError as error:
+            failed.append(error)
+
+    threads = [threading.Thread(target=call, args=(0.05 * i,)) for i in range(4)]
+    for thread in threads:
+        thread.start()
+    for thread in threads:
+        thread.join()
+    assert not failed and len(found) == 4 and len(set(map(id, found))) == 1
+    assert lib.candidate("slow") is found[0]

@@ -1117,10 +1117,8 @@ static int launch_band(const void* a, const void* b, void* c, int64_t m, int64_t
                        int64_t ldb, int64_t ldc, const Epilogue& e, hipStream_t stream) {
   if constexpr (FMT == FMT_BF16 || FMT == FMT_F16)
     return launch_pipe<FMT, 128, 256, 2, 4, 4, 64>(a, b, c, m, n, kbytes, lda, ldb, ldc, e, stream);
-  else if constexpr (FMT == FMT_I8)
-    return launch_pipe<FMT, 128, 256, 2, 4, 3, 128>(a, b, c, m, n, kbytes, lda, ldb, ldc, e, stream);
   else
-    return launch_gemm<FMT, 128, 128, 2, 2>(a, b, c, m, n, kbytes, lda, ldb, ldc, e, stream);
+    return launch_pipe<FMT, 128, 256, 2, 4, 3, 128>(a, b, c, m, n, kbytes, lda, ldb, ldc, e, stream);
 }
 
 // How a product runs: the kernel family, for RING and ANY the tile and loader, the K parts, and the workspace bytes.
@@ -1139,6 +1137,24 @@ static bool nn_direct(const void* a, const void* b, int64_t m, int64_t n, int64_
   return m > 0 && n > 0 && n % 256 == 0 && k % 64 == 0 && k >= 128 && t256 >= 128 && t256 <= 0x7fffffff &&
          (uintptr_t)a % 16 == 0 &&
          (uintptr_t)b % 16 == 0 && 256 * k * 2 <= 0x7fffffff && (k - 1) * n * 2 + 512 <= 0x7fffffff;
+}
+
+// The products of nn_direct
+static int launch_nn_whole(bool bf, const void* a, const void* b, void* c, int64_t m, int64_t n, int64_t k,
+                           const Epilogue& e, hipStream_t stream) {
+  const dim3 tiles((unsigned)(((m + 255) / 256) * (n / 256)));
+  if (bf)
+    hipLaunchKernelGGL((gemm_quad16<FMT_BF16, true>), tiles, dim3(256), 0, stream, (const uint8_t*)a, (const uint8_t*)b, c,
+                       m, n, k * 2, k * 2, n * 2, n, e);
+  else
+    hipLaunchKernelGGL((gemm_quad16<FMT_F16, true>), tiles, dim3(256), 0, stream, (const uint8_t*)a, (const uint8_t*)b, c,
+                       m, n, k * 2, k * 2, n * 2, n, e);
+  hipError_t err = hipGetLastError();
+  if (err != hipSuccess) {
+    krn_set_error("gemm_nn launch: %s", hipGetErrorString(err));
+    return (int)err;
+  }
+  return 0;
 }
 
 // Estimated microseconds of a split-kernel launch beyond its fixed cost, from sweeps of each tile over 10 to 1500
@@ -1234,7 +1250,10 @@ static int launch_planned(const Plan& p, bool nn, const SplitCall& g) {
     case SKINNY: return launch_skinny<FMT>(g, p.parts);
     case SPLIT: return launch_split(FMT, nn, p.shape, p.parts, g);
     case MID: return launch_mid<FMT>(g.a, g.b, g.c, g.m, g.n, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
-    case BAND: return launch_band<FMT>(g.a, g.b, g.c, g.m, g.n, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
+    case BAND:  // never fp8
+      if constexpr (FMT != FMT_FP8)
+        return launch_band<FMT>(g.a, g.b, g.c, g.m, g.n, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
+      break;
     case WHOLE: break;
     default:
       return launch_gemm<FMT, 128, 128, 2, 2>(g.a, g.b, g.c, g.m, g.n, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
@@ -1245,23 +1264,24 @@ static int launch_planned(const Plan& p, bool nn, const SplitCall& g) {
   // half the work each), which fills the last wave. The two launches write disjoint columns of C.
   const int64_t t256 = ((g.m + 255) / 256) * ((g.n + 255) / 256);
   const int64_t full_tiles = (t256 / 256) * 256, tile_rows = (g.m + 255) / 256;
-  const bool columns = FMT != FMT_FP8 && t256 % 256 != 0 && t256 % 256 <= 128 && full_tiles > 0 &&
-                       full_tiles % tile_rows == 0;
-  if (!columns)
-    return launch_whole<FMT>(g.a, g.b, g.c, g.m, g.n, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
-  const int64_t n_split = full_tiles / tile_rows * 256;
-  Epilogue tail = g.e;  // the epilogue of the columns from n_split on: column vectors start at that column
-  for (int i = 0; i < g.e.nops; ++i) {
-    const int op = g.e.op[i] & ((1 << VEC_KIND_SHIFT) - 1), kind = g.e.op[i] >> VEC_KIND_SHIFT;
-    if (op == MUL_COL || op == ADD_COL)
-      tail.vec[i] = static_cast<const uint8_t*>(g.e.vec[i]) + n_split * (kind == 0 ? 4 : 2);
+  if constexpr (FMT != FMT_FP8) {
+    if (t256 % 256 != 0 && t256 % 256 <= 128 && full_tiles > 0 && full_tiles % tile_rows == 0) {
+      const int64_t n_split = full_tiles / tile_rows * 256;
+      Epilogue tail = g.e;  // the epilogue of the columns from n_split on: column vectors start at that column
+      for (int i = 0; i < g.e.nops; ++i) {
+        const int op = g.e.op[i] & ((1 << VEC_KIND_SHIFT) - 1), kind = g.e.op[i] >> VEC_KIND_SHIFT;
+        if (op == MUL_COL || op == ADD_COL)
+          tail.vec[i] = static_cast<const uint8_t*>(g.e.vec[i]) + n_split * (kind == 0 ? 4 : 2);
+      }
+      const int out_bytes = (g.e.out_kind == F32 || g.e.out_kind == I32) ? 4 : 2;
+      const int rc = launch_whole<FMT>(g.a, g.b, g.c, g.m, n_split, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
+      if (rc != 0) return rc;
+      return launch_band<FMT>(g.a, static_cast<const uint8_t*>(g.b) + n_split * g.ldb,
+                              static_cast<uint8_t*>(g.c) + n_split * out_bytes, g.m, g.n - n_split, g.kbytes, g.lda,
+                              g.ldb, g.n, tail, g.stream);
+    }
   }
-  const int out_bytes = (g.e.out_kind == F32 || g.e.out_kind == I32) ? 4 : 2;
-  const int rc = launch_whole<FMT>(g.a, g.b, g.c, g.m, n_split, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
-  if (rc != 0) return rc;
-  return launch_band<FMT>(g.a, static_cast<const uint8_t*>(g.b) + n_split * g.ldb,
-                          static_cast<uint8_t*>(g.c) + n_split * out_bytes, g.m, g.n - n_split, g.kbytes, g.lda, g.ldb,
-                          g.n, tail, g.stream);
+  return launch_whole<FMT>(g.a, g.b, g.c, g.m, g.n, g.kbytes, g.lda, g.ldb, g.n, g.e, g.stream);
 }
 
 extern "C" int krn_transpose16(const void* in, void* out, int64_t rows, int64_t cols, void* stream);
@@ -1290,21 +1310,7 @@ static int gemm_dispatch(int fmt, bool nn, const void* a, const void* b, void* c
   }
   const Plan p = plan_of(fmt, nn, a, b, m, n, k, elem, workspace ? workspace_bytes : 0, in_place);
   const SplitCall g{a, b, c, m, n, k * elem, k * elem, nn ? n * 2 : k * elem, e, workspace, stream};
-  if (p.route == NN_WHOLE) {
-    const dim3 tiles((unsigned)(((m + 255) / 256) * (n / 256)));
-    if (fmt == FMT_BF16)
-      hipLaunchKernelGGL((gemm_quad16<FMT_BF16, true>), tiles, dim3(256), 0, stream, (const uint8_t*)a,
-                         (const uint8_t*)b, c, m, n, k * 2, k * 2, n * 2, n, e);
-    else
-      hipLaunchKernelGGL((gemm_quad16<FMT_F16, true>), tiles, dim3(256), 0, stream, (const uint8_t*)a,
-                         (const uint8_t*)b, c, m, n, k * 2, k * 2, n * 2, n, e);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) {
-      krn_set_error("gemm_nn launch: %s", hipGetErrorString(err));
-      return (int)err;
-    }
-    return 0;
-  }
+  if (p.route == NN_WHOLE) return launch_nn_whole(fmt == FMT_BF16, a, b, c, m, n, k, e, stream);
   if (nn && p.route != SPLIT) {
     if (n * k * 2 > (workspace ? workspace_bytes : 0) && k > 0) {
       krn_set_error("gemm: this product needs a workspace of %lld bytes for the transposed operand",
@@ -1454,19 +1460,7 @@ static int gemm_nn_through(int in_kind, const void* a, const void* b, void* c, i
       krn_set_error("gemm_nn: output kind %d is not stored by the tile GEMM", out_kind);
       return -1;
     }
-    const int64_t tiles = ((m + 255) / 256) * (n / 256);
-    if (in_kind == BF16)
-      hipLaunchKernelGGL((gemm_quad16<FMT_BF16, true>), dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream,
-                         (const uint8_t*)a, (const uint8_t*)b, c, m, n, k * 2, k * 2, n * 2, n, e);
-    else
-      hipLaunchKernelGGL((gemm_quad16<FMT_F16, true>), dim3((unsigned)tiles), dim3(256), 0, (hipStream_t)stream,
-                         (const uint8_t*)a, (const uint8_t*)b, c, m, n, k * 2, k * 2, n * 2, n, e);
-    hipError_t err = hipGetLastError();
-    if (err != hipSuccess) {
-      krn_set_error("gemm_nn launch: %s", hipGetErrorString(err));
-      return (int)err;
-    }
-    return 0;
+    return launch_nn_whole(in_kind == BF16, a, b, c, m, n, k, e, (hipStream_t)stream);
   }
   if (bt == nullptr && n > 0 && k > 0) {
     krn_set_error("gemm_nn: this product needs the transposed operand's workspace");

@@ -285,12 +285,12 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
   static_assert(LA * RPL * WAVES == BM, "whole loads");
   static_assert(NN ? LB * KPL * WAVES == KROWS : LB * RPL * WAVES == BN, "whole loads");
   constexpr int SB = (BM + BN) * BKB;
-  constexpr bool PIPE = !NN && PIPED, AGPRS = STAGES * SB > 80 * 1024;
-  static_assert(!PIPE || STAGES == 4, "four stages");
-  static_assert(STAGES >= 2 && STAGES <= 5 && (STAGES - 2) * LOADS <= 63, "the loop's stages, vmcnt range");
+  constexpr bool PIPE = !NN && PIPED;
+  static_assert(STAGES == 4 || (STAGES == 2 && !PIPE), "the loops' stages");
+  static_assert((STAGES - 2) * LOADS <= 63, "vmcnt range");
   constexpr int LDS_BYTES = STAGES * SB > WAVES * TN * PATCH_WORDS * 4 ? STAGES * SB : WAVES * TN * PATCH_WORDS * 4;
   __shared__ __attribute__((aligned(1024))) uint8_t lds[LDS_BYTES];
-  uint8_t *const s0 = lds, *const s1 = lds + SB, *const s2 = lds + 2 * SB, *const s3 = lds + 3 * SB, *const s4 = lds + 4 * SB;
+  uint8_t *const s0 = lds, *const s1 = lds + SB, *const s2 = lds + 2 * SB, *const s3 = lds + 3 * SB;
   int tm, tn;
   const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN);
   const int part = part_tile_of(tiles_m, tiles_n, parts, tm, tn);
@@ -378,8 +378,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
 #pragma unroll
     for (int j = 0; j < TN; ++j) acc[i][j] = Acc{};
   if (n > 0) { if (tail) KRN_ISSUE_TAIL(s0); else KRN_ISSUE(s0, 0); }
-  if (STAGES > 2 && n > 1) KRN_ISSUE(s1, 1);
-  if (STAGES > 3 && n > 2) KRN_ISSUE(s2, 2);
+  if (STAGES == 4 && n > 1) KRN_ISSUE(s1, 1);
+  if (STAGES == 4 && n > 2) KRN_ISSUE(s2, 2);
   if constexpr (PIPE) {
     if (n > 3) KRN_ISSUE(s3, 3);
     u32x4 fa0[KS][TM][CH], fb0[KS][TN][CH], fa1[KS][TM][CH], fb1[KS][TN][CH];
@@ -425,8 +425,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
     KRN_HELD(0);
     for (int i = 0;; i += 4) {
       // one workgroup per CU: the accumulators are AGPRs, and stay there around the loop
-      if constexpr (AGPRS)
-        _Pragma("unroll") for (int a = 0; a < TM; ++a) _Pragma("unroll") for (int b = 0; b < TN; ++b) asm volatile("" : "+a"(acc[a][b]));
+      _Pragma("unroll") for (int a = 0; a < TM; ++a) _Pragma("unroll") for (int b = 0; b < TN; ++b) asm volatile("" : "+a"(acc[a][b]));
       KRN_TURN(0, s0, s1, 0, 1)
       KRN_TURN(1, s1, s2, 1, 0)
       KRN_TURN(2, s2, s3, 0, 1)
@@ -436,7 +435,6 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
 #undef KRN_HELD
 #undef KRN_TURN
   } else {
-  if (STAGES > 4 && n > 3) KRN_ISSUE(s3, 3);
 #define KRN_SLICE(d, st, prev)                                                                                         \
     if (i + d >= n) break;                                                                                             \
     if (i + d + STAGES - 2 < n) KRN_VMWAIT((STAGES - 2) * LOADS); else KRN_VMWAIT(0);                                  \
@@ -446,9 +444,7 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __re
     KRN_COMPUTE(st);
   for (int i = 0;; i += STAGES) {
     if constexpr (STAGES == 2) { KRN_SLICE(0, s0, s1) KRN_SLICE(1, s1, s0) }
-    if constexpr (STAGES == 3) { KRN_SLICE(0, s0, s2) KRN_SLICE(1, s1, s0) KRN_SLICE(2, s2, s1) }
     if constexpr (STAGES == 4) { KRN_SLICE(0, s0, s3) KRN_SLICE(1, s1, s0) KRN_SLICE(2, s2, s1) KRN_SLICE(3, s3, s2) }
-    if constexpr (STAGES == 5) { KRN_SLICE(0, s0, s4) KRN_SLICE(1, s1, s0) KRN_SLICE(2, s2, s1) KRN_SLICE(3, s3, s2) KRN_SLICE(4, s4, s3) }
   }
   }
 #undef KRN_ISSUE

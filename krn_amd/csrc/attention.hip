@@ -388,7 +388,10 @@ static void launch_attention(const void* q, const void* k, const void* v, void* 
 
 // How a launch runs: parts = 0 is the kernel above (256 query rows per workgroup), otherwise the key-split kernel with
 // that many workgroups per block of 32 query rows. Both times are estimated in microseconds from sweeps on 256 CUs and
-// the shorter taken. A workgroup above takes 1.8 us (d = 64: 1.35) per 64 keys, whatever its rows, and the launch 4
+// the shorter taken. They count the keys that a wave walks one after the other and not the stream of K and V, which is
+// what bounds launches of 128 MiB and more (128 heads x 1 x 16384 keys, d = 128: 111 estimated, 170 measured); the number
+// of parts is the best one there too (one, two, four, eight parts: 128 x 1 x 4096 68.8, 50.6, 54.1, 59.5 us; 128 x 1 x
+// 16384 236, 170, 176, 184; 32 x 1 x 8192 in two, four, eight, sixteen 67.3, 40.3, 31.9, 39.4). A workgroup above takes 1.8 us (d = 64: 1.35) per 64 keys, whatever its rows, and the launch 4
 // more; a wave of the key-split kernel 1.6 us per 32 keys (d = 64: 0.93 alone on its CU, 1.15 in twos), a workgroup
 // 2.6, a launch 3, the reduction of several parts 3 and the planes' bytes. Measured, both sides: 128 heads x 1 query x
 // 4096 keys, d = 128: 113 -> 52 us (two parts; 268 MB of K and V); 32 x 1 x 8192: 203 -> 29 (eight); 16 x 1000 x 1000,

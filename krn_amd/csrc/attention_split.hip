@@ -251,10 +251,12 @@ static int launch(const AttentionCall& c) {
 }
 
 // Up to 32 query rows a head are one row block, whose keys and values are read once. From 128 MiB of them, half of the
-// last-level cache, their loads are non-temporal, since little would be found there by a later launch anyway (d = 128,
-// one query, bf16: 128 heads x 4096 keys 57.4 -> 52.0 us, 4.7 -> 5.2 TB/s; 128 x 16384 190.9 -> 170.3; 32 x 8192, 128 MiB,
-// 34.7 -> 32.0). Smaller ones keep ordinary loads (8 heads x 16384 keys, 64 MiB: 24.3 us, non-temporally 27.8), and so do
-// longer prompts, whose row blocks share keys in L2 (16 x 1000 x 1000, d = 64: 11.9 us, non-temporally 13.2).
+// last-level cache, their loads are non-temporal, since little would be found there by a later launch anyway (one query,
+// heads x keys, d = 128: bf16 128 x 4096 57.4 -> 52.0 us, 4.7 -> 5.2 TB/s, 128 x 16384 190.9 -> 170.3, 32 x 8192, 128 MiB,
+// 34.7 -> 32.0; f16 128 x 4096 56.5 -> 50.8, 32 x 8192 35.0 -> 32.3; d = 64: bf16 128 x 4096, 128 MiB, 31.6 -> 30.1,
+// 64 x 16384 63.7 -> 56.7, f16 31.8 -> 29.8 and 64.4 -> 58.6; 32 queries f16 128 x 4096, d = 128, 58.2 -> 53.0). Smaller
+// ones keep ordinary loads (64 MiB: bf16 8 x 16384, d = 128, 24.3 us, non-temporally 27.8; f16 25.5 and 28.4; bf16
+// 16 x 16384, d = 64, 20.5 and 22.3), and so do longer prompts, whose row blocks share keys in L2 (16 x 1000 x 1000, d = 64: 11.9 us, non-temporally 13.2).
 int krn::launch_attention_split(bool bf, int d, const AttentionCall& c) {
   const bool once = c.sq <= 32 && c.bh * c.sk * d * 4 >= (int64_t)128 << 20;
 #define KRN_SPLIT(BFV, DV) (once ? launch<BFV, DV, true>(c) : launch<BFV, DV, false>(c))

@@ -1159,10 +1159,10 @@ static int launch_nn_whole(bool bf, const void* a, const void* b, void* c, int64
 
 // Estimated microseconds of a split-kernel launch beyond its fixed cost, from sweeps of each tile over 10 to 1500
 // workgroups (bf16 unless noted): a 128-byte K slice takes a CU `slice` us, with `more` us for every workgroup the
-// busiest CU holds once that is larger. 256 x 4096 x 4096 on 64 x 64 tiles 16.6 us (one workgroup per CU), 512 rows
-// 26 us (two); 128 x 128 tiles, operands from HBM: two workgroups per CU 56.8 us at 256 x 4096 x 14336 in eight parts,
-// one with four stages 51.3 in four, 78 at 512 x 8192 x 8192 (the four-wave loop 95);
-// unaligned 1024 x 4096 x 4097 60 us on 128 x 128.
+// busiest CU holds once that is larger. 256 x 4096 x 4096 on 64 x 64 tiles 16.5 us (one workgroup per CU), 512 rows
+// 27.5 us (two); 128 x 128 tiles, operands from HBM: two workgroups per CU 57.9 us at 256 x 4096 x 14336 in eight parts,
+// one with four stages 52.9 in four; 512 x 8192 x 8192 four stages 82-83, two stages 110; unaligned 1024 x 4096 x 4097
+// 60 us on 128 x 128.
 static const struct { int bm, bn; double slice, more, more_nn; } SPLIT_TILES[] = {
     {32, 64, 0.23, 0.15, 0.17},   {64, 64, 0.28, 0.22, 0.25},   {128, 128, 0.80, 0.60, 0.52}, {128, 128, 0.62, 0.62, 0.82},
     {32, 128, 0.70, 0.75, 0.75},  {64, 64, 0.43, 0.35, 0.38},   {128, 128, 0.92, 0.92, 0.95}};
@@ -1206,9 +1206,10 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
   Plan best{TILE, 0, 1, 0};
   double least = 1e30;
   if (piped && m <= 128) {
-    // One workgroup per 32 columns; with few columns K is split as well. A slice takes a workgroup 0.11 us with one
-    // block of 32 rows, 0.35 with four (1 x 4096 x 4096 bf16: 9.2 us on 128 workgroups; 16 x 1024 x 14336: 28.1 on 32);
-    // the second launch of a split costs 8, most of it on the host (3 x 768 x 4992 f16: 7.8 us, split 11.6).
+    // One workgroup per 32 columns; with few columns K is split as well. A slice takes a workgroup RATE, with one block
+    // of 32 rows to four, beyond the launch's fixed cost (1 x 4096 x 4096 bf16, 64 slices: 9.2 us on 128 workgroups;
+    // 16 x 1024 x 14336, 224 slices: 28.2 on 32, split 11.4); the second launch of a split costs 8, most of it on the
+    // host (3 x 768 x 4992 f16: 7.8 us, split 11.6).
     static const double RATE[] = {0.10, 0.14, 0.24, 0.35};
     const int64_t groups = (n + 31) / 32;
     const double whole_k = (double)slices * RATE[(m - 1) / 32] * (double)((groups + 255) / 256);
@@ -1223,6 +1224,7 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
     if (m <= 64 || elem == 1) return best;
     least -= 2.0;  // near ties stay (89 x 1536 x 2560 f16: 11.0 us, 32 x 64 tiles 11.7)
   } else if (piped && 128 * kbytes <= 0x7fffffff) {
+    // the four-wave loop: 0.66 us a slice from the caches, 0.74 from HBM (95 us at 512 x 8192 x 8192)
     if (t128 <= 256) best = {MID, 0, 1, 0}, least = 0.66 * (double)slices;
     else if (fmt != FMT_FP8 && 256 * kbytes <= 0x7fffffff)
       best = {BAND, 0, 1, 0},

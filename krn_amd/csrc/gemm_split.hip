@@ -270,8 +270,8 @@ __device__ __forceinline__ void tr_read(uint8_t* p, u32x4 (&f)[4]) {
 // the NN form are assembly for the same reason, each block of reads with its wait.
 // Two workgroups share a CU where the ring leaves room; the accumulators then live in VGPRs. Where it does not (PIPED:
 // one wave per SIMD, nothing else to run while a wave reads its fragments), a slice's fragments are read between the
-// MFMAs of the slice before it, whose stage is refilled at once (NT bf16 512 x 8192 x 8192: 85 -> 78 us, 384 x 6144 x
-// 5120: 48.8 -> 41.7). The NN form's transposed reads wait in their own block and keep the plain loop.
+// MFMAs of the slice before it, whose stage is refilled at once (NT bf16, the plain loop and this one on one box:
+// 512 x 8192 x 8192 85.7 -> 81.6 us, 384 x 6144 x 5120 49.8 -> 42.0). The NN form's transposed reads wait in their own block and keep the plain loop.
 template <int FMT, int BM, int BN, int WM, int WN, int STAGES, bool PIPED, bool NN>
 __global__ __launch_bounds__(WM * WN * 64, 2) void gemm_ring(const uint8_t* __restrict__ A, const uint8_t* __restrict__ B,
                                                      void* __restrict__ C, int64_t M, int64_t N, int64_t kbytes,

@@ -1,14 +1,14 @@
 """Generic lowering of any captured tile program to HIP C++ for gfx950, compiled at run time with hiprtc.
 
 This is the path for tile programs that are not one of the contraction shapes the hand-written MFMA kernels serve
-(`cdna4.lower` decides). One workgroup of 256 threads runs one block; tile variables live in LDS with a validity byte
-per lane; a tile statement is one loop over its elements, strided over the workgroup. Its arithmetic is
-the tile semantics of krn's C-family lowering (reference src/krn/compiler/emit.py): a product stages both operands
-as float32 (invalid lanes zero) and runs one fused multiply-add per k in k order for each output element
+(`cdna4.lower` decides). One workgroup of 256 or 1024 threads (`threads`) runs one block; tile variables live in LDS
+with a validity byte per lane; a tile statement is one loop over its elements, strided over the workgroup. Its
+arithmetic is the tile semantics of krn's C-family lowering (reference src/krn/compiler/emit.py): a product stages both
+operands as float32 (invalid lanes zero) and runs one fused multiply-add per k in k order for each output element
 (emit.py:788-796), a reduction takes the valid lanes of its axis from the first one (emit.py:997-1034; float32 sums in
-up to 64 interleaved parts), stores skip invalid lanes and elements outside the tensor. The kernel ABI is krn's generated-kernel ABI
-(reference src/krn/compiler/cuda.py:319 and ir.py:441-452): `extern "C" __global__`, a tensor is a pointer plus one
-`long long` extent per axis, scalars by value.
+up to 64 interleaved parts), stores skip invalid lanes and elements outside the tensor. The kernel ABI is krn's
+generated-kernel ABI (reference src/krn/compiler/cuda.py:319 and ir.py:441-452): `extern "C" __global__`, a tensor is a
+pointer plus one `long long` extent per axis, scalars by value.
 """
 
 import math
@@ -763,8 +763,8 @@ class Emitter:
 
     def mfma_product(self, s: ir.Accumulate, form: "MfmaForm") -> None:
         """acc[m, n] += lhs[m, k] @ rhs[k, n] on the matrix cores: both operands staged into LDS K-contiguous as the
-        instruction's operand type (invalid lanes 0, so they add nothing), then each of the 4 waves takes 16 x 16
-        output blocks in turn, loads the block's accumulators, runs k / K_STEP MFMAs and writes them back. Lane l of
+        instruction's operand type (invalid lanes 0, so they add nothing), then each wave takes 16 x 16 output blocks
+        in turn, loads the block's accumulators, runs k / K_STEP MFMAs and writes them back. Lane l of
         a 16x16xK MFMA holds operand row (or column) l % 16 and K_STEP / 4 consecutive k from (l / 16) * K_STEP / 4,
         and accumulators rows 4 (l / 16) + i, column l % 16 (reference compiler/hip.py:70-97 `AMDMFMA.product`,
         compiler/emit.py:924-955 `matrix_stage`). Staged rows are 16 bytes longer than K: 16 rows of a multiple of 128

@@ -256,7 +256,8 @@ static int launch(const AttentionCall& c) {
 // 34.7 -> 32.0; f16 128 x 4096 56.5 -> 50.8, 32 x 8192 35.0 -> 32.3; d = 64: bf16 128 x 4096, 128 MiB, 31.6 -> 30.1,
 // 64 x 16384 63.7 -> 56.7, f16 31.8 -> 29.8 and 64.4 -> 58.6; 32 queries f16 128 x 4096, d = 128, 58.2 -> 53.0). Smaller
 // ones keep ordinary loads (64 MiB: bf16 8 x 16384, d = 128, 24.3 us, non-temporally 27.8; f16 25.5 and 28.4; bf16
-// 16 x 16384, d = 64, 20.5 and 22.3), and so do longer prompts, whose row blocks share keys in L2 (16 x 1000 x 1000, d = 64: 11.9 us, non-temporally 13.2).
+// 16 x 16384, d = 64, 20.5 and 22.3), and so do longer prompts, whose row blocks share keys in L2 (16 x 1000 x
+// 1000, d = 64: 11.9 us, non-temporally 13.2).
 int krn::launch_attention_split(bool bf, int d, const AttentionCall& c) {
   const bool once = c.sq <= 32 && c.bh * c.sk * d * 4 >= (int64_t)128 << 20;
 #define KRN_SPLIT(BFV, DV) (once ? launch<BFV, DV, true>(c) : launch<BFV, DV, false>(c))

@@ -281,10 +281,14 @@ def span(argument: object) -> tuple[int, int]:
     return argument.pointer, argument.pointer + argument.numpy.itemsize * math.prod(argument.shape)
 
 
-def share_memory(x: object, y: object) -> bool:
-    """Whether two arguments are tensors with a byte of memory in common."""
-    (x, x_end), (y, y_end) = span(x), span(y)
-    return x < y_end and y < x_end and x < x_end and y < y_end
+def share_memory(tensor: object, *others: object) -> bool:
+    """Whether a tensor has a byte of memory in common with one of the others."""
+    start, end = span(tensor)
+    for other in others:
+        first, last = span(other)
+        if start < last and first < end and start < end and first < last:
+            return True
+    return False
 
 
 def _kind(argument: object) -> object:
@@ -406,7 +410,7 @@ class Launch:
                 code = base + (1 if op.axis == "row" else 2) + library.VECTOR_KINDS[vector.dtype]
                 ops.append((code, 0.0, vector.pointer))
         need = library.gemm_workspace(plan.layout, plan.operand, a.pointer, b.pointer, m, n, k)
-        if share_memory(c, a) or share_memory(c, b):
+        if share_memory(c, a, b):
             need = max(need, library.gemm_workspace_in_place(m, n))
         if need == 0 and plan.layout == "nt":
             direct = library.gemm_nt_call(plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k, ops)

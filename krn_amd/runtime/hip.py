@@ -274,23 +274,6 @@ class HIPTensor(Tensor):
             self.pointer = 0
 
 
-def span(argument: object) -> tuple[int, int]:
-    """The first and the end address of a tensor's memory; empty for an argument that is none."""
-    if not isinstance(argument, HIPTensor):
-        return 0, 0
-    return argument.pointer, argument.pointer + argument.numpy.itemsize * math.prod(argument.shape)
-
-
-def share_memory(tensor: object, *others: object) -> bool:
-    """Whether a tensor has a byte of memory in common with one of the others."""
-    start, end = span(tensor)
-    for other in others:
-        first, last = span(other)
-        if start < last and first < end and start < end and first < last:
-            return True
-    return False
-
-
 def _kind(argument: object) -> object:
     """What compiling depends on in one argument."""
     if isinstance(argument, HIPTensor):
@@ -410,8 +393,11 @@ class Launch:
                 code = base + (1 if op.axis == "row" else 2) + library.VECTOR_KINDS[vector.dtype]
                 ops.append((code, 0.0, vector.pointer))
         need = library.gemm_workspace(plan.layout, plan.operand, a.pointer, b.pointer, m, n, k)
-        if share_memory(c, a, b):
-            need = max(need, library.gemm_workspace_in_place(m, n))
+        if isinstance(c, HIPTensor):
+            size, end = a.numpy.itemsize, c.pointer + c.numpy.itemsize * m * n
+            if (c.pointer < a.pointer + size * m * k and a.pointer < end) or (
+                    c.pointer < b.pointer + size * n * k and b.pointer < end):  # C is written over an operand
+                need = max(need, library.gemm_workspace_in_place(m, n))
         if need == 0 and plan.layout == "nt":
             direct = library.gemm_nt_call(plan.operand, a.pointer, b.pointer, c.pointer, plan.output, m, n, k, ops)
             return lambda stream: direct(stream.handle)
@@ -476,11 +462,16 @@ class Launch:
 
     def _overlapping(self, values: list[object]) -> bool:
         """Whether a tensor this program stores to shares memory with another of its tensors (an in-place call)."""
-        spans = [span(v) for v in values]
-        for (name, _), (x, x_end) in zip(self.kernel.params, spans):
-            if name in self._stored:
-                meeting = sum(1 for y, y_end in spans if x < y_end and y < x_end and y < y_end)
-                if meeting > 1:  # itself, and another
+        stored, spans = [], []
+        for (name, _), v in zip(self.kernel.params, values):
+            if isinstance(v, HIPTensor):
+                spans.append((v.pointer, v.pointer + v.numpy.itemsize * math.prod(v.shape)))
+                if name in self._stored:
+                    stored.append(len(spans) - 1)
+        for i in stored:
+            start, end = spans[i]
+            for j, (first, last) in enumerate(spans):
+                if start < last and first < end and start < end and first < last and j != i:
                     return True
         return False
 

@@ -126,8 +126,8 @@ class Emitter:
         self.depth += 1
         names = []
         for a in range(len(shape)):
-            self.put(f"long long _i{a} = _e / {math.prod(shape[a + 1:])} % {shape[a]};")
-            names.append(f"_i{a}")
+            self.put(f"long long _0i{a} = _e / {math.prod(shape[a + 1:])} % {shape[a]};")
+            names.append(f"_0i{a}")
         body(names)
         self.depth -= 1
         self.put("}")
@@ -200,13 +200,13 @@ class Emitter:
         self.put("{")
         self.depth += 1
         for a, start in enumerate(starts):
-            self.put(f"long long _s{a} = {start};")
+            self.put(f"long long _0s{a} = {start};")
 
         def store(idx):
             tile_axes = iter(idx)
             cells = []
             for a, sl in enumerate(s.slices):
-                cells.append(f"_s{a}" if sl.squeeze else f"(_s{a} + {next(tile_axes)})")
+                cells.append(f"_0s{a}" if sl.squeeze else f"(_0s{a} + {next(tile_axes)})")
             inside = " && ".join(f"{c} >= 0 && {c} < {tensor}_n{a}" for a, c in enumerate(cells))
             linear = " + ".join(
                 f"{c}" + "".join(f" * {tensor}_n{b}" for b in range(a + 1, len(cells))) for a, c in enumerate(cells))
@@ -344,11 +344,11 @@ class Emitter:
         self.put("{")
         self.depth += 1
         for a, sl in enumerate(e.slices):
-            self.put(f"long long _s{a} = {self.scalar(sl.start)};")
+            self.put(f"long long _0s{a} = {self.scalar(sl.start)};")
 
         def load(idx):
             tile_axes = iter(idx)
-            cells = [f"_s{a}" if sl.squeeze else f"(_s{a} + {next(tile_axes)})" for a, sl in enumerate(e.slices)]
+            cells = [f"_0s{a}" if sl.squeeze else f"(_0s{a} + {next(tile_axes)})" for a, sl in enumerate(e.slices)]
             inside = " && ".join(f"{c} >= 0 && {c} < {tensor}_n{a}" for a, c in enumerate(cells))
             linear = " + ".join(
                 f"{c}" + "".join(f" * {tensor}_n{b}" for b in range(a + 1, len(cells))) for a, c in enumerate(cells))

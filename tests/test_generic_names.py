@@ -43,9 +43,11 @@ def product(x: Matrix[T.f32], y: Matrix[T.f32], {p}: T.i32) -> None:
                     acc += x[{a} * 8 : {a} * 8 + 8, {d} : {d} + 16] @ x[{d} : {d} + 16, {b} * 16 : {b} * 16 + 16]
                 y[{a} * 8 : {a} * 8 + 8, {b} * 16 : {b} * 16 + 16] = acc
 """
-NAMES = [("i", "s", "r", "x1", "p"), ("s", "i", "e", "r", "bx"), ("x", "t", "o", "s", "_e"), ("i", "i0", "r", "r", "_i0"),
-         ("st", "any", "mf", "k", "kmax"), ("u", "w", "l", "q", "y_n0"), ("blk", "m0", "n0", "next", "threadIdx"),
-         ("_s", "_x", "_r", "_i", "_s1"), ("acc", "seen", "y1", "p", "int_"), ("c", "j", "g", "kok", "_block")]
+NAMES = [("i", "s", "r", "x1", "p"), ("s", "i", "r", "e", "scale"), ("s", "i", "e", "r", "bx"), ("x", "t", "o", "s", "_e"),
+         ("i", "i0", "r", "r", "_i0"), ("st", "any", "mf", "k", "kmax"), ("u", "w", "l", "q", "y_n0"),
+         ("blk", "m0", "n0", "next", "threadIdx"), ("_s", "_x", "_r", "_i", "_s1"), ("acc", "seen", "y1", "p", "int_"),
+         ("c", "j", "g", "kok", "_block")]
+ORACLES = ("bx", "_e", "y_n0", "kmax", "_block")  # parameters with names of the oracle's C
 
 
 @pytest.mark.parametrize("program", ["scalars", "starts", "product"])
@@ -57,10 +59,13 @@ def test_programs_whose_names_the_lowering_might_use_itself(tmp_path, names, pro
     kernel = capture(path, program)
     x = np.random.default_rng(3).integers(-4, 5, (32, 32)).astype(np.float32)
     want = np.full((32, 32), -7, np.float32)
-    # the oracle keeps the program's names, so it is given plain ones
     plain = tmp_path / "plain.py"
     plain.write_text(PROGRAM.format(a="one", b="two", c="three", d="four", p="five"))
     cbackend.run(capture(plain, program), Blocks(1), [x.copy(), want, 3])
+    if names[4] not in ORACLES:  # loop variables get a number, parameters keep their name
+        named = np.full((32, 32), -7, np.float32)
+        cbackend.run(kernel, Blocks(1), [x.copy(), named, 3])
+        np.testing.assert_array_equal(named, want)
     for last_first in (False, True):
         got = np.full((32, 32), -7, np.float32)
         host_threads.run(kernel, [x.copy(), got, 3], Blocks(1), last_first)

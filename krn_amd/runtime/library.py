@@ -11,8 +11,8 @@ from functools import cache
 from krn_amd.dtypes import BF16, F8E4M3, F16, F32, I8, I32, Dtype
 from krn_amd.hw import Libraries
 
-# element kinds of the C ABI (enum Kind in krn_amd/csrc/common.h)
-KINDS = {F32: 0, F16: 1, BF16: 2, F8E4M3: 3, I8: 4, I32: 5}
+# element kinds of the C ABI (enum Kind in krn_amd/csrc/common.h), by the types' names: hashing a type is a Python call
+KINDS = {d.name: code for code, d in enumerate((F32, F16, BF16, F8E4M3, I8, I32))}
 
 # epilogue operations of krn_gemm_nt, applied in order with one float32 rounding each
 MUL_SCALAR, MUL_ROW, MUL_COL, ADD_SCALAR, ADD_ROW, ADD_COL, RELU, GELU, SILU = range(9)
@@ -86,7 +86,7 @@ def check(code: int, what: str) -> None:
 
 def kind(dtype: Dtype) -> int:
     try:
-        return KINDS[dtype]
+        return KINDS[dtype.name]
     except KeyError:
         raise KernelError(f"{dtype} has no kind in the kernel library's C ABI") from None
 

@@ -232,7 +232,7 @@ def main() -> None:
     args = parser.parse_args()
     if args.gpus != 1 or int(os.environ.get("WORLD_SIZE", "1")) > 1:
         print("bench.py measures one GPU: this build has no multi-GPU path (the tile kernels shard by output "
-              "tiles or heads with no exchange; see DESIGN.md). Run with --gpus 1.", file=sys.stderr)
+              "tiles or heads with no exchange). Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
     os.environ.setdefault("KRN_TARGET", "gfx950")
     from krn_amd.runtime.api import device_of

@@ -193,8 +193,11 @@ class HIPStream(Stream):
         self._marks.clear()
 
     def __del__(self) -> None:
-        if self._retire is not None:
-            self._retire(self.handle, (self._open, self._marks) if self._open or self._marks else ())
+        try:
+            if self._retire is not None:
+                self._retire(self.handle, (self._open, self._marks) if self._open or self._marks else ())
+        except Exception:  # the interpreter is ending
+            pass
 
 
 class Retired:

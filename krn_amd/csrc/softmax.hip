@@ -8,12 +8,11 @@
 // past its tile) are neither read nor written; a row is a run of valid lanes, so no padding value enters the
 // maximum or the sum.
 //
-// Layout (HBM-bound: one read, one write per element). A row belongs to one wave (four rows per workgroup), four waves
-// or sixteen: thread l owns the 16-byte chunks l, l + T, ... of its row. Up to CACHE chunks per thread stay in registers
-// as they were read, so rows of up to 65536 16-bit columns are read from HBM once; longer rows are read again (from
-// L2). A thread keeps a running maximum m and sum s of exp(x - m) over its chunks as they arrive (the maximum of all of
-// them first: f16 8192 x 2048 12.6 -> 13.1 us), the threads' pairs meet by shuffles and in LDS, and a second pass writes
-// exp(x - m) * (1 / s).
+// Layout (HBM-bound: one read, one write per element). A row belongs to one wave (four rows per workgroup), four waves,
+// eight or sixteen: thread l owns the 16-byte chunks l, l + T, ... of its row. Up to CACHE chunks per thread stay in
+// registers as they were read; what a longer row has past them is read again (from L2). A thread keeps a running
+// maximum m and sum s of exp(x - m) over its chunks as they arrive (the maximum of all of them first: f16 8192 x 2048
+// 12.6 -> 13.1 us), the threads' pairs meet by shuffles and in LDS, and a second pass writes exp(x - m) * (1 / s).
 //
 // Rows may start at any element: the chunks are loaded and stored 16 bytes at a time at any alignment, and only a chunk
 // that crosses the end of its row goes element by element (bf16 1024 x 50001, rows at every alignment, element by
@@ -125,9 +124,6 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : WAVES * 64) void softmax_rows(co
 #pragma unroll
   for (int i = 0; i < CACHE; ++i) kept[i] = load_chunk<KIND>(x, lane + T * i, width);
   float m = -INFINITY, s = 0.0f;
-  // before the second pass: the chunks stay as they were read (the compiler would keep all their float32 values, twice
-  // the registers)
-#define KRN_OPAQUE() _Pragma("unroll") for (int i = 0; i < CACHE; ++i) asm volatile("" : "+v"(kept[i]))
 #pragma unroll
   for (int i = 0; i < CACHE; ++i) {
     float top = m;
@@ -168,8 +164,14 @@ __global__ __launch_bounds__(WAVES == 1 ? 256 : WAVES * 64) void softmax_rows(co
     for (int w = 1; w < WAVES; ++w) combine(m, s, part[0][w], part[1][w]);
   }
   const float inv = 1.0f / s;
-  KRN_OPAQUE();
-#undef KRN_OPAQUE
+  // Before the second pass: the chunks stay as they were read (the compiler would keep 16-bit chunks' float32 values,
+  // twice the registers). It pays where it lets another workgroup fit: f16 4096 x 16400 on eight waves 53.1 -> 49.8 us.
+  // Elsewhere converting twice costs more: 20000 x 2048 25.2 -> 27.0, 4096 x 8192 20.9 -> 22.3, 1000 x 16384 12.7 ->
+  // 13.3, 1000 x 40000 29.2 -> 30.7 (4096 x 12000 on four waves alone would gain, 35.6 -> 34.2).
+  if constexpr (CACHE > 4 && CACHE < 8 && WAVES != 4) {
+#pragma unroll
+    for (int i = 0; i < CACHE; ++i) asm volatile("" : "+v"(kept[i]));
+  }
 #pragma unroll
   for (int i = 0; i < CACHE; ++i)
     if (lane + T * i < chunks) store_chunk<KIND, ALIGNED>(y, lane + T * i, width, kept[i], m, inv);
@@ -207,22 +209,35 @@ static int launch_softmax(const void* x, void* y, int64_t rows, int64_t width, i
   const bool aligned = (ldy * Chunk<KIND>::BYTES) % 16 == 0 && (uintptr_t)y % 16 == 0;
   const int64_t chunks = (width + N - 1) / N;
 #define KRN_ROWS(CACHE, WAVES) launch_rows<KIND, CACHE, WAVES>(aligned, x, y, rows, width, ldx, ldy, stream)
-  // chunks per thread that stay in registers (no more than the row needs: bf16 20000 x 1000 on two 14.9 us, on four
-  // 18.4): a wave's row up to 512 chunks (4096 16-bit columns), four waves' up to
-  // 2048, sixteen waves' up to 8192; longer rows are read again. Few rows of more than 256 chunks take four waves for
-  // the loads in flight.
-  if (chunks <= 512 && !(rows <= 4096 && chunks > 256)) {
-    if (chunks <= 64) KRN_ROWS(1, 1);
-    else if (chunks <= 128) KRN_ROWS(2, 1);
-    else if (chunks <= 256) KRN_ROWS(4, 1);
-    else KRN_ROWS(8, 1);
-  } else if (chunks <= 1024) {
-    KRN_ROWS(4, 4);
-  } else if (chunks <= 2048) {
-    KRN_ROWS(8, 4);
-  } else {
-    KRN_ROWS(8, 16);
-  }
+  // No more chunks per thread than the row needs, because a chunk past the row costs what one in it does; no more waves
+  // than keep the row in registers, because they wait for each other; and eight waves before sixteen, of which only one
+  // workgroup fits a compute unit where two or more of eight do. us, the other choice -> this one:
+  //   bf16 20000 x 1000: four chunks 18.4 -> two 14.9; f16 4096 x 3000: two of four waves 12.2 -> six of one 10.5
+  //   f16 4096 (1000) x 4096: eight of one wave 12.9 (5.5) -> two of four 13.2 (4.9); 20000 x 4096: 58.3 -> 56.6; f32
+  //   4096 (1000) x 2048: 10.3 (4.4) -> 10.9 (4.2); 20000 x 2048: 57.2 -> 54.3
+  //   f16 4096 x 8200: eight of four 28 -> five 23.2; x 16384: eight of four 47.7, four of eight 47.3
+  //   f16 4096 x 16400: eight of sixteen 110 -> five of eight 49.7, and eight of four with the rest read again 50.1 (at
+  //   1000 rows that is the faster by 4 to 9 %); x 20000: 62 -> 58; x 24576: 76 -> 71
+  //   f16 4096 x 32768: four of sixteen 101.7, eight of eight 101.7 to 105; 1000 x 32768: 25.6 -> 23.6
+  // Past what eight waves keep, reading up to three more chunks a thread again is still the better one: f32 4096 x 20000
+  // 126 (five of sixteen) -> 113, 4096 x 24576 147 -> 142; with fewer rows than compute units it is not: 128 x 57344 f16
+  // 12.9 against 11.9 us. Rows of 8192 chunks: 202 -> 193.
+  if (chunks <= 64) KRN_ROWS(1, 1);
+  else if (chunks <= 128) KRN_ROWS(2, 1);
+  else if (chunks <= 256) KRN_ROWS(4, 1);
+  else if (chunks <= 320) KRN_ROWS(5, 1);
+  else if (chunks <= 384) KRN_ROWS(6, 1);
+  else if (chunks <= 512) KRN_ROWS(2, 4);
+  else if (chunks <= 768) KRN_ROWS(3, 4);
+  else if (chunks <= 1024) KRN_ROWS(4, 4);
+  else if (chunks <= 1280) KRN_ROWS(5, 4);
+  else if (chunks <= 1536) KRN_ROWS(6, 4);
+  else if (chunks <= 1792) KRN_ROWS(7, 4);
+  else if (chunks <= 2048) KRN_ROWS(8, 4);
+  else if (chunks <= 2560) KRN_ROWS(5, 8);
+  else if (chunks <= 3072) KRN_ROWS(6, 8);
+  else if (chunks <= 4096 || (chunks <= 7168 && rows > 256)) KRN_ROWS(8, 8);
+  else KRN_ROWS(8, 16);
 #undef KRN_ROWS
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) {

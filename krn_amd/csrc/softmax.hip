@@ -216,9 +216,10 @@ static int launch_softmax(const void* x, void* y, int64_t rows, int64_t width, i
   //   f16 4096 (1000) x 4096: eight of one wave 12.9 (5.5) -> two of four 13.2 (4.9); 20000 x 4096: 58.3 -> 56.6; f32
   //   4096 (1000) x 2048: 10.3 (4.4) -> 10.9 (4.2); 20000 x 2048: 57.2 -> 54.3
   //   f16 4096 x 8200: eight of four 28 -> five 23.2; x 16384: eight of four 47.7, four of eight 47.3
-  //   f16 4096 x 16400: eight of sixteen 110 -> five of eight 49.7, and eight of four with the rest read again 50.1 (at
+  //   f16 4096 x 16400: eight of sixteen 151 -> five of eight 49.7, and eight of four with the rest read again 50.1 (at
   //   1000 rows that is the faster by 4 to 9 %); x 20000: 62 -> 58; x 24576: 76 -> 71
-  //   f16 4096 x 32768: four of sixteen 101.7, eight of eight 101.7 to 105; 1000 x 32768: 25.6 -> 23.6
+  //   f16 4096 x 32768: eight of sixteen 172, four of sixteen 101.7, eight of eight 101.7 to 105; 1000 x 32768:
+  //   25.6 -> 23.6
   // Past what eight waves keep, reading up to three more chunks a thread again is still the better one: f32 4096 x 20000
   // 126 (five of sixteen) -> 113, 4096 x 24576 147 -> 142; with fewer rows than compute units it is not: 128 x 57344 f16
   // 12.9 against 11.9 us. Rows of 8192 chunks: 202 -> 193.

@@ -1179,6 +1179,24 @@ static double split_cost(int shape, bool nn, int64_t m, int64_t n, int64_t slice
   return us;
 }
 
+// Whether the four-wave loop (MID) is the faster of the two 128 x 128 loops that run one tile per CU, the other being the
+// ring's four stages (RING_128x128_DEEP, one part). The ring reads whole lines and takes the same time per slice whatever
+// K is, but costs 2 us more where MID stores whole blocks straight from its accumulators; MID's blocks that a ragged N
+// cuts go out element by element. Measured on 129 to 256 tiles, MID against the ring, us:
+//   16-bit, up to 32 slices: 2048 x 2048 x 512 8.5 / 10.8, x 2048 21.2 / 23.3, 1500 x 2000 x 1024 14.0 / 15.7; from 33 on
+//   x 3072 32.9 / 31.3, except on rows of 8 and 16 KiB whose operands the last-level cache holds (2048 x 2048 x 4096
+//   38.5 / 40.4, x 8192 70.6 / 72.5; from HBM 512 x 8192 x 8192 93.4 / 79.1). N not a multiple of 16: 400 x 7000 x 512
+//   12.4 / 11.0.
+//   int8, up to 18 slices: 2048 x 2048 x 1024 15.3 / 17.3, x 2304 22.9 / 23.4, x 2560 25.6 / 24.9; 1500 x 2000 20.5 / 17.1.
+//   fp8, up to 8 slices: 2048 x 2048 x 1024 11.6 / 11.9, x 1280 13.5 / 12.9; ragged M, 1181 x 1792 x 512 9.0 / 9.1, x 640
+//   10.1 / 9.6; 1500 x 2000 x 512 11.2 / 10.1.
+static bool four_wave_wins(int fmt, int64_t m, int64_t n, int64_t slices) {
+  if (fmt == FMT_I8) return n % 64 == 0 && slices <= 18;
+  if (fmt == FMT_FP8) return n % 64 == 0 && slices <= (m % 64 == 0 ? 8 : 4);
+  if (n % 16 != 0) return false;
+  return slices <= 32 || ((slices == 64 || slices == 128) && (m + n) * slices * 128 <= (int64_t)80 << 20);
+}
+
 // Workgroups of a launch: of 256 threads, and a launch's threads along an axis stay below 2^32 (a launch past that runs
 // nothing: 2^30 rows of 64 x 64 tiles left C unwritten)
 constexpr int64_t MOST_TILES = ((int64_t)1 << 24) - 1;
@@ -1239,6 +1257,7 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
     for (int parts = 1; parts <= 16 && (parts == 1 || slices / parts >= 8); ++parts) {
       const int64_t need = parts > 1 ? parts * split_plane(m, n) : 0;
       if (need > workspace || split_tiles(shape, m, n) > MOST_TILES) break;
+      if (shape == RING_128x128_DEEP && parts == 1 && best.route == MID && four_wave_wins(fmt, m, n, slices)) continue;
       if (in_place && shape != RING_128x128 && shape != RING_128x128_DEEP && shape != ANY_128x128) break;
       const double us = split_cost(shape, nn, m, n, slices, parts);
       if (us < least) best = {SPLIT, shape, parts, need}, least = us;

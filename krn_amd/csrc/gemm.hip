@@ -1227,14 +1227,19 @@ static Plan plan_of(int fmt, bool nn, const void* a, const void* b, int64_t m, i
     // One workgroup per 32 columns; with few columns K is split as well. A slice takes a workgroup RATE, with one block
     // of 32 rows to four, beyond the launch's fixed cost (1 x 4096 x 4096 bf16, 64 slices: 9.2 us on 128 workgroups;
     // 16 x 1024 x 14336, 224 slices: 28.2 on 32, split 11.4); the second launch of a split costs 8, most of it on the
-    // host (3 x 768 x 4992 f16: 7.8 us, split 11.6).
-    static const double RATE[] = {0.10, 0.14, 0.24, 0.35};
+    // host (3 x 768 x 4992 f16: 7.8 us, split 11.6). Parts of whole 16 KiB start on the same memory channels, which costs
+    // 6 us or more once B is too large for the last-level cache to help: 4096 x 16384 in 16 bits, whole and in two parts,
+    // 1 row 30.1 and 35.5 us, 8 rows 32.7 and 36.0; 16 rows, where a slice takes longer, 36.3 and 34.3, 32 rows 43.9 and
+    // 34.3. Not so at 96 MiB (3072 x 16384, 1 row: 26.2 and 23.6) and for other parts (4096 x 28672: 46.4 and 38.6).
+    static const double RATE[] = {0.12, 0.14, 0.24, 0.35};
     const int64_t groups = (n + 31) / 32;
-    const double whole_k = (double)slices * RATE[(m - 1) / 32] * (double)((groups + 255) / 256);
+    const double rate = m <= 12 ? 0.10 : RATE[(m - 1) / 32];
+    const double whole_k = (double)slices * rate * (double)((groups + 255) / 256);
     best = {SKINNY, 0, 1, 0}, least = whole_k;
     for (int parts = 2; parts <= 16 && groups * parts <= 256 && slices / parts >= 8; ++parts) {
       const int64_t need = parts * split_plane(m, n);
-      const double us = whole_k / parts + 8.0 + (double)need / 5e6;
+      const bool same_channels = slices % (parts * 128) == 0 && n * kbytes >= (int64_t)112 << 20;
+      const double us = whole_k / parts + (same_channels ? 14.0 : 8.0) + (double)need / 5e6;
       if (need <= workspace && us < least) best = {SKINNY, 0, parts, need}, least = us;
     }
     // 65 to 128 rows of 16-bit operands: four row blocks per wave make the skinny loop slower than 128 x 128 tiles

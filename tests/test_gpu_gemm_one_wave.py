@@ -1,12 +1,14 @@
 """Products whose 128 x 128 tiles fill at most one wave of the chip, on both sides of the line between their two loops (up
-to 32 slices of 128 bytes in 16 bits, 18 of int8, 8 or 4 of fp8, and columns that are no multiple of the store blocks).
-int8 is bit-exact; 16-bit and fp8 products are checked
+to 32 slices of 128 bytes in 16 bits, 18 of int8, 8 or 4 of fp8, and columns that are no multiple of the store blocks),
+and of at most 128 rows on both sides of the rule that splits K. int8 is bit-exact; 16-bit and fp8 products are checked
 against float64 within 8 * 2^-24 * (k + 8) * |A| |B| plus the rounding of the result."""
 
 import numpy as np
 import pytest
 
 from krn_amd import T
+from krn_amd.dtypes import BF16
+from krn_amd.runtime import library
 from oracle.numerics import bf16_values, e4m3_decode, e4m3_encode
 from tests.helpers import assert_agrees, bf16_normal
 from tests.kernels import tile_programs as programs
@@ -45,3 +47,14 @@ def test_fp8(device, m, n, slices):
     c = device.empty(T.bf16, m, n)
     programs.gemm_fp8[TILING](device.to_device(a, T.f8e4m3fn), device.to_device(b, T.f8e4m3fn), c, 1.0, 1.0)
     assert_agrees(bf16_values(c.to_host()), e4m3_decode(a), e4m3_decode(b).T, k, "bf16")
+
+
+@pytest.mark.parametrize("m,n,k,split", [(1, 4096, 16384, False), (12, 4096, 16384, False), (13, 4096, 16384, True),
+                                         (8, 4096, 12288, True), (16, 1536, 6144, True), (12, 1536, 4096, False)])
+def test_few_rows_split_k_where_that_pays(device, m, n, k, split):
+    rng = np.random.default_rng(m + n + k)
+    (aw, a), (bw, b) = bf16_normal(rng, (m, k)), bf16_normal(rng, (n, k))
+    da, db, c = device.to_device(aw, T.bf16), device.to_device(bw, T.bf16), device.empty(T.bf16, m, n)
+    assert (library.gemm_workspace("nt", BF16, da.pointer, db.pointer, m, n, k) > 0) == split
+    programs.gemm_nt[TILING](da, db, c)
+    assert_agrees(bf16_values(c.to_host()), a, b.T, k, "bf16")

@@ -410,7 +410,11 @@ static int attention_parts(int64_t bh, int64_t sq, int64_t sk, int64_t d, int ca
   for (int parts = 1; parts <= 16; ++parts) {
     const double steps = fmax(1.0, mean / 32 / (4 * parts)), wgs = (double)(bh * q32 * parts);
     if (parts > 1 && (steps < 2.0 || attention_split_bytes(bh, sq, d, parts) > workspace)) break;
-    double us = d == 128 ? 3.0 + fmax(1.0, wgs / 256) * (2.6 + 1.6 * steps)
+    // causal workgroups take unlike times: past two for every CU, one more for some costs as much as one more for all
+    // (d = 128, one part, the kernel above and this one: 48 heads x 333 14.2 and 17.7, 48 x 300 12.9 and 13.4, 40 x 400
+    // 16.5 and 18.1, 32 x 700 23.9 and 25.7; 24 x 700 23.7 and 22.1 is the one of 24 that loses by it)
+    const double rounds = causal && wgs > 512 ? ceil(wgs / 256) : fmax(1.0, wgs / 256);
+    double us = d == 128 ? 3.0 + rounds * (2.6 + 1.6 * steps)
                          : 3.0 + fmax(1.0, wgs / 512) * (2.6 + (wgs > 256 ? 1.15 : 0.93) * steps);
     if (parts > 1) us += 3.0 + (double)attention_split_bytes(bh, sq, d, parts) / 5e6;
     if (us < least) best = parts, least = us;

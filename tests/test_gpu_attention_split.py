@@ -59,6 +59,17 @@ def test_few_query_rows_match_a_float64_softmax(device, dtype, d, causal, bh, sq
         np.testing.assert_allclose(got, want, atol=2e-2 if dtype == BF16 else 3e-3)
 
 
+@pytest.mark.parametrize("bh,s", [(32, 512), (33, 512), (48, 320), (48, 333), (32, 768)])
+def test_causal_launches_around_two_workgroups_for_every_compute_unit(device, bh, s):
+    """On both sides of the estimate's step at 512 workgroups of 32 rows, d = 128, whichever kernel it takes."""
+    rng = np.random.default_rng(bh + s)
+    words = [rng.standard_normal((bh, s, 128)).astype(np.float16) for _ in range(3)]
+    got, _ = attend(device, F16, *words, 0.13, True)
+    some = [0, 1, bh // 2, bh - 1]
+    want = reference(*(w[some].astype(np.float64) for w in words), 0.13, True)
+    np.testing.assert_allclose(got[some].astype(np.float64), want, atol=3e-3)
+
+
 def test_decoding_shares_a_head_among_workgroups_and_keeps_it_in_one_without_memory():
     assert library.attention_workspace(32, 1, 8192, 128, False) > 0
     assert library.attention_workspace(128, 4096, 4096, 128, True) == 0

@@ -16,7 +16,7 @@
 //
 // Rows may start at any element: the chunks are loaded and stored 16 bytes at a time at any alignment, and only a chunk
 // that crosses the end of its row goes element by element (bf16 1024 x 50001, rows at every alignment, element by
-// element before: 145 -> 59 us; the copy of as many bytes takes 31).
+// element before: 145 -> 57 us; the copy of as many bytes takes 31).
 #include "common.h"
 
 namespace krn {

@@ -1,6 +1,6 @@
 """Products whose 128 x 128 tiles fill at most one wave of the chip, on both sides of the line between their two loops (up
 to 32 slices of 128 bytes in 16 bits, 18 of int8, 8 or 4 of fp8, and columns that are no multiple of the store blocks),
-and of at most 128 rows on both sides of the rule that splits K. int8 is bit-exact; 16-bit and fp8 products are checked
+and products of few rows on both sides of the rule that splits K. int8 is bit-exact; 16-bit and fp8 products are checked
 against float64 within 8 * 2^-24 * (k + 8) * |A| |B| plus the rounding of the result."""
 
 import numpy as np

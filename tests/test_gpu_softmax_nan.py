@@ -1,6 +1,6 @@
 """krn_softmax_rows: a NaN makes its whole row NaN wherever it lies, also among -infinity in a thread, a half wave or a
-wave that holds no other value, while the finite values of the row lie in other lanes. One, four and sixteen waves a
-row, and rows longer than the registers hold."""
+wave that holds no other value, while the finite values of the row lie in other lanes. One, four, eight and sixteen
+waves a row, and rows longer than the registers hold."""
 
 import numpy as np
 import pytest
@@ -16,7 +16,7 @@ KIND = {F32: T.f32, F16: T.f16, BF16: T.bf16}
 
 
 @pytest.mark.parametrize("dtype", [F32, F16, BF16])
-@pytest.mark.parametrize("width", [40, 511, 1500, 4000, 6000, 16000, 40001, 70001, 140000])
+@pytest.mark.parametrize("width", [40, 511, 1500, 4000, 6000, 16000, 20001, 40001, 70001, 140000])
 def test_a_nan_among_minus_infinity_reaches_every_element_of_its_row(device, dtype, width):
     rng = np.random.default_rng(width)
     rows = 96
